@@ -41,6 +41,7 @@
 #include "common.hpp"
 #include "cplx.hpp"
 #include "spectral.hpp"
+#include "vhs_planar.hpp"
 
 namespace dgfs {
 
@@ -1330,7 +1331,7 @@ __global__ __launch_bounds__(RRShape<N>::NT) void k_vhs_prep_rr(PrepArgs<T> a) {
       rr_x_forward<T, N, G, false>(s, v0, v1, Xb, r, g, l);
     }
     cpx<T>* F = a.F + static_cast<size_t>(pt) * n;
-    cpx<T>* Ft = a.Ft + static_cast<size_t>(pt) * n;
+    cpx<T>* Ft = a.Ft ? a.Ft + static_cast<size_t>(pt) * n : nullptr;
     __syncthreads();  // the exchange buffer's readers are done before the wave-local transposes reuse it
 #pragma unroll
     for (int sr = 0; sr < 2; ++sr) {
@@ -1341,9 +1342,11 @@ __global__ __launch_bounds__(RRShape<N>::NT) void k_vhs_prep_rr(PrepArgs<T> a) {
       rr_plane_transpose<T, N, G, true, false>(v, Xb, g, l);  // (kx, ky = l, z)
       FFT<T, N, -1>::run(v);                            // z: (kx, ky = l, kz)
       __builtin_amdgcn_sched_barrier(0);
-      cpx<T>* ft = Ft + kx * NN + l;
+      if (a.Ft) {
+        cpx<T>* ft = Ft + kx * NN + l;
 #pragma unroll
-      for (int kz = 0; kz < N; ++kz) ft[kz * N] = rn * cpx<T>{v[kz].x - v[kz].y, v[kz].x + v[kz].y};  // (1 + i) F
+        for (int kz = 0; kz < N; ++kz) ft[kz * N] = rn * cpx<T>{v[kz].x - v[kz].y, v[kz].x + v[kz].y};  // (1 + i) F
+      }
       rr_plane_transpose<T, N, G, true, true>(v, Xb, g, l);  // (kx, ky, kz = l)
       cpx<T>* fp = F + kx * NN + l;
 #pragma unroll
@@ -1545,9 +1548,11 @@ __global__ __launch_bounds__(RR1Shape<N>::NT) void k_vhs_prep_rr1(PrepArgs<T> a)
 #pragma unroll
     for (int z = 0; z < N; ++z) v[z] = Xp[l * PP + z];
     FFT<T, N, -1>::run(v);  // z: (kx = g, ky = l, kz)
-    cpx<T>* ft = a.Ft + static_cast<size_t>(pt) * n + g * NN + l;
+    if (a.Ft) {
+      cpx<T>* ft = a.Ft + static_cast<size_t>(pt) * n + g * NN + l;
 #pragma unroll
-    for (int kz = 0; kz < N; ++kz) ft[kz * N] = rn * cpx<T>{v[kz].x - v[kz].y, v[kz].x + v[kz].y};  // (1 + i) F
+      for (int kz = 0; kz < N; ++kz) ft[kz * N] = rn * cpx<T>{v[kz].x - v[kz].y, v[kz].x + v[kz].y};  // (1 + i) F
+    }
     __syncthreads();
 #pragma unroll
     for (int kz = 0; kz < N; ++kz) Xp[l * PP + kz] = v[kz];
@@ -1842,6 +1847,15 @@ struct VhsHandle {
   size_t cap_wny = 0;
   void* Tb = nullptr;    // slab kernel's forward-transformed slabs [cap_pts][Nrho][n]
   size_t cap_tb = 0;
+  // planar-direction gain (vhs_planar.hpp): the design's groups, the operand
+  // values of the moves, and the points' operand form
+  int planar = 0;        // the design is planar and the kernels exist for this grid
+  int nshift = 0;
+  std::vector<PlanarGroup> pgroups;
+  void* smat = nullptr;  // [Nrho][nshift][64][N/2] operand values of R(shift)
+  double* pbeta = nullptr;  // [Nrho][nshift]
+  void* plop = nullptr;  // operand form of the points
+  size_t cap_plop = 0;
   int last_groups = 0, last_slots = 0, threads = 0;
   // set for the duration of an allocation-free call: the workspace pointers
   // above then point into the device scratch array and growing any of them
@@ -1871,6 +1885,9 @@ static void free_ws(VhsHandle* h) {
   (void)hipFree(h->Ft);
   h->Ft = nullptr;
   h->cap_ft = 0;
+  (void)hipFree(h->plop);
+  h->plop = nullptr;
+  h->cap_plop = 0;
   (void)hipFree(h->fc); (void)hipFree(h->Qc); (void)hipFree(h->F); (void)hipFree(h->Ghat);
   (void)hipFree(h->Z); (void)hipFree(h->S); (void)hipFree(h->W);
   h->fc = h->Qc = nullptr; h->F = h->Ghat = h->Z = h->S = h->W = nullptr;
@@ -1965,6 +1982,14 @@ static int rr_kind(const VhsHandle* h) {
 }
 
 static bool use_rr(const VhsHandle* h) { return rr_kind(h) != 1; }
+
+// the planar-direction gain stands in for the automatic choice's kernel where
+// the design allows it (an explicit set_algorithm runs what it names)
+template <int N>
+constexpr bool planar_available() {
+  return N == 16 || N == 24 || N == 32;
+}
+static bool use_planar(const VhsHandle* h) { return h->planar && h->algorithm == 0; }
 
 template <typename T, int N>
 static int run_gain_rr(VhsHandle* h, int npts, int groups, int ppg, size_t items, hipStream_t st) {
@@ -2175,7 +2200,7 @@ static int pick_groups(const VhsHandle* h, int npts, int slots, int min_groups =
 // gain), gain partial buffer; returns the gain kernel's arguments
 template <typename T, int N>
 static int stage_prep(VhsHandle* h, const double* fc, int npts, int groups, int slots, bool rr, GainArgs<T>* ga,
-                      hipStream_t st) {
+                      hipStream_t st, bool transposed = true) {
   constexpr int n = N * N * N;
   const int ppg = (h->Nrho + groups - 1) / groups;
   const size_t items = static_cast<size_t>(npts) * groups;
@@ -2190,7 +2215,7 @@ static int stage_prep(VhsHandle* h, const double* fc, int npts, int groups, int 
   h->last_groups = groups;
   h->last_slots = slots;
   h->threads = Shape<N>::NT;
-  if (rr) {
+  if (rr && transposed) {
     const size_t fbytes = static_cast<size_t>(npts) * n * sizeof(cpx<T>);
     if (fbytes > h->cap_ft) {
       if (h->no_alloc) return fail(DGFS_ERR_ALLOC, "allocation-free call: transposed spectra exceed their scratch share");
@@ -2201,7 +2226,7 @@ static int stage_prep(VhsHandle* h, const double* fc, int npts, int groups, int 
       h->cap_ft = fbytes;
     }
   }
-  PrepArgs<T> pa{fc, static_cast<cpx<T>*>(h->F), rr ? static_cast<cpx<T>*>(h->Ft) : nullptr,
+  PrepArgs<T> pa{fc, static_cast<cpx<T>*>(h->F), rr && transposed ? static_cast<cpx<T>*>(h->Ft) : nullptr,
                  static_cast<cpx<T>*>(h->Z), npts};
   KTimerT<VhsHandle> t0(h, 0, st);
   bool done = false;
@@ -2301,8 +2326,94 @@ static int stage_finish(VhsHandle* h, const double* fc, double* Qc, int npts, in
   return DGFS_OK;
 }
 
+// grow a workspace buffer to `bytes`
+static int grow_ws(VhsHandle* h, void** buf, size_t* cap, size_t bytes, const char* what) {
+  if (bytes <= *cap) return DGFS_OK;
+  if (h->no_alloc) return fail(DGFS_ERR_ALLOC, "allocation-free call: %s exceed their scratch share", what);
+  (void)hipFree(*buf);
+  *buf = nullptr;
+  *cap = 0;
+  DGFS_HIP_TRY(hipMalloc(buf, bytes));
+  *cap = bytes;
+  return DGFS_OK;
+}
+
+// work items of the planar gain resident on the device
+template <typename T, int N>
+static int planar_slots() {
+  using PS = PlanarShape<T, N>;
+  const void* kfn = reinterpret_cast<const void*>(k_vhs_gain_planar<T, N>);
+  (void)hipFuncSetAttribute(kfn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(PS::lds_bytes));
+  int occ = 1;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, kfn, PS::NW * 64, PS::lds_bytes) != hipSuccess || occ < 1)
+    occ = 1;
+  return occ * cu_count();
+}
+
+// planar-direction gain: spectra, operand form, the planes, x transform, finish
+template <typename T, int N>
+static int run_planar(VhsHandle* h, const double* fc, double* Qc, int npts, hipStream_t st) {
+  if constexpr (planar_available<N>()) {
+    using PS = PlanarShape<T, N>;
+    const int slots = planar_slots<T, N>();
+    const int groups = pick_groups(h, npts * PS::XH, slots);
+    const int ppg = (h->Nrho + groups - 1) / groups;
+    int rc = grow_ws(h, &h->plop, &h->cap_plop, static_cast<size_t>(npts) * PS::per_point * sizeof(T), "plane operands");
+    if (!rc)
+      rc = grow_ws(h, &h->Tb, &h->cap_tb,
+                   static_cast<size_t>(npts) * h->Nrho * PS::nslots * PS::NN * sizeof(cpx<T>), "plane transforms");
+    if (rc) return rc;
+    GainArgs<T> ga;
+    rc = stage_prep<T, N>(h, fc, npts, 1, slots, true, &ga, st, false);
+    if (rc) return rc;
+    h->last_algorithm = rr_kind(h);
+    h->last_groups = groups;
+    {
+      PlanarPrepArgs<T> pa{fc, static_cast<T*>(h->plop), npts};
+      const size_t lds = (static_cast<size_t>(2 * PS::RN) + 3) * N * (N + 1) * sizeof(T);
+      const void* kfn = reinterpret_cast<const void*>(k_planar_prep<T, N>);
+      DGFS_HIP_TRY(hipFuncSetAttribute(kfn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
+      const int grid = rr_edge_grid(kfn, 256, lds, npts);
+      KTimerT<VhsHandle> t0(h, 0, st);
+      hipLaunchKernelGGL((k_planar_prep<T, N>), dim3(grid), dim3(256), lds, st, pa);
+      DGFS_LAUNCH_CHECK("planar_prep");
+      t0.stop();
+    }
+    PlanarGainArgs<T> pg;
+    pg.op = static_cast<const T*>(h->plop);
+    pg.smat = static_cast<const T*>(h->smat);
+    pg.beta = h->pbeta;
+    pg.Tb = static_cast<cpx<T>*>(h->Tb);
+    pg.nitems = npts * groups * PS::XH;
+    pg.ngroups = groups;
+    pg.ppg = ppg;
+    pg.Nrho = h->Nrho;
+    pg.nshift = h->nshift;
+    pg.ngr = static_cast<int>(h->pgroups.size());
+    std::copy(h->pgroups.begin(), h->pgroups.end(), pg.gr);
+    const int grid = std::min(pg.nitems, slots);
+    KTimerT<VhsHandle> t1(h, 1, st);
+    hipLaunchKernelGGL((k_vhs_gain_planar<T, N>), dim3(grid), dim3(PS::NW * 64), PS::lds_bytes, st, pg);
+    DGFS_LAUNCH_CHECK("vhs_gain_planar");
+    PlanarXfwdArgs<T> xa{static_cast<const cpx<T>*>(h->Tb), static_cast<const T*>(h->b1), h->wgt,
+                         static_cast<cpx<T>*>(h->Ghat), npts, h->Nrho};
+    const long cols = static_cast<long>(npts) * (N / 2 + 1) * N;
+    const long per = (sizeof(T) == 8) ? 128 : 256;
+    hipLaunchKernelGGL((k_planar_xfwd<T, N>), dim3(static_cast<unsigned>((cols + per - 1) / per)), dim3(256), 0, st, xa);
+    DGFS_LAUNCH_CHECK("planar_xfwd");
+    t1.stop();
+    h->threads = PS::NW * 64;
+    h->last_slots = grid;
+    return stage_finish<T, N>(h, fc, Qc, npts, 1, st);
+  } else {
+    (void)h; (void)fc; (void)Qc; (void)npts; (void)st;
+    return fail(DGFS_ERR_UNSUPPORTED, "planar gain kernel not built for Nv=%d", N);
+  }
+}
+
 template <typename T, int N>
 static int run_chunk(VhsHandle* h, const double* fc, double* Qc, int npts, hipStream_t st) {
+  if (use_planar(h)) return run_planar<T, N>(h, fc, Qc, npts, st);
   const bool rr = use_rr(h);
   int slots = rr ? cu_count() : h->cap_slots;
   if (!rr && h->slots_override > 0) slots = std::min(slots, h->slots_override);
@@ -2364,8 +2475,10 @@ static int ensure_ws(VhsHandle* h, int pts) {
 // kept under 48 GiB of the 288 GB of HBM; launches are balanced in size
 static int chunk_points(const VhsHandle* h, int total) {
   double per = static_cast<double>(h->n) * (2.0 * h->tsize * (1 + h->Nrho) + 16.0);
-  if (use_rr(h)) per += 3.0 * h->N * h->N * h->Nrho * h->M * 2.0 * h->tsize + 2.0 * h->tsize * h->n;
-  if (rr_kind(h) == 6) per += 2.0 * h->tsize * h->n * h->Nrho;  // the slab kernel's T
+  if (use_planar(h))  // spectrum, one G^, operands, T, f and Q
+    per = static_cast<double>(h->n) * (h->tsize * (2.0 + 2.0 + 3.5 + h->Nrho) + 16.0);
+  else if (use_rr(h)) per += 3.0 * h->N * h->N * h->Nrho * h->M * 2.0 * h->tsize + 2.0 * h->tsize * h->n;
+  if (rr_kind(h) == 6 && !use_planar(h)) per += 2.0 * h->tsize * h->n * h->Nrho;  // the slab kernel's T
   const double budget = 48.0 * 1024.0 * 1024.0 * 1024.0;
   const int cap = std::max(1, static_cast<int>(budget / per));
   if (total <= cap) return std::max(total, 1);
@@ -2421,6 +2534,90 @@ static int dispatch(VhsHandle* h, const double* f, double* Q, bool aosoa, int nu
   }
 }
 
+// Groups of a planar design (vhs_planar.hpp): every direction has exactly one
+// zero component and its mirror image (a, -b) in the set.  shifts receives the
+// distinct |components|; false if the design is not planar.
+static bool planar_groups(const double* sz, int M, std::vector<PlanarGroup>* groups, std::vector<double>* shifts) {
+  groups->clear();
+  shifts->clear();
+  std::vector<char> used(M, 0);
+  auto shift_of = [&](double v) {
+    for (size_t k = 0; k < shifts->size(); ++k)
+      if ((*shifts)[k] == v) return static_cast<int>(k);
+    shifts->push_back(v);
+    return static_cast<int>(shifts->size()) - 1;
+  };
+  for (int q = 0; q < M; ++q) {
+    if (used[q]) continue;
+    const double* d = sz + 3 * q;
+    const int zeros = (d[0] == 0.0) + (d[1] == 0.0) + (d[2] == 0.0);
+    if (zeros != 1) return false;
+    const int pair = (d[2] == 0.0) ? 0 : (d[1] == 0.0) ? 1 : 2;
+    const int u = pair == 2 ? 1 : 0, v = pair == 0 ? 1 : 2;
+    int mate = -1;
+    for (int r = q + 1; r < M && mate < 0; ++r) {
+      const double* e = sz + 3 * r;
+      if (!used[r] && e[3 - u - v] == 0.0 && std::fabs(e[u]) == std::fabs(d[u]) &&
+          std::fabs(e[v]) == std::fabs(d[v]) && e[u] * e[v] * d[u] * d[v] < 0.0)
+        mate = r;
+    }
+    if (mate < 0) return false;
+    used[q] = used[mate] = 1;
+    const int ia = shift_of(std::fabs(d[u])), ib = shift_of(std::fabs(d[v]));
+    groups->push_back(PlanarGroup{pair, ia, ib});
+  }
+  std::stable_sort(groups->begin(), groups->end(),
+                   [](const PlanarGroup& a, const PlanarGroup& b) { return a.pair < b.pair; });
+  return !groups->empty() && groups->size() <= static_cast<size_t>(kPlanarMaxGroups) &&
+         shifts->size() <= static_cast<size_t>(kPlanarMaxShifts);
+}
+
+// operand values of R(shift) (vhs_planar.hpp) for every radial node and shift:
+// [Nrho][nshift][64 lanes][even/odd][tile][r], and beta = -sin(theta N/2) / N
+template <typename T>
+static void planar_tables(int N, const std::vector<double>& alpha, const std::vector<double>& shifts,
+                          std::vector<double>* smat, std::vector<double>* beta) {
+  const int RN = N / 8, NR = 4 * RN, D = static_cast<int>(shifts.size()), P = static_cast<int>(alpha.size());
+  const double pi = 3.14159265358979323846;
+  std::vector<double> cs(N), R(N);
+  for (int m = 0; m < N; ++m) cs[m] = std::cos(2.0 * pi * m / N);
+  smat->assign(static_cast<size_t>(P) * D * 64 * NR, 0.0);
+  beta->assign(static_cast<size_t>(P) * D, 0.0);
+  for (int p = 0; p < P; ++p)
+    for (int d = 0; d < D; ++d) {
+      const double th = alpha[p] * shifts[d];
+      std::vector<double> ct(N / 2 + 1), sn(N / 2 + 1);
+      for (int l = 0; l <= N / 2; ++l) {
+        ct[l] = std::cos(th * l);
+        sn[l] = std::sin(th * l);
+      }
+      // R(j) = Re (1/N) sum_l exp(i th l) exp(2 pi i l j / N), l = -N/2 .. N/2 - 1
+      for (int j = 0; j < N; ++j) {
+        double s = 1.0 + ct[N / 2] * cs[(static_cast<long>(j) * (N / 2)) % N];
+        for (int l = 1; l < N / 2; ++l) {
+          const int m = static_cast<int>((static_cast<long>(j) * l) % N);
+          s += 2.0 * (ct[l] * cs[m] - sn[l] * cs[(m + N - N / 4) % N]);  // sin x = cos(x - pi/2)
+        }
+        R[j] = s / N;
+      }
+      (*beta)[static_cast<size_t>(p) * D + d] = -sn[N / 2] / N;
+      double* o = smat->data() + (static_cast<size_t>(p) * D + d) * 64 * NR;
+      for (int lane = 0; lane < 64; ++lane) {
+        const int g = lane / 16, i = lane % 16;
+        if (!MmaTile<T>::valid(i, RN)) continue;
+        for (int t = 0; t < 2; ++t) {
+          const int row = t ? N - 1 - MmaTile<T>::col(i) : MmaTile<T>::col(i);
+          for (int r = 0; r < RN; ++r) {
+            const int k = 4 * r + g;
+            const double a = R[(row - k + N) % N], b = R[(row - (N - 1 - k) + N) % N];
+            o[lane * NR + t * RN + r] = a + b;
+            o[lane * NR + (2 + t) * RN + r] = a - b;
+          }
+        }
+      }
+    }
+}
+
 // two handles (velocity grids NA > NB, same precision) in one persistent gain
 // launch; both take the multi-pass gain
 // ---------------------------------------------------------------------------
@@ -2464,8 +2661,8 @@ static size_t align_up(size_t b) { return (b + kScratchAlign - 1) / kScratchAlig
 struct ScratchPlan {
   int pts = 0, groups = 0, slots = 0;
   size_t items = 0;  // gain partial buffers the Ghat share holds
-  size_t z = 0, s = 0, w = 0, F = 0, Ghat = 0, Ft = 0, Wny = 0, Tb = 0;
-  size_t total() const { return z + s + w + F + Ghat + Ft + Wny + Tb; }
+  size_t z = 0, s = 0, w = 0, F = 0, Ghat = 0, Ft = 0, Wny = 0, Tb = 0, plop = 0;
+  size_t total() const { return z + s + w + F + Ghat + Ft + Wny + Tb + plop; }
 };
 
 template <typename T, int N>
@@ -2477,6 +2674,18 @@ static ScratchPlan plan_scratch(const VhsHandle* h, int pts, int slots) {
   ScratchPlan p;
   p.pts = pts;
   p.slots = slots;
+  if constexpr (planar_available<N>()) {
+    if (use_planar(h)) {  // one G^ per point whatever the split; only the FP64 prep and finalize take slot cubes
+      using PS = PlanarShape<T, N>;
+      p.groups = 1;
+      p.items = static_cast<size_t>(pts);
+      p.z = align_up(static_cast<size_t>(slots) * n * sizeof(cpx<T>));
+      p.F = p.Ghat = align_up(static_cast<size_t>(pts) * n * sizeof(cpx<T>));
+      p.Tb = align_up(static_cast<size_t>(pts) * h->Nrho * PS::nslots * PS::NN * sizeof(cpx<T>));
+      p.plop = align_up(static_cast<size_t>(pts) * PS::per_point * sizeof(T));
+      return p;
+    }
+  }
   p.groups = pick_groups(h, pts, gain_slots);
   if constexpr (slab_available<N>()) {
     if (rr_kind(h) == 6) {
@@ -2504,14 +2713,14 @@ static ScratchPlan plan_scratch(const VhsHandle* h, int pts, int slots) {
 // array and put back however the call ends
 struct NoAllocScope {
   VhsHandle* h;
-  void *F, *Ghat, *Z, *S, *W, *Wny, *Ft, *Tb;
+  void *F, *Ghat, *Z, *S, *W, *Wny, *Ft, *Tb, *plop;
   double *fc, *Qc;
-  size_t cap_pts, cap_items, cap_ft, cap_wny, cap_tb;
+  size_t cap_pts, cap_items, cap_ft, cap_wny, cap_tb, cap_plop;
   int cap_slots, timing;
   explicit NoAllocScope(VhsHandle* hh)
       : h(hh), F(hh->F), Ghat(hh->Ghat), Z(hh->Z), S(hh->S), W(hh->W), Wny(hh->Wny), Ft(hh->Ft), Tb(hh->Tb),
-        fc(hh->fc), Qc(hh->Qc), cap_pts(hh->cap_pts), cap_items(hh->cap_items), cap_ft(hh->cap_ft),
-        cap_wny(hh->cap_wny), cap_tb(hh->cap_tb), cap_slots(hh->cap_slots), timing(hh->timing) {
+        plop(hh->plop), fc(hh->fc), Qc(hh->Qc), cap_pts(hh->cap_pts), cap_items(hh->cap_items), cap_ft(hh->cap_ft),
+        cap_wny(hh->cap_wny), cap_tb(hh->cap_tb), cap_plop(hh->cap_plop), cap_slots(hh->cap_slots), timing(hh->timing) {
     h->no_alloc = 1;
     h->timing = 0;  // the event pool may grow; no timing in this mode
   }
@@ -2530,6 +2739,7 @@ struct NoAllocScope {
     h->Ft = take(p.Ft);
     h->Wny = take(p.Wny);
     h->Tb = take(p.Tb);
+    h->plop = take(p.plop);
     h->fc = h->Qc = nullptr;  // the contiguous form reads f and writes Q in place
     h->cap_slots = p.slots;
     h->cap_pts = static_cast<size_t>(p.pts);
@@ -2537,9 +2747,11 @@ struct NoAllocScope {
     h->cap_ft = p.Ft;
     h->cap_wny = p.Wny;
     h->cap_tb = p.Tb;
+    h->cap_plop = p.plop;
   }
   ~NoAllocScope() {
     h->F = F; h->Ghat = Ghat; h->Z = Z; h->S = S; h->W = W; h->Wny = Wny; h->Ft = Ft; h->Tb = Tb;
+    h->plop = plop; h->cap_plop = cap_plop;
     h->fc = fc; h->Qc = Qc;
     h->cap_pts = cap_pts; h->cap_items = cap_items; h->cap_ft = cap_ft; h->cap_wny = cap_wny; h->cap_tb = cap_tb;
     h->cap_slots = cap_slots;
@@ -2763,6 +2975,20 @@ extern "C" int dgfs_vhs_create(const dgfs_vhs_desc* d, void** out) {
     rc = upload(&h->ephtab, tab);
     if (rc) return rc;
   }
+  std::vector<double> shifts;
+  if ((N == 16 || N == 24 || N == 32) && planar_groups(d->sz, h->M, &h->pgroups, &shifts)) {
+    std::vector<double> smat, pbeta;
+    if (h->prec == 64)
+      planar_tables<double>(N, alpha, shifts, &smat, &pbeta);
+    else
+      planar_tables<float>(N, alpha, shifts, &smat, &pbeta);
+    rc = upload(&h->smat, smat);
+    if (rc) return rc;
+    DGFS_HIP_TRY(hipMalloc(&h->pbeta, pbeta.size() * sizeof(double)));
+    DGFS_HIP_TRY(hipMemcpy(h->pbeta, pbeta.data(), pbeta.size() * sizeof(double), hipMemcpyHostToDevice));
+    h->nshift = static_cast<int>(shifts.size());
+    h->planar = 1;
+  }
 
   // (C C^T)^{-1} / cw^2 for the projection: A_jk = sum_r phi_j phi_k cw
   double A[25] = {};
@@ -2796,6 +3022,7 @@ extern "C" int dgfs_vhs_destroy(void* p) {
   (void)hipFree(h->b1); (void)hipFree(h->b2); (void)hipFree(h->alpha); (void)hipFree(h->wgt);
   (void)hipFree(h->szd);
   (void)hipFree(h->ephtab);
+  (void)hipFree(h->smat); (void)hipFree(h->pbeta);
   h->magic = 0;
   delete h;
   return DGFS_OK;

@@ -75,6 +75,8 @@ class Autotuner:
             algos[:0] = [2, 3, 5]
         if op.precision == 64 and op.Nv in (16, 24, 32):
             algos[:0] = [6]
+        if getattr(op, "planar", False):
+            algos[:0] = [0]  # the planar-direction gain has no number of its own
         groups = [0]
         g = 1
         while g <= op.Nrho:
@@ -83,7 +85,7 @@ class Autotuner:
         out = []
         for a in algos:
             for gr in groups:
-                slots = [0] if a >= 2 else [0, cus, 2 * cus, 4 * cus]
+                slots = [0] if a != 1 else [0, cus, 2 * cus, 4 * cus]
                 for sl in slots:
                     out.append({"algorithm": a, "groups": gr, "slots": sl})
         return out

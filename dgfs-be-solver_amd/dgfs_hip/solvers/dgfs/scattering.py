@@ -64,6 +64,9 @@ class VHSOperator:
         self._h = h
         self.Nv, self.vsize, self.precision, self.project = Nv, Nv ** 3, precision, project
         self.Nrho, self.M, self.K = Nrho, M, Nrho * M
+        # whether the automatic choice may take the planar-direction gain, which
+        # no algorithm number names (the autotuner then tries it as well)
+        self.planar = Nv in (16, 24, 32) and bool(np.all((self._sz == 0.0).sum(axis=1) == 1))
 
     @classmethod
     def from_mesh(cls, vm, gamma, prefac, precision=64, project=False):

@@ -133,8 +133,12 @@ int dgfs_vhs_set_slots(void* handle, int nslots);
  * x-transform decimated to the slab's planes; a second kernel completes the
  * forward transform along x and sums over the radial nodes).  The automatic
  * choice is, in FP32, 4 at Nv 16 and 24 and 5 at Nv 32; in FP64, 6 at Nv 16,
- * 24 and 32; 1 otherwise.
- * get_algorithm reports the one the last eval ran.
+ * 24 and 32; 1 otherwise.  At Nv 16, 24 and 32 the automatic choice runs the
+ * planar-direction gain (csrc/vhs_planar.hpp) in that kernel's place when
+ * every direction of the design has exactly one zero component and comes with
+ * its mirror image (the 24-point design, M = 12); it is not selectable by
+ * number.  get_algorithm reports the kernel the last eval ran, or the one the
+ * planar-direction gain stood in for.
  * No reference counterpart (the reference has one cuFFT dataflow). */
 int dgfs_vhs_set_algorithm(void* handle, int algorithm);
 int dgfs_vhs_get_algorithm(void* handle, int* algorithm);

@@ -1,0 +1,124 @@
+"""The planar-direction gain (csrc/vhs_planar.hpp), the automatic choice at Nv
+16, 24 and 32 when every direction of the half-sphere design has exactly one
+zero component and comes with its mirror image, against the multi-pass kernel
+(algorithm 1), which transforms every direction on its own.
+
+FP64: the two are the same sum in another order, so roundoff (1e-12 relative
+L2).  The rough states are white noise: the unpaired Nyquist modes, which the
+planar form carries as separate terms, are then as large as any other.
+FP32: the distance of Q from the FP64 operator is within a factor of 1.5 of
+the multi-pass kernel's on the same states."""
+import sys
+
+import numpy as np
+import pytest
+
+from oracle import vhs as O
+
+pytestmark = pytest.mark.gpu
+
+
+def say(*a):
+    print(*a, flush=True)
+    sys.stdout.flush()
+
+
+def rel(a, b):
+    return float(np.linalg.norm(a - b) / np.linalg.norm(b))
+
+
+def designs():
+    twelve = O.half_sphere_design(12)
+    rng = np.random.default_rng(5)
+    signs = rng.choice([-1.0, 1.0], size=(12, 1))
+    cubo = np.array([[1, 1, 0], [1, -1, 0], [1, 0, 1], [1, 0, -1], [0, 1, 1], [0, 1, -1]]) / np.sqrt(2.0)
+    # one axis pair only, unequal components
+    flat = np.array([[0.6, 0.8, 0.0], [0.6, -0.8, 0.0], [0.28, 0.96, 0.0], [-0.28, 0.96, 0.0]])
+    return {"m12": twelve, "m12_shuffled": (twelve * signs)[rng.permutation(12)], "m6_cuboctahedron": cubo,
+            "m4_one_pair": flat}
+
+
+def make(N, sz, precision, project=False, Nrho=4, algorithm=0):
+    from dgfs_hip.solvers.dgfs.scattering import VHSOperator
+    from dgfs_hip.solvers.dgfs.velocitymesh import DGFSVelocityMesh
+    vm = DGFSVelocityMesh.from_params(None, N, 6.0, Nrho, 6)
+    op = VHSOperator(N, Nrho, len(sz), vm.L(), 0.38, 1.0, vm.qz(), vm.qw(), sz, 2 * np.pi / len(sz), vm.cw(),
+                     precision=precision, project=project)
+    op.set_algorithm(algorithm)
+    return op
+
+
+def run(op, f, device):
+    import torch
+    ft = torch.as_tensor(f, device=device)
+    Qt = torch.full_like(ft, float("nan"))
+    op.eval_contig(ft.data_ptr(), Qt.data_ptr(), f.shape[0], torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    return Qt.cpu().numpy()
+
+
+@pytest.mark.parametrize("name", list(designs()))
+@pytest.mark.parametrize("N", [16, 24, 32])
+def test_planar_matches_multipass_on_rough_states(N, name, device):
+    rng = np.random.default_rng(N)
+    sz = designs()[name]
+    f = rng.uniform(0.0, 1.0, size=(3, N ** 3))
+    say("planar", N, name)
+    ref = run(make(N, sz, 64, algorithm=1), f, device)
+    op = make(N, sz, 64)
+    for groups in (0, 1, 3):
+        op.set_groups(groups)
+        e = rel(run(op, f, device), ref)
+        say("  fp64 groups", groups, e)
+        assert e < 1e-12
+    e_mp = rel(run(make(N, sz, 32, algorithm=1), f, device), ref)
+    e_pl = rel(run(make(N, sz, 32), f, device), ref)
+    say("  fp32 multi-pass", e_mp, "planar", e_pl)
+    assert e_pl < 1.5 * e_mp
+
+
+@pytest.mark.parametrize("precision", [64, 32])
+@pytest.mark.parametrize("N,npts", [(16, 1), (16, 300), (24, 5), (32, 1), (32, 37)])
+def test_planar_batches_and_registers(N, npts, precision, device):
+    """One point to more items than the chip holds, contiguous and as AoSoA
+    registers of a ragged element count, with the projection."""
+    import torch
+    sz = designs()["m12"]
+    vm = O.VelocityMesh(N, 6.0, 4, 12)
+    rng = np.random.default_rng(npts)
+    f = np.stack([0.5 * O.maxwellian(vm, 1, rng.uniform(-0.6, 0.6, 3), rng.uniform(0.5, 1.5)) +
+                  0.5 * O.maxwellian(vm, 1, rng.uniform(-0.6, 0.6, 3), rng.uniform(0.5, 1.5)) for _ in range(npts)])
+    say("planar batch", N, npts, precision)
+    op = make(N, sz, precision, project=True)
+    Q = run(op, f, device)
+    sub = np.unique(np.linspace(0, npts - 1, 6).astype(int))
+    ref = run(make(N, sz, 64, project=True, algorithm=1), f[sub], device)
+    e = rel(Q[sub], ref)
+    say("  vs FP64 multi-pass", e)
+    assert e < (1e-11 if precision == 64 else 1e-3)
+    # elements [1, neles) of a register of one point per element
+    neles, n = npts + 1, N ** 3
+    nparr = -(-neles // 32) * 32
+    reg = np.zeros((1, nparr // 32, n, 32))
+    for e in range(npts):
+        reg[0, (e + 1) // 32, :, (e + 1) % 32] = f[e]
+    rt = torch.as_tensor(reg.reshape(1, -1), device=device)
+    qt = torch.zeros_like(rt)
+    op.eval_aosoa(rt.data_ptr(), qt.data_ptr(), 1, nparr * n, n, neles, 1, npts,
+                  torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    qr = qt.cpu().numpy().reshape(nparr // 32, n, 32)
+    got = np.stack([qr[(e + 1) // 32, :, (e + 1) % 32] for e in range(npts)])
+    assert np.array_equal(got, Q)
+    assert not qr[0, :, 0].any()
+
+
+def test_other_designs_keep_the_general_gain(device):
+    """A direction with no zero component, or a missing mirror image, takes
+    the general kernels: same Q as with the algorithm named."""
+    N = 16
+    f = np.random.default_rng(3).uniform(0.0, 1.0, size=(2, N ** 3))
+    for sz in (O.half_sphere_design(6), designs()["m12"][:11]):
+        say("general design", len(sz))
+        auto, named = run(make(N, sz, 64), f, device), run(make(N, sz, 64, algorithm=6), f, device)
+        assert np.array_equal(auto, named)
