@@ -483,43 +483,132 @@ __global__ __launch_bounds__(256) void k_copy_reg(int nblocks, int count, const 
 // (plugins/dgfsmomwriterstd.py:14-214): rho, U, T, q, P with
 // T = (2/3) sum f |c-U|^2 cw / rho, q_i = sum f c'_i |c'|^2 cw, P_ij = 2 sum f c'_i c'_j cw,
 // p = rho T.  out[upt][m][e] for m over the 15 outputs (3D layout).
-__global__ __launch_bounds__(256) void k_moments(int nupts, int neles, int vsize, const double* __restrict__ f,
-                                                 long ld, const double* __restrict__ cv, double cw,
-                                                 double* __restrict__ out) {
-  // one thread per (upt, e): two passes over v (bulk velocity, then peculiar moments)
-  const long t = static_cast<long>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (t >= static_cast<long>(nupts) * neles) return;
-  const int upt = static_cast<int>(t / neles);
-  const long e = t % neles;
-  const double* fu = f + upt * ld;
-  double rho = 0, ux = 0, uy = 0, uz = 0;
-  for (int v = 0; v < vsize; ++v) {
-    const double x = fu[soa_ix(e, v, vsize)];
-    rho += x;
-    ux += x * cv[v];
-    uy += x * cv[vsize + v];
-    uz += x * cv[2L * vsize + v];
+//
+// A workgroup takes EW neighbouring elements of one AoSoA block at one solution
+// point: a thread two of them at every (512 / (EW/2))-th velocity (so that a
+// velocity's abscissae are read once for two values), kMomUnroll velocities in
+// flight; then a sum over the threads of a wave and over the waves, always in
+// the same order.  Two passes over f, the bulk velocity first (the second
+// mostly from the last-level cache).  EW is the widest that still gives every
+// CU a workgroup: half of the time is FP64 arithmetic, which needs the whole
+// chip.  2304 points at 24^3 on MI355X: 9019 us with one thread per point,
+// 470 us with 72 workgroups of 32 elements, 205 us with 288 of 8 (floor: 56 us
+// for reading f once).
+constexpr int kMomUnroll = 4, kMomWaves = 8;
+
+// totals over the workgroup of NQ values of two elements per thread; red:
+// [kMomWaves][NQ][EW]
+template <int NQ, int EW>
+__device__ __forceinline__ void mom_reduce(double (&s)[NQ][2], double* red) {
+  constexpr int TPR = EW / 2;
+  const int sub = threadIdx.x % TPR, wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int j = 0; j < NQ; ++j)
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int d = 32; d >= TPR; d >>= 1) s[j][h] += __shfl_xor(s[j][h], d);
+  __syncthreads();
+  if ((threadIdx.x & 63) < TPR)
+#pragma unroll
+    for (int j = 0; j < NQ; ++j)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) red[(wave * NQ + j) * EW + 2 * sub + h] = s[j][h];
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < NQ; ++j)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      double t = 0.0;
+#pragma unroll 1
+      for (int w = 0; w < kMomWaves; ++w) t += red[(w * NQ + j) * EW + 2 * sub + h];
+      s[j][h] = t;
+    }
+}
+
+template <int EW>
+__global__ __launch_bounds__(64 * kMomWaves) void k_moments(int neles, int vsize, const double* __restrict__ f,
+                                                            long ld, const double* __restrict__ cv, double cw,
+                                                            double* __restrict__ out) {
+  constexpr int TPR = EW / 2, ROWS = 64 * kMomWaves / TPR, NB = 32 / EW;
+  __shared__ double red[kMomWaves * 10 * EW];
+  const int sub = threadIdx.x % TPR, row = threadIdx.x / TPR, upt = blockIdx.y;
+  const int eb = blockIdx.x / NB, l0 = (blockIdx.x % NB) * EW + 2 * sub;
+  const long e = static_cast<long>(eb) * 32 + l0;
+  const bool on0 = e < neles, on1 = e + 1 < neles;  // the padding of the last block is not read
+  const double* fb = f + upt * ld + static_cast<long>(eb) * vsize * 32 + l0;
+  double m[4][2] = {};
+  for (int v0 = row; v0 < vsize; v0 += ROWS * kMomUnroll) {
+    double x[kMomUnroll][2], c[kMomUnroll][3];
+#pragma unroll
+    for (int k = 0; k < kMomUnroll; ++k) {
+      const int v = v0 + k * ROWS, vc = min(v, vsize - 1);
+      x[k][0] = (on0 && v < vsize) ? fb[32L * v] : 0.0;
+      x[k][1] = (on1 && v < vsize) ? fb[32L * v + 1] : 0.0;
+#pragma unroll
+      for (int d = 0; d < 3; ++d) c[k][d] = cv[d * static_cast<long>(vsize) + vc];
+    }
+#pragma unroll
+    for (int k = 0; k < kMomUnroll; ++k)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        m[0][h] += x[k][h];
+        m[1][h] += x[k][h] * c[k][0];
+        m[2][h] += x[k][h] * c[k][1];
+        m[3][h] += x[k][h] * c[k][2];
+      }
   }
-  rho *= cw;
-  ux = ux * cw / rho;
-  uy = uy * cw / rho;
-  uz = uz * cw / rho;
-  double T = 0, qx = 0, qy = 0, qz = 0, pxx = 0, pxy = 0, pxz = 0, pyy = 0, pyz = 0, pzz = 0;
-  for (int v = 0; v < vsize; ++v) {
-    const double x = fu[soa_ix(e, v, vsize)];
-    const double cx = cv[v] - ux, cy = cv[vsize + v] - uy, cz = cv[2L * vsize + v] - uz;
-    const double c2 = cx * cx + cy * cy + cz * cz;
-    T += x * c2;
-    qx += x * cx * c2;
-    qy += x * cy * c2;
-    qz += x * cz * c2;
-    pxx += x * cx * cx; pxy += x * cx * cy; pxz += x * cx * cz;
-    pyy += x * cy * cy; pyz += x * cy * cz; pzz += x * cz * cz;
+  mom_reduce<4, EW>(m, red);
+  double rho[2], u[2][3];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    rho[h] = m[0][h] * cw;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) u[h][d] = m[1 + d][h] * cw / rho[h];
   }
-  T = T * cw * (2.0 / 3.0) / rho;
-  const double vals[15] = {rho, ux, uy, uz, T, qx * cw, qy * cw, qz * cw, 2 * pxx * cw, 2 * pxy * cw,
-                           2 * pxz * cw, 2 * pyy * cw, 2 * pyz * cw, 2 * pzz * cw, rho * T};
-  for (int m = 0; m < 15; ++m) out[(static_cast<long>(upt) * 15 + m) * neles + e] = vals[m];
+  // T, qx, qy, qz, Pxx, Pxy, Pxz, Pyy, Pyz, Pzz
+  double q[10][2] = {};
+  for (int v0 = row; v0 < vsize; v0 += ROWS * kMomUnroll) {
+    double x[kMomUnroll][2], c[kMomUnroll][3];
+#pragma unroll
+    for (int k = 0; k < kMomUnroll; ++k) {
+      const int v = v0 + k * ROWS, vc = min(v, vsize - 1);
+      x[k][0] = (on0 && v < vsize) ? fb[32L * v] : 0.0;
+      x[k][1] = (on1 && v < vsize) ? fb[32L * v + 1] : 0.0;
+#pragma unroll
+      for (int d = 0; d < 3; ++d) c[k][d] = cv[d * static_cast<long>(vsize) + vc];
+    }
+#pragma unroll
+    for (int k = 0; k < kMomUnroll; ++k)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const double cx = c[k][0] - u[h][0], cy = c[k][1] - u[h][1], cz = c[k][2] - u[h][2];
+        const double c2 = cx * cx + cy * cy + cz * cz, xc = x[k][h] * c2;
+        const double xx = x[k][h] * cx, xy = x[k][h] * cy, xz = x[k][h] * cz;
+        q[0][h] += xc;
+        q[1][h] += xc * cx; q[2][h] += xc * cy; q[3][h] += xc * cz;
+        q[4][h] += xx * cx; q[5][h] += xx * cy; q[6][h] += xx * cz;
+        q[7][h] += xy * cy; q[8][h] += xy * cz; q[9][h] += xz * cz;
+      }
+  }
+  __syncthreads();  // red is read for m above
+  mom_reduce<10, EW>(q, red);
+  if (row != 0) return;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    if (!(h ? on1 : on0)) continue;
+    const double T = q[0][h] * cw * (2.0 / 3.0) / rho[h];
+    double* o = out + static_cast<long>(upt) * 15 * neles + e + h;
+    const long s = neles;
+    o[0] = rho[h];
+    o[s] = u[h][0]; o[2 * s] = u[h][1]; o[3 * s] = u[h][2];
+    o[4 * s] = T;
+#pragma unroll
+    for (int j = 0; j < 3; ++j) o[(5 + j) * s] = q[1 + j][h] * cw;
+#pragma unroll
+    for (int j = 0; j < 6; ++j) o[(8 + j) * s] = 2 * q[4 + j][h] * cw;
+    o[14 * s] = rho[h] * T;
+  }
 }
 
 static bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
@@ -714,8 +803,18 @@ extern "C" int dgfs_moments(int nupts, int neles, int vsize, const double* f, lo
   if (ld < nparr * vsize) return fail(DGFS_ERR_INVALID_VALUE, "dgfs_moments: leading dimension");
   const long total = static_cast<long>(nupts) * neles;
   if (total == 0) return DGFS_OK;
-  hipLaunchKernelGGL(k_moments, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0,
-                     static_cast<hipStream_t>(stream), nupts, neles, vsize, f, ld, cv, cw, out);
+  const long blocks = nparr / 32, cus = cu_count();
+  auto st = static_cast<hipStream_t>(stream);
+#define DGFS_MOM(EW)                                                                                            \
+  hipLaunchKernelGGL(k_moments<EW>, dim3(static_cast<unsigned>(blocks * (32 / EW)), nupts), dim3(64 * kMomWaves), \
+                     0, st, neles, vsize, f, ld, cv, cw, out)
+  if (blocks * nupts >= cus)
+    DGFS_MOM(32);
+  else if (2 * blocks * nupts >= cus)
+    DGFS_MOM(16);
+  else
+    DGFS_MOM(8);
+#undef DGFS_MOM
   DGFS_LAUNCH_CHECK("dgfs_moments");
   return DGFS_OK;
 }
