@@ -27,6 +27,7 @@
 // exceeds a threshold are evaluated by the exact spectral operator.
 #include <algorithm>
 #include <cmath>
+#include <cstdint>
 #include <cstring>
 #include <memory>
 #include <vector>
@@ -240,6 +241,124 @@ __global__ __launch_bounds__(256) void k_gemm_bf16_big(GemmArgs g) {
       }
 }
 
+// Large-tile FP32 variant: 128 x 64 block tile, 4 waves of 64 x 32 (4 x 2 MFMA
+// tiles), K 32 at a time in K-contiguous LDS rows (As[m][k], Bs[n][k], padded
+// to 36 floats), double buffered: the next tile is in flight in registers
+// while one is multiplied, one barrier per tile.  A lane reads four
+// consecutive k of a row as one 16-byte value and gives MFMA step j the value
+// k = 4 g + j of its lane group g, for A and B alike, so the four steps of a
+// read cover 16 k in another order than step by step.  Two workgroups (55 KB of
+// LDS each) share a CU.  For outputs of at least 128 x 64 with 16-byte
+// aligned operands; the 64 x 64 kernel above stages every value through a
+// bounds-checked scalar load and two barriers per 32 k and ran the network's
+// products (512 x 32 P x 512) at 39 TFLOP/s on MI355X, this one at 82 (P =
+// 256) to 89 (P = 1000).
+constexpr int kFM = 128, kFN = 64, kFK = 32, kFP = kFK + 4;
+
+// this thread's share of an R x 32 operand tile (R rows of op(A) or columns of
+// op(B)): R * 32 / 4 / 256 vectors of 4 consecutive k of one row.  KC: k is the
+// contiguous index in memory, read as vectors; else the lanes run along the
+// rows and read k by k, so that the LDS stores are 16-byte rows either way
+// (vectors along the rows would be scattered into LDS with 16-way conflicts).
+template <int R, bool KC>
+__device__ __forceinline__ void gemm_load(const float* __restrict__ X, long ld, int r0, int rows, int k0, int kend,
+                                          fl4 (&v)[R / 32]) {
+#pragma unroll
+  for (int i = 0; i < R / 32; ++i) {
+    const int e = threadIdx.x + 256 * i;
+    const int r = KC ? e >> 3 : e % R, k = KC ? (e & 7) * 4 : (e / R) * 4;
+    const int gr = r0 + r, gk = k0 + k;
+    const float* p = KC ? X + static_cast<long>(gr) * ld + gk : X + static_cast<long>(gk) * ld + gr;
+    const int left = gr < rows ? kend - gk : 0;  // values of k that exist
+    if (left >= 4) {
+      if constexpr (KC) {
+        v[i] = *reinterpret_cast<const fl4*>(p);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[i][j] = p[j * ld];
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[i][j] = (j < left) ? p[KC ? j : j * ld] : 0.f;
+    }
+  }
+}
+template <int R, bool KC>
+__device__ __forceinline__ void gemm_store(float (*T)[kFP], const fl4 (&v)[R / 32]) {
+#pragma unroll
+  for (int i = 0; i < R / 32; ++i) {
+    const int e = threadIdx.x + 256 * i;
+    const int r = KC ? e >> 3 : e % R, k = KC ? (e & 7) * 4 : (e / R) * 4;
+    *reinterpret_cast<fl4*>(&T[r][k]) = v[i];
+  }
+}
+
+template <bool TA, bool TB>
+__global__ __launch_bounds__(256, 2) void k_gemm_f32_big(GemmArgs g) {
+  __shared__ __attribute__((aligned(16))) float As[2][kFM][kFP];
+  __shared__ __attribute__((aligned(16))) float Bs[2][kFN][kFP];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 15, lg = lane >> 4;
+  const int m0 = blockIdx.y * kFM, n0 = blockIdx.x * kFN;
+  const int wm = (wave >> 1) * 64, wn = (wave & 1) * 32;
+  const int kbeg = blockIdx.z * g.kchunk, kend = min(g.K, kbeg + g.kchunk);
+  fl4 acc[4][2];
+#pragma unroll
+  for (int a = 0; a < 4; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b) acc[a][b] = fl4{0.f, 0.f, 0.f, 0.f};
+  fl4 va[kFM / 32], vb[kFN / 32];
+  gemm_load<kFM, !TA>(g.A, g.lda, m0, g.M, kbeg, kend, va);
+  gemm_load<kFN, TB>(g.B, g.ldb, n0, g.N, kbeg, kend, vb);
+  gemm_store<kFM, !TA>(As[0], va);
+  gemm_store<kFN, TB>(Bs[0], vb);
+  __syncthreads();
+  int cur = 0;
+  for (int k0 = kbeg; k0 < kend; k0 += kFK, cur ^= 1) {
+    const bool more = k0 + kFK < kend;
+    if (more) {
+      gemm_load<kFM, !TA>(g.A, g.lda, m0, g.M, k0 + kFK, kend, va);
+      gemm_load<kFN, TB>(g.B, g.ldb, n0, g.N, k0 + kFK, kend, vb);
+    }
+#pragma unroll
+    for (int s = 0; s < kFK / 16; ++s) {
+      fl4 av[4], bv[2];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) av[t] = *reinterpret_cast<const fl4*>(&As[cur][wm + t * 16 + li][s * 16 + 4 * lg]);
+#pragma unroll
+      for (int t = 0; t < 2; ++t) bv[t] = *reinterpret_cast<const fl4*>(&Bs[cur][wn + t * 16 + li][s * 16 + 4 * lg]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int a = 0; a < 4; ++a)
+#pragma unroll
+          for (int b = 0; b < 2; ++b)
+            acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[a][j], bv[b][j], acc[a][b], 0, 0, 0);
+    }
+    if (more) {  // the other buffer: its readers passed the last barrier
+      gemm_store<kFM, !TA>(As[cur ^ 1], va);
+      gemm_store<kFN, TB>(Bs[cur ^ 1], vb);
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int a = 0; a < 4; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = m0 + wm + a * 16 + 4 * lg + r, col = n0 + wn + b * 16 + li;
+        if (row < g.M && col < g.N) {
+          if (g.part) {
+            g.part[(static_cast<long>(blockIdx.z) * g.M + row) * g.N + col] = acc[a][b][r];
+          } else {
+            float* cp = g.C + static_cast<long>(row) * g.ldc + col;
+            const float v = g.alpha * acc[a][b][r];
+            *cp = (g.beta == 0.f) ? v : v + g.beta * *cp;
+          }
+        }
+      }
+}
+
 __global__ __launch_bounds__(256) void k_gemm_reduce(const float* __restrict__ part, int splits, int M, int N,
                                                      float alpha, float beta, float* C, long ldc) {
   const long i = static_cast<long>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -298,6 +417,46 @@ static int gemm(GemmWs* ws, int transA, int transB, int M, int N, int K, float a
     return DGFS_OK;
   }
   GemmArgs g{A, B, C, nullptr, lda, ldb, ldc, transA, transB, M, N, K, K, alpha, beta};
+  const bool aligned = reinterpret_cast<uintptr_t>(A) % 16 == 0 && reinterpret_cast<uintptr_t>(B) % 16 == 0 &&
+                       lda % 4 == 0 && ldb % 4 == 0;
+  if (!bf16 && M >= kFM && N >= kFN && aligned && (M + kFM - 1) / kFM <= 65535) {
+    // large FP32 outputs; K is split while the tiles are fewer than two per
+    // CU, into chunks of at least 256 (the reduction then reads the partials)
+    const int bx = (N + kFN - 1) / kFN, by = (M + kFM - 1) / kFM;
+    const long tl = static_cast<long>(bx) * by, want = 2L * cu_count();
+    int splits = 1;
+    if (ws && tl < want && K >= 512) splits = static_cast<int>(std::min<long>(want / tl, K / 256));
+    if (splits > 1) {
+      int kchunk = (K + splits - 1) / splits;
+      kchunk = (kchunk + kFK - 1) / kFK * kFK;
+      splits = (K + kchunk - 1) / kchunk;
+      if (splits > 1 && static_cast<size_t>(splits) * M * N <= kGemmPartFloats) {
+        int rc = ws->init();
+        if (rc) return rc;
+        g.kchunk = kchunk;
+        g.part = ws->part;
+      } else {
+        splits = 1;
+      }
+    }
+    const dim3 grid(bx, by, splits);
+    if (transA && transB)
+      hipLaunchKernelGGL((k_gemm_f32_big<true, true>), grid, dim3(256), 0, st, g);
+    else if (transA)
+      hipLaunchKernelGGL((k_gemm_f32_big<true, false>), grid, dim3(256), 0, st, g);
+    else if (transB)
+      hipLaunchKernelGGL((k_gemm_f32_big<false, true>), grid, dim3(256), 0, st, g);
+    else
+      hipLaunchKernelGGL((k_gemm_f32_big<false, false>), grid, dim3(256), 0, st, g);
+    DGFS_LAUNCH_CHECK("gemm_f32");
+    if (splits > 1) {
+      const long tot = static_cast<long>(M) * N;
+      hipLaunchKernelGGL(k_gemm_reduce, dim3(static_cast<unsigned>((tot + 255) / 256)), dim3(256), 0, st, ws->part,
+                         splits, M, N, alpha, beta, C, ldc);
+      DGFS_LAUNCH_CHECK("gemm_reduce");
+    }
+    return DGFS_OK;
+  }
   const int gx = (N + kGT - 1) / kGT, gy = (M + kGT - 1) / kGT;
   // split the reduction when the output has few tiles and K is long
   int splits = 1;
@@ -396,6 +555,205 @@ __global__ __launch_bounds__(256) void k_act_bwd(const float* __restrict__ V, fl
   dZ[i] *= gelu_d(V[i]);
 }
 
+// One layer's channel mixing with FP32 operands, fused:
+//   V = U W + Z R + bias, Znext = act(V)
+// over the rows (m, p) of U and Z.  A wave takes 32 rows: the rows are the A
+// operand of v_mfma_f32_16x16x4f32 (lane i of a group holds row i, channels
+// 16 h + 4 g + j as one 16-byte load), W and R stay in registers as B.  Bound by
+// reading U, Z and writing V, Znext once; as two products and an elementwise
+// pass V was written three times and read twice (P = 256: 42 -> 16 us per
+// layer on MI355X).
+constexpr int kLayRows = 32;
+
+// B operand values of a 32 x 32 matrix X (transposed: X^T) for column tile t:
+// step (h, j) takes row 16 h + 4 g + j
+template <bool TR>
+__device__ __forceinline__ void chan_operand(const float* __restrict__ X, int li, int lg, float (&b)[2][8]) {
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int row = 16 * (k >> 2) + 4 * lg + (k & 3), col = 16 * t + li;
+      b[t][k] = TR ? X[col * kSurWidth + row] : X[row * kSurWidth + col];
+    }
+}
+
+__global__ __launch_bounds__(256) void k_layer_fwd(const float* __restrict__ U, const float* __restrict__ Z,
+                                                   const float* __restrict__ W, const float* __restrict__ R,
+                                                   const float* __restrict__ bias, float* __restrict__ V,
+                                                   float* __restrict__ Zn, long rows, int act) {
+  const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
+  float bw[2][8], br[2][8], bb[2];
+  chan_operand<false>(W, li, lg, bw);
+  chan_operand<false>(R, li, lg, br);
+#pragma unroll
+  for (int t = 0; t < 2; ++t) bb[t] = bias[16 * t + li];
+  const long nw = static_cast<long>(gridDim.x) * 4, nt = rows / kLayRows;
+  for (long w = static_cast<long>(blockIdx.x) * 4 + (threadIdx.x >> 6); w < nt; w += nw) {
+    const long r0 = w * kLayRows;
+    fl4 u[2][2], z[2][2];
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const long o = (r0 + 16 * a + li) * kSurWidth + 16 * h + 4 * lg;
+        u[a][h] = *reinterpret_cast<const fl4*>(U + o);
+        z[a][h] = *reinterpret_cast<const fl4*>(Z + o);
+      }
+    fl4 acc[2][2];
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) acc[a][t] = fl4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+          acc[a][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(u[a][k >> 2][k & 3], bw[t][k], acc[a][t], 0, 0, 0);
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+          acc[a][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(z[a][k >> 2][k & 3], br[t][k], acc[a][t], 0, 0, 0);
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const long o = (r0 + 16 * a + 4 * lg + r) * kSurWidth + 16 * t + li;
+          const float v = acc[a][t][r] + bb[t];
+          V[o] = v;
+          Zn[o] = act ? gelu(v) : v;
+        }
+  }
+}
+
+// The same layer backward, fused: with dV = dZ act'(V) (act = 0: dV = dZ)
+//   dU = dV W^T, dZn = dV R^T, and the block's partial sums of
+//   gW = U^T dV, gR = Z^T dV, gb = sum dV over its rows.
+// dV is formed twice in registers, as A operand (rows on lanes) for dU and dZn
+// and as B operand (channels on lanes) for the weight gradients; nothing but
+// dU and dZn is written per row.  part[block][2 * 32 * 32 + 32]; the partials
+// are summed by k_sum_parts, in a fixed order.  As separate kernels the weight
+// gradients were 32 x 32 products over 512 P rows on 64 workgroups: 670 us per
+// layer at P = 256 on MI355X, 39 us fused.
+constexpr int kLayPart = 2 * kSurWidth * kSurWidth + kSurWidth;
+
+__global__ __launch_bounds__(256) void k_layer_bwd(const float* __restrict__ dZ, const float* __restrict__ V,
+                                                   const float* __restrict__ U, const float* __restrict__ Z,
+                                                   const float* __restrict__ W, const float* __restrict__ R,
+                                                   float* __restrict__ dU, float* __restrict__ dZn,
+                                                   float* __restrict__ part, long rows, int act) {
+  __shared__ float red[kLayPart];
+  const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4, wave = threadIdx.x >> 6;
+  float bw[2][8], br[2][8];
+  chan_operand<true>(W, li, lg, bw);
+  chan_operand<true>(R, li, lg, br);
+  fl4 gw[2][2], gr[2][2];  // [channel tile of U / Z][channel tile of dV]
+  float gb[2] = {0.f, 0.f};
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int t = 0; t < 2; ++t) gw[a][t] = gr[a][t] = fl4{0.f, 0.f, 0.f, 0.f};
+  const long nw = static_cast<long>(gridDim.x) * 4, nt = rows / kLayRows;
+  for (long w = static_cast<long>(blockIdx.x) * 4 + wave; w < nt; w += nw) {
+    const long r0 = w * kLayRows;
+    {
+      fl4 dv[2][2];
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const long o = (r0 + 16 * a + li) * kSurWidth + 16 * h + 4 * lg;
+          dv[a][h] = *reinterpret_cast<const fl4*>(dZ + o);
+          if (act) {
+            const fl4 v = *reinterpret_cast<const fl4*>(V + o);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) dv[a][h][j] *= gelu_d(v[j]);
+          }
+        }
+      fl4 au[2][2], az[2][2];
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) au[a][t] = az[a][t] = fl4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+          for (int t = 0; t < 2; ++t) {
+            const float d = dv[a][k >> 2][k & 3];
+            au[a][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(d, bw[t][k], au[a][t], 0, 0, 0);
+            az[a][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(d, br[t][k], az[a][t], 0, 0, 0);
+          }
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const long o = (r0 + 16 * a + 4 * lg + r) * kSurWidth + 16 * t + li;
+            dU[o] = au[a][t][r];
+            dZn[o] = az[a][t][r];
+          }
+    }
+    // rows 4 s + g on the k index, channels on the lanes
+#pragma unroll
+    for (int s = 0; s < kLayRows / 4; ++s) {
+      float d[2], u[2], z[2];
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const long o = (r0 + 4 * s + lg) * kSurWidth + 16 * t + li;
+        d[t] = dZ[o];
+        if (act) d[t] *= gelu_d(V[o]);
+        u[t] = U[o];
+        z[t] = Z[o];
+        gb[t] += d[t];
+      }
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          gw[a][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(u[a], d[t], gw[a][t], 0, 0, 0);
+          gr[a][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(z[a], d[t], gr[a][t], 0, 0, 0);
+        }
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    gb[t] += __shfl_xor(gb[t], 16);
+    gb[t] += __shfl_xor(gb[t], 32);
+  }
+  for (int w = 0; w < 4; ++w) {  // the waves in turn
+    if (wave == w) {
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int o = (16 * a + 4 * lg + r) * kSurWidth + 16 * t + li;
+            red[o] = (w ? red[o] : 0.f) + gw[a][t][r];
+            red[kSurWidth * kSurWidth + o] = (w ? red[kSurWidth * kSurWidth + o] : 0.f) + gr[a][t][r];
+          }
+      if (lg == 0)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          const int o = 2 * kSurWidth * kSurWidth + 16 * t + li;
+          red[o] = (w ? red[o] : 0.f) + gb[t];
+        }
+    }
+    __syncthreads();
+  }
+  for (int i = threadIdx.x; i < kLayPart; i += 256) part[static_cast<long>(blockIdx.x) * kLayPart + i] = red[i];
+}
+
 // Per-channel and per-mode reductions of the backward pass, two stages
 // (block partials, then one block) so the sums are deterministic.
 //   kind 0: out[c]     = sum_{m,p} X[m][p][c]                 (bias)
@@ -439,32 +797,53 @@ __global__ __launch_bounds__(256) void k_chan_reduce(ChanRedArgs a) {
   }
 }
 
-__global__ __launch_bounds__(64) void k_sum_parts(const float* __restrict__ part, int nparts, int width,
-                                                 float* __restrict__ out) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= width) return;
+// out[c] = sum_k part[k][c]: 32 columns per block, 32 rows of threads over k,
+// then the rows in order (one thread per column summed 240 partials one after
+// another: 54 us, 5 us this way)
+__global__ __launch_bounds__(1024) void k_sum_parts(const float* __restrict__ part, int nparts, int width,
+                                                   float* __restrict__ out) {
+  __shared__ float red[32][33];
+  const int lc = threadIdx.x & 31, row = threadIdx.x >> 5, c = blockIdx.x * 32 + lc;
   float s = 0.f;
-  for (int k = 0; k < nparts; ++k) s += part[static_cast<long>(k) * width + c];
-  out[c] = s;
+  if (c < width)
+    for (int k = row; k < nparts; k += 32) s += part[static_cast<long>(k) * width + c];
+  red[row][lc] = s;
+  __syncthreads();
+  if (row == 0 && c < width) {
+    float t = 0.f;
+    for (int k = 0; k < 32; ++k) t += red[k][lc];
+    out[c] = t;
+  }
 }
 
-// dE[m][c] = sum_p dZ0[m][p][c]
+// dE[m][c] = sum_p dZ0[m][p][c]: a block per mode, 8 rows of threads over p
 __global__ __launch_bounds__(256) void k_mode_reduce(const float* __restrict__ dZ, float* __restrict__ out, int P) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;  // over (m, c)
-  if (i >= kSurModes * kSurWidth) return;
-  const int c = i % kSurWidth, m = i / kSurWidth;
+  __shared__ float red[8][kSurWidth];
+  const int c = threadIdx.x & 31, row = threadIdx.x >> 5, m = blockIdx.x;
   float s = 0.f;
-  for (int p = 0; p < P; ++p) s += dZ[(static_cast<long>(m) * P + p) * kSurWidth + c];
-  out[i] = s;
+  for (int p = row; p < P; p += 8) s += dZ[(static_cast<long>(m) * P + p) * kSurWidth + c];
+  red[row][c] = s;
+  __syncthreads();
+  if (row == 0) {
+    float t = 0.f;
+    for (int k = 0; k < 8; ++k) t += red[k][c];
+    out[m * kSurWidth + c] = t;
+  }
 }
 
-// dbout[m] = sum_p dout[p][m]
-__global__ __launch_bounds__(256) void k_bout_reduce(const float* __restrict__ dout, float* __restrict__ out, int P) {
-  const int m = blockIdx.x * blockDim.x + threadIdx.x;
-  if (m >= kSurModes) return;
+// dbout[m] = sum_p dout[p][m]: 32 modes per block, 32 rows of threads over p
+__global__ __launch_bounds__(1024) void k_bout_reduce(const float* __restrict__ dout, float* __restrict__ out, int P) {
+  __shared__ float red[32][33];
+  const int lm = threadIdx.x & 31, row = threadIdx.x >> 5, m = blockIdx.x * 32 + lm;
   float s = 0.f;
-  for (int p = 0; p < P; ++p) s += dout[static_cast<long>(p) * kSurModes + m];
-  out[m] = s;
+  for (int p = row; p < P; p += 32) s += dout[static_cast<long>(p) * kSurModes + m];
+  red[row][lm] = s;
+  __syncthreads();
+  if (row == 0) {
+    float t = 0.f;
+    for (int k = 0; k < 32; ++k) t += red[k][lm];
+    out[m] = t;
+  }
 }
 
 __global__ __launch_bounds__(256) void k_adam(float* __restrict__ th, const float* __restrict__ g,
@@ -969,13 +1348,20 @@ static SurHandle* as_sur(void* p) {
 
 static inline unsigned nblk(long tot) { return static_cast<unsigned>((tot + 255) / 256); }
 constexpr int kRedBlocks = 240;
+// workgroups of the fused layer kernels: four waves of kLayRows rows each, and
+// at most two per CU backward, whose partial sums are read back per workgroup
+constexpr unsigned kLayBwdBlocks = 512;
+static unsigned lay_blocks(int P) {
+  static_assert(kSurModes % (4 * kLayRows) == 0, "whole rows for every wave");
+  return static_cast<unsigned>(static_cast<long>(kSurModes) * P / (4 * kLayRows));
+}
 
 static int chan_reduce(SurHandle* h, int kind, const float* X, const float* Y, const float* xin, const float* lt,
                        int P, float* out, hipStream_t st) {
   ChanRedArgs ca{X, Y, xin, lt, nullptr, h->part, P, kind};
   hipLaunchKernelGGL(k_chan_reduce, dim3(kRedBlocks), dim3(256), 0, st, ca);
   DGFS_LAUNCH_CHECK("chan_reduce");
-  hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(64), 0, st, h->part, kRedBlocks, kSurWidth, out);
+  hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(1024), 0, st, h->part, kRedBlocks, kSurWidth, out);
   DGFS_LAUNCH_CHECK("sum_parts");
   return DGFS_OK;
 }
@@ -992,6 +1378,12 @@ static int sur_forward(SurHandle* h, const float* th, const float* x, const floa
     const float* bias = R + kSurWidth * kSurWidth;
     int rc = gemm(&h->ws, 0, 0, kSurModes, kSurWidth * P, kSurModes, 1.f, K, kSurModes, h->Z[l],
                   static_cast<long>(kSurWidth) * P, 0.f, h->U[l], static_cast<long>(kSurWidth) * P, bf16, st);
+    if (!rc && !bf16) {
+      hipLaunchKernelGGL(k_layer_fwd, dim3(lay_blocks(P)), dim3(256), 0, st, h->U[l], h->Z[l], W, R, bias, h->Vv[l],
+                         h->Z[l + 1], static_cast<long>(kSurModes) * P, l + 1 < kSurLayers ? 1 : 0);
+      DGFS_LAUNCH_CHECK("layer_fwd");
+      continue;
+    }
     if (!rc) rc = gemm(&h->ws, 0, 0, kSurModes * P, kSurWidth, kSurWidth, 1.f, h->U[l], kSurWidth, W, kSurWidth, 0.f,
                        h->Vv[l], kSurWidth, bf16, st);
     if (!rc) rc = gemm(&h->ws, 0, 0, kSurModes * P, kSurWidth, kSurWidth, 1.f, h->Z[l], kSurWidth, R, kSurWidth, 1.f,
@@ -1023,7 +1415,7 @@ static int sur_backward(SurHandle* h, const float* th, const float* dout, float*
     // dPout[c] = sum_{m,p} Z4[m][p][c] dout[p][m] (kind 2 with xin = dout)
     int rc = chan_reduce(h, 2, h->Z[kSurLayers], nullptr, dout, nullptr, P, grad + kSurOffPout, st);
     if (rc) return rc;
-    hipLaunchKernelGGL(k_bout_reduce, dim3(nblk(kSurModes)), dim3(256), 0, st, dout, grad + kSurOffBout, P);
+    hipLaunchKernelGGL(k_bout_reduce, dim3(kSurModes / 32), dim3(1024), 0, st, dout, grad + kSurOffBout, P);
     DGFS_LAUNCH_CHECK("bout_reduce");
   }
   float* dZ = h->dA;    // gradient w.r.t. Z_{l+1}
@@ -1036,6 +1428,23 @@ static int sur_backward(SurHandle* h, const float* th, const float* dout, float*
     float* gW = gK + static_cast<long>(kSurModes) * kSurModes;
     float* gR = gW + kSurWidth * kSurWidth;
     float* gb = gR + kSurWidth * kSurWidth;
+    if (!bf16) {
+      const unsigned nb = std::min<unsigned>(lay_blocks(P), kLayBwdBlocks);
+      hipLaunchKernelGGL(k_layer_bwd, dim3(nb), dim3(256), 0, st, dZ, h->Vv[l], h->U[l], h->Z[l], W, R, h->dU, dZn,
+                         h->part, static_cast<long>(kSurModes) * P, l + 1 < kSurLayers ? 1 : 0);
+      DGFS_LAUNCH_CHECK("layer_bwd");
+      // gW, gR and gb follow each other in the parameter vector as in a partial
+      hipLaunchKernelGGL(k_sum_parts, dim3((kLayPart + 31) / 32), dim3(1024), 0, st, h->part, static_cast<int>(nb),
+                         kLayPart, gW);
+      DGFS_LAUNCH_CHECK("layer_grads");
+      int rc = gemm(&h->ws, 0, 1, kSurModes, kSurModes, kSurWidth * P, 1.f, h->dU, ld, h->Z[l], ld, 0.f, gK,
+                    kSurModes, false, st);
+      if (!rc) rc = gemm(&h->ws, 1, 0, kSurModes, kSurWidth * P, kSurModes, 1.f, K, kSurModes, h->dU, ld, 1.f, dZn, ld,
+                         false, st);
+      if (rc) return rc;
+      std::swap(dZ, dZn);
+      continue;
+    }
     if (l + 1 < kSurLayers) {
       hipLaunchKernelGGL(k_act_bwd, dim3(nblk(act)), dim3(256), 0, st, h->Vv[l], dZ, act);
       DGFS_LAUNCH_CHECK("act_bwd");
@@ -1061,7 +1470,7 @@ static int sur_backward(SurHandle* h, const float* th, const float* dout, float*
   int rc = chan_reduce(h, 2, dZ, nullptr, h->x_last, nullptr, P, grad + kSurOffP0, st);
   if (!rc) rc = chan_reduce(h, 3, dZ, nullptr, nullptr, h->lt_last, P, grad + kSurOffP1, st);
   if (rc) return rc;
-  hipLaunchKernelGGL(k_mode_reduce, dim3(nblk(kSurModes * kSurWidth)), dim3(256), 0, st, dZ, grad + kSurOffE, P);
+  hipLaunchKernelGGL(k_mode_reduce, dim3(kSurModes), dim3(256), 0, st, dZ, grad + kSurOffE, P);
   DGFS_LAUNCH_CHECK("mode_reduce");
   return DGFS_OK;
 }
@@ -1205,7 +1614,8 @@ extern "C" int dgfs_sur_create(const dgfs_sur_desc* d, void** out) {
   DGFS_HIP_TRY(hipMalloc(&h->dA, act));
   DGFS_HIP_TRY(hipMalloc(&h->dB, act));
   DGFS_HIP_TRY(hipMalloc(&h->dU, act));
-  DGFS_HIP_TRY(hipMalloc(&h->part, static_cast<size_t>(kRedBlocks) * kSurWidth * sizeof(float)));
+  DGFS_HIP_TRY(hipMalloc(&h->part, std::max(static_cast<size_t>(kRedBlocks) * kSurWidth,
+                                            static_cast<size_t>(kLayBwdBlocks) * kLayPart) * sizeof(float)));
   *out = h.release();
   return DGFS_OK;
 }

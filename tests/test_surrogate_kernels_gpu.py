@@ -1,0 +1,69 @@
+"""The surrogate's large-tile FP32 GEMM and fused layer kernels at the sizes
+where they can go wrong: edges of the 128 x 64 x 32 tiles, short and split
+reductions, every transposition, unaligned leading dimensions (which take the
+general kernel), and batches of one and odd sizes through a whole layer stack.
+FP32 sums of K products: |error| <= sqrt(K) 2^-22 |A| |B| entrywise bound of a
+random-sign sum with a margin of 4."""
+import numpy as np
+import pytest
+
+from oracle import surrogate as S
+
+pytestmark = pytest.mark.gpu
+
+
+def say(*a):
+    print(*a, flush=True)
+
+
+@pytest.mark.parametrize("M,N,K", [(128, 64, 32), (129, 65, 33), (200, 100, 7), (512, 96, 512), (131, 67, 4100),
+                                   (128, 64, 1), (300, 64, 1030)])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_gemm_f32_edges(M, N, K, ta, tb, device):
+    import torch
+    from dgfs_hip import surrogate as D
+    rng = np.random.default_rng(M + K)
+    A, B = rng.normal(size=(M, K)).astype(np.float32), rng.normal(size=(K, N)).astype(np.float32)
+    C0 = rng.normal(size=(M, N)).astype(np.float32)
+    for pad in (0, 3):  # leading dimensions rounded up to 4, or odd
+        def store(X):
+            ld = -(-X.shape[1] // 4) * 4 + pad
+            out = np.full((X.shape[0], ld), np.nan, dtype=np.float32)
+            out[:, :X.shape[1]] = X
+            return torch.as_tensor(out, device=device), ld
+        At, lda = store(A.T if ta else A)
+        Bt, ldb = store(B.T if tb else B)
+        Ct = torch.as_tensor(C0, device=device)
+        say("gemm", M, N, K, ta, tb, pad)
+        D.gemm(ta, tb, M, N, K, 0.5, At, lda, Bt, ldb, 2.0, Ct, N, bf16=False,
+               stream=torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        ref = 0.5 * (A.astype(np.float64) @ B.astype(np.float64)) + 2.0 * C0
+        err = np.abs(Ct.cpu().numpy() - ref)
+        assert err.max() <= 4 * np.sqrt(K) * 2.0 ** -22 * np.abs(A).max() * np.abs(B).max() + 4 * 2.0 ** -23 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("P", [1, 3, 17])
+def test_layers_small_batches(P, device):
+    """Forward and every gradient at small and odd batches against the FP64
+    checker: 1e-5 of each output's norm (FP32 sums of up to 512 P terms)."""
+    import torch
+    from dgfs_hip.surrogate import SpectralSurrogate
+    sur = SpectralSurrogate(8, 5.0, (10.0 / 8) ** 3, 0.38, 1.0, max_batch=32, device=device, seed=3)
+    rng = np.random.default_rng(P)
+    x, lt = rng.normal(size=(P, 512)), rng.normal(size=P) * 0.2
+    dout = rng.normal(size=(P, 512))
+    f32 = lambda a: torch.as_tensor(a, dtype=torch.float32, device=device).contiguous()
+    xt, ltt, dt = f32(x), f32(lt), f32(dout)
+    out = torch.empty((P, 512), dtype=torch.float32, device=device)
+    say("layers", P)
+    sur.forward(xt, ltt, P, out)
+    sur.backward(dt)
+    torch.cuda.synchronize()
+    th = sur.params_bf16.cpu().numpy().astype(np.float64)
+    ref, cache = S.forward(th, xt.cpu().numpy(), ltt.cpu().numpy())
+    g = S.backward(th, cache, dt.cpu().numpy().astype(np.float64))
+    e = np.linalg.norm(out.cpu().numpy() - ref) / np.linalg.norm(ref)
+    eg = np.linalg.norm(sur.grad.cpu().numpy() - g) / np.linalg.norm(g)
+    say("  forward", e, "gradient", eg)
+    assert e < 1e-5 and eg < 1e-5
