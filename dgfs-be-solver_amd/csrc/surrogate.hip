@@ -903,49 +903,78 @@ __device__ __forceinline__ void herm_table(double* V, double c0, double h, doubl
   }
 }
 
-__device__ __forceinline__ double block_sum(double v, double* red) {
-  const int tid = threadIdx.x;
-  red[tid] = v;
+// totals of NQ values per thread over a workgroup of NT threads; red holds
+// NT / 64 * NQ doubles and is free on return
+template <int NQ, int NT>
+__device__ __forceinline__ void block_sums(double (&s)[NQ], double* red) {
+#pragma unroll
+  for (int j = 0; j < NQ; ++j)
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) s[j] += __shfl_xor(s[j], d);
+  if ((threadIdx.x & 63) == 0)
+#pragma unroll
+    for (int j = 0; j < NQ; ++j) red[(threadIdx.x >> 6) * NQ + j] = s[j];
   __syncthreads();
-  for (int s = blockDim.x / 2; s > 0; s >>= 1) {
-    if (tid < s) red[tid] += red[tid + s];
-    __syncthreads();
+#pragma unroll
+  for (int j = 0; j < NQ; ++j) {
+    double t = 0.0;
+#pragma unroll
+    for (int w = 0; w < NT / 64; ++w) t += red[w * NQ + j];
+    s[j] = t;
   }
-  const double r = red[0];
   __syncthreads();
-  return r;
 }
 
 // Linv[d] = L_d^{-1}, L_d the Cholesky factor of the per-axis Gram matrix
-// G_d = (h/s) V_d^T V_d (one thread per axis; work holds 3 x 8 x 8 doubles).
+// G_d = (h/s) V_d^T V_d (work holds 3 x 8 x 8 doubles).  The Gram sums take a
+// thread each; the 8 x 8 factorisation is one thread per axis in registers
+// (with its operands in LDS every step waited for the one before: the encoder
+// spent a third of its time there).
 // The 1D functions V_d L_d^{-T} are orthonormal on the grid with the measure
 // dx' = h/s, so their tensor products are orthonormal in 3D.
 template <int N>
 __device__ void herm_chol_inv(const double* V, double hs, double* Linv, double* work) {
-  if (threadIdx.x < 3) {
-    const int d = threadIdx.x;
+  for (int e = threadIdx.x; e < 3 * kSurD * kSurD; e += blockDim.x) {
+    const int d = e / (kSurD * kSurD), a = (e / kSurD) % kSurD, b = e % kSurD;
+    if (b > a) continue;
     const double* Vd = V + d * N * kSurD;
-    double* Lw = work + d * kSurD * kSurD;
-    double* Li = Linv + d * kSurD * kSurD;
+    double s = 0.0;
+    for (int i = 0; i < N; ++i) s += Vd[i * kSurD + a] * Vd[i * kSurD + b];
+    work[e] = s * hs;
+  }
+  __syncthreads();
+  if (threadIdx.x < 3) {
+    double G[kSurD][kSurD], rd[kSurD];
+#pragma unroll
     for (int a = 0; a < kSurD; ++a)
-      for (int b = 0; b <= a; ++b) {
-        double s = 0.0;
-        for (int i = 0; i < N; ++i) s += Vd[i * kSurD + a] * Vd[i * kSurD + b];
-        s *= hs;
-        for (int k = 0; k < b; ++k) s -= Lw[a * kSurD + k] * Lw[b * kSurD + k];
-        Lw[a * kSurD + b] = (a == b) ? sqrt(fmax(s, 1e-300)) : s / Lw[b * kSurD + b];
+#pragma unroll
+      for (int b = 0; b <= a; ++b) G[a][b] = work[threadIdx.x * kSurD * kSurD + a * kSurD + b];
+#pragma unroll
+    for (int b = 0; b < kSurD; ++b) {
+#pragma unroll
+      for (int k = 0; k < b; ++k) G[b][b] -= G[b][k] * G[b][k];
+      rd[b] = 1.0 / sqrt(fmax(G[b][b], 1e-300));
+#pragma unroll
+      for (int a = b + 1; a < kSurD; ++a) {
+#pragma unroll
+        for (int k = 0; k < b; ++k) G[a][b] -= G[a][k] * G[b][k];
+        G[a][b] *= rd[b];
       }
+    }
     // forward substitution for the inverse of the lower triangle
-    for (int c = 0; c < kSurD; ++c)
+    double* Li = Linv + threadIdx.x * kSurD * kSurD;
+#pragma unroll
+    for (int c = 0; c < kSurD; ++c) {
+      double x[kSurD];
+#pragma unroll
       for (int a = 0; a < kSurD; ++a) {
-        if (a < c) {
-          Li[a * kSurD + c] = 0.0;
-          continue;
-        }
-        double s = (a == c) ? 1.0 : 0.0;
-        for (int k = c; k < a; ++k) s -= Lw[a * kSurD + k] * Li[k * kSurD + c];
-        Li[a * kSurD + c] = s / Lw[a * kSurD + a];
+        double t = (a == c) ? 1.0 : 0.0;
+#pragma unroll
+        for (int k = c; k < a; ++k) t -= G[a][k] * x[k];
+        x[a] = (a < c) ? 0.0 : t * rd[a];
+        Li[a * kSurD + c] = x[a];
       }
+    }
   }
   __syncthreads();
 }
@@ -988,12 +1017,14 @@ __device__ void kron3(const double* Linv, bool transpose, double* in, double* tm
 // the span, so the modes stay bounded and a mean-square error of the modes is
 // the L2 error of the decoded field.
 template <int N>
+__device__ void herm_project_rest(const double* V, const double* Linv, double* t1, double* t2, double* b3,
+                                  double factor, float* out, float shift0);
+
+template <int N>
 __device__ void herm_project(const double* __restrict__ g, const double* V, const double* Linv, double* t1,
                              double* t2, double* b3, double factor, float* out, float shift0) {
   constexpr int NN = N * N;
   const double* Vx = V;
-  const double* Vy = V + N * kSurD;
-  const double* Vz = V + 2 * N * kSurD;
   // t1[a][j][k]: each thread owns columns jk and reads every g value once,
   // accumulating all kSurD x-modes of it
   for (int jk = threadIdx.x; jk < NN; jk += blockDim.x) {
@@ -1008,6 +1039,16 @@ __device__ void herm_project(const double* __restrict__ g, const double* V, cons
 #pragma unroll
     for (int a = 0; a < kSurD; ++a) t1[a * NN + jk] = acc[a];
   }
+  herm_project_rest<N>(V, Linv, t1, t2, b3, factor, out, shift0);
+}
+
+// the other two axes of the projection, from t1[a][j][k] (not yet synchronised)
+template <int N>
+__device__ void herm_project_rest(const double* V, const double* Linv, double* t1, double* t2, double* b3,
+                                  double factor, float* out, float shift0) {
+  constexpr int NN = N * N;
+  const double* Vy = V + N * kSurD;
+  const double* Vz = V + 2 * N * kSurD;
   __syncthreads();
   for (int e = threadIdx.x; e < kSurD * kSurD * N; e += blockDim.x) {  // t2[a][b][k]
     const int a = e / (kSurD * N), rem = e - a * kSurD * N, b = rem / N, k = rem - b * N;
@@ -1037,9 +1078,17 @@ constexpr size_t enc_lds_doubles() {
          3 * kSurD * kSurD + kSurModes + 256;
 }
 
+// A thread owns columns (j, k) and walks along x, so a value's abscissae and
+// basis factors are one LDS row for all of its columns; f is read twice, once
+// for the moments (the frame) and once for the x-modes and the indicator
+// together.  The Maxwellian is the product of the tables' order-0 columns, not
+// an exp per velocity.  Bound by reading f (2 x 8 n bytes per point) and by the
+// 8 FP64 multiply-adds per value: 1000 points at 32^3, 704 -> 253 us on MI355X.
+constexpr int kEncThreads = 512;
+
 template <int N>
-__global__ __launch_bounds__(256) void k_sur_encode(EncArgs a) {
-  constexpr int n = N * N * N, NN = N * N;
+__global__ __launch_bounds__(kEncThreads) void k_sur_encode(EncArgs a) {
+  constexpr int n = N * N * N, NN = N * N, NT = kEncThreads;
   extern __shared__ double sm[];
   double* t1 = sm;                          // kSurD * N * N
   double* t2 = t1 + kSurD * NN;             // kSurD * kSurD * N
@@ -1052,59 +1101,79 @@ __global__ __launch_bounds__(256) void k_sur_encode(EncArgs a) {
   const double pi = 3.14159265358979323846;
   for (int pt = blockIdx.x; pt < a.npts; pt += gridDim.x) {
     const double* f = a.f + static_cast<size_t>(pt) * n;
-    double s0 = 0, s1 = 0, s2 = 0, s3 = 0, s4 = 0;
-    for (int r = threadIdx.x; r < n; r += blockDim.x) {
-      const double cx = c0 + (r / NN) * hh, cy = c0 + ((r / N) % N) * hh, cz = c0 + (r % N) * hh, v = f[r];
-      s0 += v;
-      s1 += v * cx;
-      s2 += v * cy;
-      s3 += v * cz;
-      s4 += v * (cx * cx + cy * cy + cz * cz);
+    double m[5] = {0, 0, 0, 0, 0};
+    for (int jk = threadIdx.x; jk < NN; jk += NT) {
+      const double cy = c0 + (jk / N) * hh, cz = c0 + (jk % N) * hh;
+      double a0 = 0, a1 = 0, a2 = 0;
+#pragma unroll 8
+      for (int i = 0; i < N; ++i) {
+        const double v = f[i * NN + jk], cx = c0 + i * hh, vc = v * cx;
+        a0 += v;
+        a1 += vc;
+        a2 += vc * cx;
+      }
+      m[0] += a0;
+      m[1] += a1;
+      m[2] += a0 * cy;
+      m[3] += a0 * cz;
+      m[4] += a2 + a0 * (cy * cy + cz * cz);
     }
-    const double rho = block_sum(s0, red) * a.cw;
-    const double ux = block_sum(s1, red) * a.cw / rho;
-    const double uy = block_sum(s2, red) * a.cw / rho;
-    const double uz = block_sum(s3, red) * a.cw / rho;
-    const double T = (2.0 / 3.0) * (block_sum(s4, red) * a.cw / rho - (ux * ux + uy * uy + uz * uz));
+    block_sums<5, NT>(m, red);
+    const double rho = m[0] * a.cw;
+    const double ux = m[1] * a.cw / rho, uy = m[2] * a.cw / rho, uz = m[3] * a.cw / rho;
+    const double T = (2.0 / 3.0) * (m[4] * a.cw / rho - (ux * ux + uy * uy + uz * uz));
     const double Mn = rho / pow(pi * T, 1.5);
-    double d2 = 0, f2 = 0;
-    for (int r = threadIdx.x; r < n; r += blockDim.x) {
-      const double cx = c0 + (r / NN) * hh - ux, cy = c0 + ((r / N) % N) * hh - uy, cz = c0 + (r % N) * hh - uz;
-      const double M = Mn * exp(-(cx * cx + cy * cy + cz * cz) / T), v = f[r];
-      d2 += (v - M) * (v - M);
-      f2 += v * v;
+    const double s = sqrt(0.5 * T), hs = hh / s;
+    herm_table(V, c0, hh, ux, s, N);
+    herm_table(V + N * kSurD, c0, hh, uy, s, N);
+    herm_table(V + 2 * N * kSurD, c0, hh, uz, s, N);
+    __syncthreads();
+    double ds[2] = {0, 0};  // sums of (f - M)^2 and f^2
+    for (int jk = threadIdx.x; jk < NN; jk += NT) {
+      const double My = Mn * V[(N + jk / N) * kSurD] * V[(2 * N + jk % N) * kSurD];
+      double acc[kSurD];
+#pragma unroll
+      for (int q = 0; q < kSurD; ++q) acc[q] = 0.0;
+#pragma unroll 8
+      for (int i = 0; i < N; ++i) {
+        const double v = f[i * NN + jk];
+        const double* Vi = V + i * kSurD;
+        const double d = v - My * Vi[0];
+        ds[0] += d * d;
+        ds[1] += v * v;
+#pragma unroll
+        for (int q = 0; q < kSurD; ++q) acc[q] += v * Vi[q];
+      }
+      if (a.x) {
+#pragma unroll
+        for (int q = 0; q < kSurD; ++q) t1[q * NN + jk] = acc[q];
+      }
     }
-    const double ind = sqrt(block_sum(d2, red) / block_sum(f2, red));
+    block_sums<2, NT>(ds, red);
     if (threadIdx.x == 0) {
       double* mo = a.mom + static_cast<size_t>(pt) * 8;
-      mo[0] = rho; mo[1] = ux; mo[2] = uy; mo[3] = uz; mo[4] = T; mo[5] = ind; mo[6] = 0; mo[7] = 0;
+      mo[0] = rho; mo[1] = ux; mo[2] = uy; mo[3] = uz; mo[4] = T; mo[5] = sqrt(ds[0] / ds[1]); mo[6] = 0; mo[7] = 0;
       if (a.lt) a.lt[pt] = static_cast<float>(log(T));
     }
     if (a.x) {
-      const double s = sqrt(0.5 * T), hs = hh / s;
-      herm_table(V, c0, hh, ux, s, N);
-      herm_table(V + N * kSurD, c0, hh, uy, s, N);
-      herm_table(V + 2 * N * kSurD, c0, hh, uz, s, N);
-      __syncthreads();
       herm_chol_inv<N>(V, hs, Linv, work);
       // f = M is the 000 basis function: its coefficient is prod_d L_d[0][0],
       // subtracted so that equilibrium maps to zero
       const double c000 = 1.0 / (Linv[0] * Linv[kSurD * kSurD] * Linv[2 * kSurD * kSurD]);
-      herm_project<N>(f, V, Linv, t1, t2, b3, hs * hs * hs / Mn, a.x + static_cast<size_t>(pt) * kSurModes,
-                      static_cast<float>(c000));
+      herm_project_rest<N>(V, Linv, t1, t2, b3, hs * hs * hs / Mn, a.x + static_cast<size_t>(pt) * kSurModes,
+                           static_cast<float>(c000));
       // second indicator: the share of f's norm in the modes of total degree
       // >= 4 (zero for Maxwellians carrying the heat-flux and stress modes of
       // Grad's 13-moment description)
-      double hi = 0.0, all = 0.0;
-      for (int e = threadIdx.x; e < kSurModes; e += blockDim.x) {
+      double hv[2] = {0, 0};
+      for (int e = threadIdx.x; e < kSurModes; e += NT) {
         const int deg = e / (kSurD * kSurD) + (e / kSurD) % kSurD + e % kSurD;
         const double v = b3[e];
-        all += v * v;
-        if (deg >= 4) hi += v * v;
+        hv[1] += v * v;
+        if (deg >= 4) hv[0] += v * v;
       }
-      hi = block_sum(hi, red);
-      all = block_sum(all, red);
-      if (threadIdx.x == 0) a.mom[static_cast<size_t>(pt) * 8 + 6] = sqrt(hi / all);
+      block_sums<2, NT>(hv, red);
+      if (threadIdx.x == 0) a.mom[static_cast<size_t>(pt) * 8 + 6] = sqrt(hv[0] / hv[1]);
     }
     __syncthreads();
   }
@@ -1158,18 +1227,28 @@ struct DecArgs {
   double* Q;         // [npts][n]
   double L, gamma, prefac;
   int nidx;
+  // FP64 projection onto the collision invariants, or none
+  int project;
+  double cw;
+  double Ainv[25];
 };
 
+// A thread owns columns (j, k): the y and z sums of a column's eight x-modes
+// stay in its registers and the x sum gives its Q values.  With the projection
+// the values are formed twice, first for the moments and then, corrected, to
+// be written: Q is written once and never read (decode and the separate
+// projection moved 4 x 8 n bytes per point: 402 -> 145 us per 1000 points at
+// 32^3 on MI355X).
 template <int N>
-__global__ __launch_bounds__(256) void k_sur_decode(DecArgs a) {
-  constexpr int n = N * N * N, NN = N * N;
+__global__ __launch_bounds__(256, 2) void k_sur_decode(DecArgs a) {
+  constexpr int n = N * N * N, NN = N * N, NT = 256, CPT = (NN + NT - 1) / NT;
   extern __shared__ double sm[];
-  double* s2 = sm;                      // kSurD * N * N   [a][j][k]
-  double* s1 = s2 + kSurD * NN;         // kSurD * kSurD * N [a][b][k] (>= 512)
+  double* s1 = sm;                      // kSurD * kSurD * N [a][b][k] (>= 512)
   double* V = s1 + kSurD * kSurD * N;   // 3 * N * kSurD
   double* bb = V + 3 * N * kSurD;       // 512
   double* Linv = bb + kSurModes;        // 3 * 64
   double* work = Linv + 3 * kSurD * kSurD;  // 3 * 64
+  double* red = work + 3 * kSurD * kSurD;   // NT / 64 * 5
   const double hh = 2.0 * a.L / N, c0 = -a.L + 0.5 * hh;
   const double pi = 3.14159265358979323846;
   for (int i = blockIdx.x; i < a.nidx; i += gridDim.x) {
@@ -1181,7 +1260,7 @@ __global__ __launch_bounds__(256) void k_sur_decode(DecArgs a) {
     herm_table(V + 2 * N * kSurD, c0, hh, uz, s, N);
     const double scale = a.prefac * rho * pow(T, 0.5 * a.gamma);
     const float* yi = a.y + static_cast<size_t>(i) * kSurModes;
-    for (int e = threadIdx.x; e < kSurModes; e += blockDim.x) bb[e] = scale * static_cast<double>(yi[e]);
+    for (int e = threadIdx.x; e < kSurModes; e += NT) bb[e] = scale * static_cast<double>(yi[e]);
     __syncthreads();
     herm_chol_inv<N>(V, hh / s, Linv, work);
     kron3(Linv, true, bb, s1, bb);
@@ -1192,29 +1271,87 @@ __global__ __launch_bounds__(256) void k_sur_decode(DecArgs a) {
       bb[0] = 0.0; bb[kSurD * kSurD] = 0.0; bb[kSurD] = 0.0; bb[1] = 0.0;
     }
     __syncthreads();
-    for (int e = threadIdx.x; e < kSurD * kSurD * N; e += blockDim.x) {  // s1[a][b][k]
+    for (int e = threadIdx.x; e < kSurD * kSurD * N; e += NT) {  // s1[a][b][k]
       const int ab = e / N, k = e - ab * N;
       double t = 0.0;
       for (int c = 0; c < kSurD; ++c) t += bb[ab * kSurD + c] * V[2 * N * kSurD + k * kSurD + c];
       s1[e] = t;
     }
     __syncthreads();
-    for (int e = threadIdx.x; e < kSurD * NN; e += blockDim.x) {  // s2[a][j][k]
-      const int aa = e / NN, jk = e - aa * NN, j = jk / N, k = jk - j * N;
-      double t = 0.0;
-      for (int b = 0; b < kSurD; ++b) t += s1[(aa * kSurD + b) * N + k] * V[N * kSurD + j * kSurD + b];
-      s2[e] = t;
-    }
-    __syncthreads();
     // the tables carry the per-axis Gaussian factors of M
     const double Mn = rho / pow(pi * T, 1.5);
-    double* Q = a.Q + static_cast<size_t>(pt) * n;
-    for (int jk = threadIdx.x; jk < NN; jk += blockDim.x) {
+    double x[CPT][kSurD];  // x-modes of the thread's columns
+#pragma unroll
+    for (int c = 0; c < CPT; ++c) {
+      const int jk = threadIdx.x + c * NT;
+      if (jk < NN) {
+        const int j = jk / N, k = jk - j * N;
+#pragma unroll
+        for (int q = 0; q < kSurD; ++q) {
+          double t = 0.0;
+#pragma unroll
+          for (int b = 0; b < kSurD; ++b) t += s1[(q * kSurD + b) * N + k] * V[(N + j) * kSurD + b];
+          x[c][q] = Mn * t;
+        }
+      } else {
+#pragma unroll
+        for (int q = 0; q < kSurD; ++q) x[c][q] = 0.0;
+      }
+    }
+    double m[5] = {0, 0, 0, 0, 0};
+    if (a.project) {
+      double a0[CPT] = {}, a1 = 0.0, a2 = 0.0;
+#pragma unroll 2
       for (int ii = 0; ii < N; ++ii) {
+        const double cx = c0 + ii * hh;
+        double qs = 0.0;
+#pragma unroll
+        for (int c = 0; c < CPT; ++c) {
+          double t = 0.0;
+#pragma unroll
+          for (int q = 0; q < kSurD; ++q) t += x[c][q] * V[ii * kSurD + q];
+          a0[c] += t;
+          qs += t;
+        }
+        a1 += qs * cx;
+        a2 += qs * (cx * cx);
+      }
+#pragma unroll
+      for (int c = 0; c < CPT; ++c) {
+        const int jk = threadIdx.x + c * NT;
+        const double cy = c0 + (jk / N) * hh, cz = c0 + (jk % N) * hh;
+        m[0] += a0[c];
+        m[2] += a0[c] * cy;
+        m[3] += a0[c] * cz;
+        m[4] += a0[c] * (cy * cy + cz * cz);
+      }
+      m[1] = a1;
+      m[4] += a2;
+      block_sums<5, NT>(m, red);
+      double lam[5];
+#pragma unroll
+      for (int p = 0; p < 5; ++p) {
+        lam[p] = 0.0;
+#pragma unroll
+        for (int k = 0; k < 5; ++k) lam[p] += a.Ainv[p * 5 + k] * (m[k] * a.cw);
+      }
+#pragma unroll
+      for (int p = 0; p < 5; ++p) m[p] = a.cw * lam[p];
+    }
+    double* Q = a.Q + static_cast<size_t>(pt) * n;
+#pragma unroll
+    for (int c = 0; c < CPT; ++c) {
+      const int jk = threadIdx.x + c * NT;
+      if (jk >= NN) continue;
+      const double cy = c0 + (jk / N) * hh, cz = c0 + (jk % N) * hh;
+      const double l0 = m[0] + m[2] * cy + m[3] * cz + m[4] * (cy * cy + cz * cz);
+#pragma unroll 4
+      for (int ii = 0; ii < N; ++ii) {
+        const double cx = c0 + ii * hh;
         double t = 0.0;
 #pragma unroll
-        for (int aa = 0; aa < kSurD; ++aa) t += s2[aa * NN + jk] * V[ii * kSurD + aa];
-        Q[ii * NN + jk] = Mn * t;
+        for (int q = 0; q < kSurD; ++q) t += x[c][q] * V[ii * kSurD + q];
+        Q[ii * NN + jk] = t - (l0 + cx * (m[1] + m[4] * cx));
       }
     }
     __syncthreads();
@@ -1481,8 +1618,8 @@ static size_t enc_lds() {
 }
 template <int N>
 static size_t dec_lds() {
-  return (static_cast<size_t>(kSurD) * N * N + kSurD * kSurD * N + 3 * N * kSurD + kSurModes +
-          6 * kSurD * kSurD) * sizeof(double);
+  return (static_cast<size_t>(kSurD) * kSurD * N + 3 * N * kSurD + kSurModes + 6 * kSurD * kSurD + 20) *
+         sizeof(double);
 }
 
 template <int N>
@@ -1490,7 +1627,7 @@ static int launch_encode(const EncArgs& ea, hipStream_t st) {
   const size_t lds = enc_lds<N>();
   DGFS_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(k_sur_encode<N>),
                                    hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
-  hipLaunchKernelGGL(k_sur_encode<N>, dim3(std::min(ea.npts, 4 * cu_count())), dim3(256), lds, st, ea);
+  hipLaunchKernelGGL(k_sur_encode<N>, dim3(std::min(ea.npts, 4 * cu_count())), dim3(kEncThreads), lds, st, ea);
   DGFS_LAUNCH_CHECK("sur_encode");
   return DGFS_OK;
 }
@@ -1533,6 +1670,15 @@ static int do_targets(SurHandle* h, const TgtArgs& ta, hipStream_t st) {
     default: return fail(DGFS_ERR_UNSUPPORTED, "Nv=%d not built for the surrogate", h->N);
   }
 }
+// unprojected decode of rows of y into the points idx (null: row i, point i)
+static DecArgs dec_args(const SurHandle* h, const float* y, const double* mom, const int* idx, double* Q, int nidx) {
+  DecArgs da{};
+  da.y = y; da.mom = mom; da.idx = idx; da.Q = Q;
+  da.L = h->L; da.gamma = h->gamma; da.prefac = h->prefac;
+  da.nidx = nidx;
+  return da;
+}
+
 static int do_decode(SurHandle* h, const DecArgs& da, hipStream_t st) {
   switch (h->N) {
     case 8: return launch_decode<8>(da, st);
@@ -1687,10 +1833,13 @@ extern "C" int dgfs_sur_decode(void* p, const float* y, const double* mom, const
   if (nidx == 0) return DGFS_OK;
   if (project && idx) return fail(DGFS_ERR_INVALID_VALUE, "projection of an index subset: project the rows afterwards");
   auto st = static_cast<hipStream_t>(stream);
-  DecArgs da{y, mom, idx, Q, h->L, h->gamma, h->prefac, nidx};
-  int rc = do_decode(h, da, st);
-  if (!rc && project) rc = launch_invariant_projection(Q, h->Ainv, h->L, h->cw, h->N, nidx, st);
-  return rc;
+  DecArgs da = dec_args(h, y, mom, idx, Q, nidx);
+  if (project) {
+    da.project = 1;
+    da.cw = h->cw;
+    std::memcpy(da.Ainv, h->Ainv, sizeof(da.Ainv));
+  }
+  return do_decode(h, da, st);
 }
 
 namespace dgfs {
@@ -1769,7 +1918,7 @@ static int network_rows(SurHandle* h, const float* params, double* Q, const int*
     DGFS_LAUNCH_CHECK("lt_gather");
     int rc = sur_forward(h, params, h->xg, h->ltg, nb, h->yout, bf16, st);
     if (rc) return rc;
-    DecArgs da{h->yout, h->mom, idx + b0, Q, h->L, h->gamma, h->prefac, nb};
+    const DecArgs da = dec_args(h, h->yout, h->mom, idx + b0, Q, nb);
     rc = do_decode(h, da, st);
     if (rc) return rc;
   }

@@ -67,3 +67,54 @@ def test_layers_small_batches(P, device):
     eg = np.linalg.norm(sur.grad.cpu().numpy() - g) / np.linalg.norm(g)
     say("  forward", e, "gradient", eg)
     assert e < 1e-5 and eg < 1e-5
+
+
+@pytest.mark.parametrize("N", [12, 16, 24, 32])
+def test_encode_decode_grids(N, device):
+    """Encoder and projecting decoder on every built grid, one point and more
+    points than fit one sweep of workgroups' columns, against the FP64
+    checker: FP32 rounding on the modes, 1e-10 on the FP64 outputs plus the
+    forward error of the per-axis factorisations, at most about eps times the
+    condition number of their Gram matrices, three axes, with a margin of 4.
+    (At N = 8 the eight functions fill the eight points: the Gram matrix is
+    numerically singular and its modes mean nothing.)"""
+    import torch
+    from dgfs_hip.surrogate import SpectralSurrogate
+    L = 6.0 if N >= 16 else 5.0
+    rng = np.random.default_rng(N)
+    P = 3
+    c = S.grid(N, L)
+    I, J, K = np.meshgrid(c, c, c, indexing="ij")
+    f = []
+    for _ in range(P):
+        u, T = rng.uniform(-0.4, 0.4, 3), rng.uniform(0.9, 1.6)
+        g = np.exp(-((I - u[0]) ** 2 + (J - u[1]) ** 2 + (K - u[2]) ** 2) / T) / (np.pi * T) ** 1.5
+        f.append((g * (1 + 0.05 * (I - u[0]) * (J - u[1]))).ravel())
+    f = np.array(f)
+    sur = SpectralSurrogate(N, L, (2 * L / N) ** 3, 0.38, 1.0, max_batch=8, device=device, seed=1)
+    ft = torch.as_tensor(f, device=device)
+    mom = torch.empty((P, 8), dtype=torch.float64, device=device)
+    x = torch.empty((P, 512), dtype=torch.float32, device=device)
+    lt = torch.empty((P,), dtype=torch.float32, device=device)
+    say("encode / decode", N)
+    sur.encode(ft, P, mom, x, lt)
+    y = rng.normal(size=(P, 512)).astype(np.float32)
+    yt = torch.as_tensor(y, device=device)
+    Q = torch.full_like(ft, float("nan"))
+    Q0 = torch.full_like(ft, float("nan"))
+    sur.decode(yt, mom, P, Q, project=True)
+    sur.decode(yt, mom, P, Q0, project=False)
+    torch.cuda.synchronize()
+    mh = mom.cpu().numpy()
+    for i in range(P):
+        mref, a, _ = S.encode(f[i], N, L)
+        cond = max(np.linalg.cond(v.T @ v) for v in S._vander(N, L, mref[1:4], mref[4]))
+        tol = 1e-10 + 12 * 2.0 ** -52 * cond
+        say("  largest condition number", cond, "errors", np.abs(mh[i, :7] - mref).max())
+        assert np.abs(mh[i, :6] - mref[:6]).max() < 1e-10
+        assert np.abs(mh[i, 6] - mref[6]) < tol
+        assert np.abs(x.cpu().numpy()[i] - a).max() < (1e-6 + tol) * max(1.0, np.abs(a).max())
+        q0 = S.decode(y[i], mref, N, L, 0.38, 1.0)
+        sc = np.abs(q0).max()
+        assert np.abs(Q0.cpu().numpy()[i] - q0).max() < tol * sc
+        assert np.abs(Q.cpu().numpy()[i] - S.project(q0, N, L)).max() < tol * sc
