@@ -326,11 +326,18 @@ struct BcArgs {
   double U[3];
 };
 
-// ghost state (bcs/dgfs-*.mako) then the upwind flux; ul = |n| fn
-__global__ __launch_bounds__(256) void k_bccflux(BcArgs a) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+// ghost state (bcs/dgfs-*.mako) then the upwind flux; ul = |n| fn.  A
+// workgroup takes kBcPts boundary points (consecutive ones are neighbouring
+// elements of an AoSoA block) by kBcRows rows of vchunk velocities: a boundary
+// has few points and many velocities, and one thread per point with 64
+// velocities each left most of the chip idle (36 points at 24^3: 47 -> 15 us on
+// MI355X).
+constexpr int kBcPts = 32, kBcRows = 8;
+
+__global__ __launch_bounds__(kBcPts * kBcRows) void k_bccflux(BcArgs a) {
+  const int i = blockIdx.x * kBcPts + (threadIdx.x % kBcPts);
   if (i >= a.nfpts) return;
-  const int v0 = blockIdx.y * a.vchunk, v1 = min(v0 + a.vchunk, a.nvars);
+  const int v0 = (blockIdx.y * kBcRows + threadIdx.x / kBcPts) * a.vchunk, v1 = min(v0 + a.vchunk, a.nvars);
   const long ol = a.loff[i];
   double n[3] = {0, 0, 0};
   for (int d = 0; d < a.ndims; ++d) n[d] = a.nl[d * static_cast<long>(a.nfpts) + i];
@@ -384,8 +391,12 @@ __global__ __launch_bounds__(256) void k_bccflux(BcArgs a) {
 // bc1 += sum_{fac<0} fac f0 cw; reset when vidx == 0.  With st set (the
 // cylinder wall, dgfs-wall-diffuse-cyl-update.mako:12-44) U and T are
 // per point and f0 is the unnormalised Maxwellian.  One block per wall
-// point, a tree reduction over the velocity index.
-__global__ __launch_bounds__(256) void k_bccupdate_diffuse(int ndims, int nfpts, int nvars, int vidx,
+// point, kUpdUnroll velocities of every thread in flight (each is a cache line
+// of its own in the AoSoA register, so the loads are latency), a tree
+// reduction over the velocity index.  36 points at 24^3: 56 -> 27 us on MI355X
+// against 256 threads with one load at a time.
+constexpr int kUpdThreads = 1024, kUpdUnroll = 4;
+__global__ __launch_bounds__(kUpdThreads) void k_bccupdate_diffuse(int ndims, int nfpts, int nvars, int vidx,
                                                            const double* __restrict__ L,
                                                            const long* __restrict__ loff,
                                                            const double* __restrict__ nl,
@@ -394,7 +405,7 @@ __global__ __launch_bounds__(256) void k_bccupdate_diffuse(int ndims, int nfpts,
                                                            double Uy, double Uz, double cw,
                                                            const double* __restrict__ cv, int vsize,
                                                            const double* __restrict__ st) {
-  __shared__ double r0[256], r1[256];
+  __shared__ double r0[kUpdThreads], r1[kUpdThreads];
   const int i = blockIdx.x, tid = threadIdx.x;
   const long ol = loff[i];
   double n[3] = {0, 0, 0};
@@ -405,17 +416,29 @@ __global__ __launch_bounds__(256) void k_bccupdate_diffuse(int ndims, int nfpts,
     Tw = st[3L * nfpts + i];
   }
   double s0 = 0.0, s1 = 0.0;
-  for (int v = tid; v < nvars; v += 256) {
-    const int vv = vidx + v;
-    double fac = 0.0;
-    for (int d = 0; d < ndims; ++d) fac += (cv[d * static_cast<long>(vsize) + vv] - U[d]) * n[d];
-    if (fac >= 0) s0 += fac * L[ol + 32L * v] * cw;
-    else s1 += fac * (st ? cyl_wall_f(cv, vsize, vv, U, Tw) : f0[vv]) * cw;
+  for (int v0 = tid; v0 < nvars; v0 += kUpdThreads * kUpdUnroll) {
+    double fac[kUpdUnroll], x[kUpdUnroll];
+#pragma unroll
+    for (int k = 0; k < kUpdUnroll; ++k) {
+      const int v = v0 + k * kUpdThreads, vv = vidx + min(v, nvars - 1);
+      fac[k] = 0.0;
+      for (int d = 0; d < ndims; ++d) fac[k] += (cv[d * static_cast<long>(vsize) + vv] - U[d]) * n[d];
+      x[k] = 0.0;
+      if (v < nvars) {
+        if (fac[k] >= 0) x[k] = L[ol + 32L * v];
+        else x[k] = st ? cyl_wall_f(cv, vsize, vv, U, Tw) : f0[vv];
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < kUpdUnroll; ++k) {
+      if (fac[k] >= 0) s0 += fac[k] * x[k] * cw;
+      else s1 += fac[k] * x[k] * cw;
+    }
   }
   r0[tid] = s0;
   r1[tid] = s1;
   __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
+  for (int s = kUpdThreads / 2; s > 0; s >>= 1) {
     if (tid < s) {
       r0[tid] += r0[tid + s];
       r1[tid] += r1[tid + s];
@@ -730,11 +753,15 @@ extern "C" int dgfs_bccflux(int bctype, int ndims, int nfpts, int nvars, int vid
   if (nfpts == 0 || nvars == 0) return DGFS_OK;
   BcArgs a;
   a.bctype = bctype; a.ndims = ndims; a.nfpts = nfpts; a.nvars = nvars; a.vidx = vidx;
-  a.vchunk = vchunk_for(nvars); a.vsize = vsize;
+  a.vsize = vsize;
+  // 4 velocities per thread, more where the grid's second dimension (65535)
+  // or an already full chip asks for it
+  a.vchunk = 4;
+  while ((nvars + a.vchunk * kBcRows - 1) / (a.vchunk * kBcRows) > 16384) a.vchunk *= 2;
   a.L = L; a.loff = loff; a.nl = nl; a.magnl = magnl; a.f0 = f0; a.bcvals = bcvals; a.rmap = rmap; a.cv = cv;
   a.U[0] = Ux; a.U[1] = Uy; a.U[2] = Uz;
-  dim3 grid((nfpts + 255) / 256, (nvars + a.vchunk - 1) / a.vchunk);
-  hipLaunchKernelGGL(k_bccflux, grid, dim3(256), 0, static_cast<hipStream_t>(stream), a);
+  dim3 grid((nfpts + kBcPts - 1) / kBcPts, (nvars + a.vchunk * kBcRows - 1) / (a.vchunk * kBcRows));
+  hipLaunchKernelGGL(k_bccflux, grid, dim3(kBcPts * kBcRows), 0, static_cast<hipStream_t>(stream), a);
   DGFS_LAUNCH_CHECK("dgfs_bccflux");
   return DGFS_OK;
 }
@@ -750,7 +777,7 @@ extern "C" int dgfs_bccupdate(int bctype, int ndims, int nfpts, int nvars, int v
   if (bctype == BC_DIFFUSE || bctype == BC_DIFFUSE_CYL) {
     if (!f0) return fail(DGFS_ERR_INVALID_VALUE, "dgfs_bccupdate: diffuse wall needs f0");
     const bool cyl = bctype == BC_DIFFUSE_CYL;
-    hipLaunchKernelGGL(k_bccupdate_diffuse, dim3(nfpts), dim3(256), 0, st, ndims, nfpts, nvars, vidx, L, loff,
+    hipLaunchKernelGGL(k_bccupdate_diffuse, dim3(nfpts), dim3(kUpdThreads), 0, st, ndims, nfpts, nvars, vidx, L, loff,
                        nl, cyl ? nullptr : f0, bcvals, Ux, Uy, Uz, cw, cv, vsize, cyl ? f0 : nullptr);
   } else if (bctype == BC_SPECULAR) {
     hipLaunchKernelGGL(k_bccupdate_specular, dim3((nfpts + 255) / 256, nvars), dim3(256), 0, st, nfpts, nvars,

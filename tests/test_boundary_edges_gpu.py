@@ -1,0 +1,50 @@
+"""The boundary kernels at the sizes where their thread shapes can go wrong:
+one point, a ragged last group of 32 points, velocity counts around the rows
+and the unrolled sweeps, a velocity batch in the middle of the grid.  Against
+the same sums in numpy (FP64, 1e-13 of the largest value)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("nf,nvars,vidx,vsize", [(1, 27, 0, 27), (33, 64, 0, 64), (36, 1000, 24, 1030),
+                                                 (70, 4100, 0, 4100), (5, 9000, 0, 9000)])
+def test_diffuse_wall_edges(nf, nvars, vidx, vsize, device):
+    import torch
+    from dgfs_hip import fr
+    rng = np.random.default_rng(nf + nvars)
+    nblk = -(-nf // 32)
+    ld = nblk * nvars * 32
+    L = rng.uniform(0.1, 1.0, size=ld)
+    off = np.array([(i // 32) * nvars * 32 + i % 32 for i in range(nf)], dtype=np.int64)
+    ang = rng.uniform(0, 2 * np.pi, nf)
+    nl, mag = np.stack([np.cos(ang), np.sin(ang)]), rng.uniform(0.5, 2.0, nf)
+    cv = rng.uniform(-5, 5, size=(3, vsize))
+    f0 = rng.uniform(0.1, 1.0, vsize)
+    bc0 = rng.uniform(0.1, 1.0, 2 * nf)
+    U, cw = (0.3, -0.1, 0.0), 0.7
+    t = lambda a, d=torch.float64: torch.as_tensor(np.ascontiguousarray(a), dtype=d, device=device)
+    Lt, ot, nt, mt, ct, ft, bt = t(L), t(off, torch.int64), t(nl), t(mag), t(cv), t(f0), t(bc0)
+    st = torch.cuda.current_stream().cuda_stream
+    print("wall", nf, nvars, vidx, flush=True)
+    fr.bccupdate(fr.BC_DIFFUSE, 2, nf, nvars, vidx, Lt, ot, nt, ft, bt, U, cw, ct, vsize, st)
+    c = cv[:, vidx:vidx + nvars]
+    ul = L[off[:, None] + 32 * np.arange(nvars)[None]]
+    fac = nl[0][:, None] * (c[0] - U[0]) + nl[1][:, None] * (c[1] - U[1])
+    f0b = f0[vidx:vidx + nvars]
+    b0 = np.where(fac >= 0, fac * ul * cw, 0).sum(1)
+    b1 = np.where(fac < 0, fac * f0b * cw, 0).sum(1)
+    if vidx:
+        b0, b1 = b0 + bc0[:nf], b1 + bc0[nf:]
+    got = bt.cpu().numpy()
+    assert np.abs(got - np.concatenate([b0, b1])).max() < 1e-13 * max(np.abs(b0).max(), np.abs(b1).max())
+    fr.bccflux(fr.BC_DIFFUSE, 2, nf, nvars, vidx, Lt, ot, nt, mt, ft, bt, None, U, ct, vsize, st)
+    torch.cuda.synchronize()
+    nc = nl[0][:, None] * c[0] + nl[1][:, None] * c[1]
+    ur = np.where(fac < 0, f0b * (-got[:nf] / got[nf:])[:, None], ul)
+    fn = (0.5 * nc * (ul + ur) + 0.5 * np.abs(nc) * (ul - ur)) * mag[:, None]
+    out = Lt.cpu().numpy()
+    ref = L.copy()
+    ref[off[:, None] + 32 * np.arange(nvars)[None]] = fn
+    assert np.abs(out - ref).max() < 1e-13 * np.abs(ref).max()
