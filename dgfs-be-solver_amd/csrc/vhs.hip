@@ -1852,7 +1852,7 @@ struct VhsHandle {
   int planar = 0;        // the design is planar and the kernels exist for this grid
   int nshift = 0;
   std::vector<PlanarGroup> pgroups;
-  void* smat = nullptr;  // [Nrho][nshift][64][N/2] operand values of R(shift)
+  void* smat = nullptr;  // [Nrho][nshift][64][NR] operand values of R(shift)
   double* pbeta = nullptr;  // [Nrho][nshift]
   void* plop = nullptr;  // operand form of the points
   size_t cap_plop = 0;
@@ -2370,7 +2370,7 @@ static int run_planar(VhsHandle* h, const double* fc, double* Qc, int npts, hipS
     h->last_groups = groups;
     {
       PlanarPrepArgs<T> pa{fc, static_cast<T*>(h->plop), npts};
-      const size_t lds = (static_cast<size_t>(2 * PS::RN) + 3) * N * (N + 1) * sizeof(T);
+      const size_t lds = (static_cast<size_t>(4 * PS::RQ) + 3) * N * (N + 1) * sizeof(T);
       const void* kfn = reinterpret_cast<const void*>(k_planar_prep<T, N>);
       DGFS_HIP_TRY(hipFuncSetAttribute(kfn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
       const int grid = rr_edge_grid(kfn, 256, lds, npts);
@@ -2476,7 +2476,7 @@ static int ensure_ws(VhsHandle* h, int pts) {
 static int chunk_points(const VhsHandle* h, int total) {
   double per = static_cast<double>(h->n) * (2.0 * h->tsize * (1 + h->Nrho) + 16.0);
   if (use_planar(h))  // spectrum, one G^, operands, T, f and Q
-    per = static_cast<double>(h->n) * (h->tsize * (2.0 + 2.0 + 3.5 + h->Nrho) + 16.0);
+    per = static_cast<double>(h->n) * (h->tsize * (2.0 + 2.0 + 6.0 + h->Nrho) + 16.0);
   else if (use_rr(h)) per += 3.0 * h->N * h->N * h->Nrho * h->M * 2.0 * h->tsize + 2.0 * h->tsize * h->n;
   if (rr_kind(h) == 6 && !use_planar(h)) per += 2.0 * h->tsize * h->n * h->Nrho;  // the slab kernel's T
   const double budget = 48.0 * 1024.0 * 1024.0 * 1024.0;
@@ -2573,11 +2573,14 @@ static bool planar_groups(const double* sz, int M, std::vector<PlanarGroup>* gro
 }
 
 // operand values of R(shift) (vhs_planar.hpp) for every radial node and shift:
-// [Nrho][nshift][64 lanes][even/odd][tile][r], and beta = -sin(theta N/2) / N
-template <typename T>
-static void planar_tables(int N, const std::vector<double>& alpha, const std::vector<double>& shifts,
-                          std::vector<double>* smat, std::vector<double>* beta) {
-  const int RN = N / 8, NR = 4 * RN, D = static_cast<int>(shifts.size()), P = static_cast<int>(alpha.size());
+// [Nrho][nshift][64 lanes][part][K step], and beta = -sin(theta N/2) / N
+template <typename T, int N>
+static void planar_tables_n(const std::vector<double>& alpha, const std::vector<double>& shifts,
+                            std::vector<double>* smat, std::vector<double>* beta) {
+  using PS = PlanarShape<T, N>;
+  using MT = MmaTile<T>;
+  constexpr int RQ = PS::RQ, NR = PS::NR, M = PS::M;
+  const int D = static_cast<int>(shifts.size()), P = static_cast<int>(alpha.size());
   const double pi = 3.14159265358979323846;
   std::vector<double> cs(N), R(N);
   for (int m = 0; m < N; ++m) cs[m] = std::cos(2.0 * pi * m / N);
@@ -2601,21 +2604,36 @@ static void planar_tables(int N, const std::vector<double>& alpha, const std::ve
         R[j] = s / N;
       }
       (*beta)[static_cast<size_t>(p) * D + d] = -sn[N / 2] / N;
+      // part matrices: R^c = R(i - j) + R(i - j - M), R^d their difference; rows
+      // at j + M take R^d negated
+      auto rc = [&](int i, int j) { return R[(i - j + 2 * N) % N] + R[(i - j - M + 2 * N) % N]; };
+      auto rd = [&](int i, int j) { return R[(i - j + 2 * N) % N] - R[(i - j - M + 2 * N) % N]; };
       double* o = smat->data() + (static_cast<size_t>(p) * D + d) * 64 * NR;
       for (int lane = 0; lane < 64; ++lane) {
         const int g = lane / 16, i = lane % 16;
-        if (!MmaTile<T>::valid(i, RN)) continue;
-        for (int t = 0; t < 2; ++t) {
-          const int row = t ? N - 1 - MmaTile<T>::col(i) : MmaTile<T>::col(i);
-          for (int r = 0; r < RN; ++r) {
-            const int k = 4 * r + g;
-            const double a = R[(row - k + N) % N], b = R[(row - (N - 1 - k) + N) % N];
-            o[lane * NR + t * RN + r] = a + b;
-            o[lane * NR + (2 + t) * RN + r] = a - b;
-          }
+        if (!PS::filled(MT::reg(i), MT::grp(i))) continue;
+        const int sl = PS::slot(MT::reg(i), MT::grp(i)), row = sl % M;
+        const double sd = sl >= M ? -1.0 : 1.0;
+        for (int q = 0; q < RQ; ++q) {
+          const int k = 4 * q + g;
+          if (k >= PS::Q) continue;
+          o[lane * NR + 0 * RQ + q] = rc(row, k) + rc(row, M - 1 - k);
+          o[lane * NR + 1 * RQ + q] = rc(row, k) - rc(row, M - 1 - k);
+          o[lane * NR + 2 * RQ + q] = sd * (rd(row, k) + rd(row, M - 1 - k));
+          o[lane * NR + 3 * RQ + q] = sd * (rd(row, k) - rd(row, M - 1 - k));
         }
       }
     }
+}
+template <typename T>
+static void planar_tables(int N, const std::vector<double>& alpha, const std::vector<double>& shifts,
+                          std::vector<double>* smat, std::vector<double>* beta) {
+  if (N == 16)
+    planar_tables_n<T, 16>(alpha, shifts, smat, beta);
+  else if (N == 24)
+    planar_tables_n<T, 24>(alpha, shifts, smat, beta);
+  else
+    planar_tables_n<T, 32>(alpha, shifts, smat, beta);
 }
 
 // two handles (velocity grids NA > NB, same precision) in one persistent gain

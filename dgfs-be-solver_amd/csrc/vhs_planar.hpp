@@ -13,10 +13,18 @@
 // One plane of one such group costs three "pair moves": f -> X+- = R(+-a) f
 // along u, then X+ and X- by +-b along v each, for
 //   S += Z(+,+) Z(-,-) + Z(+,-) Z(-,+).
-// R(-s) = J R(s) J with J the index reversal, so with f = e + o (even and
-// odd under J) R(+-s) f needs only the products G = R e and H = R o of half
-// length: R(s) f = G + H, R(-s) f = J (G - H).  Rows are kept in two tiles,
-// idx and N-1-idx, so that J is a swap of the tiles.
+// Two splits cut a pair move from 4 N^2 to N^2 multiply-adds per line:
+//   c_j = (f_j + f_{j+M}) / 2, d_j = (f_j - f_{j+M}) / 2, M = N/2: a circulant
+//   of N is a circulant R^c of M on c and a skew circulant R^d on d, with
+//   (R f)_j = c'_j + d'_j and (R f)_{j+M} = c'_j - d'_j;
+//   R^{c,d}(-s) = K R^{c,d}(s) K with K the index reversal of M, so with even
+//   and odd parts under K, R(s) = G + H and R(-s) = K (G - H), G and H the
+//   products with the even and the odd half.
+// The four parts ce, co, de, do of N/4 values each are the K index of the
+// products, the M outputs the rows of one 16 x 16 tile; K is a swap of result
+// registers (rows) or of neighbouring lanes (columns), because every output
+// and its mirror image share a lane group.  At N = 16 the tile has room for
+// both j and j + M (the d rows negated).
 //
 // A plane is one wave's work and never leaves its registers: the first move
 // takes the plane as the A operand of v_mfma 16x16x4 and R as B, which leaves
@@ -59,16 +67,23 @@ namespace dgfs {
 
 template <typename T>
 struct MmaTile;
-// result row of register r in lane group g = lane / 16 is index 4 r + g; col()
-// and valid() give the index of lane i = lane % 16 (operand row or column)
+// Row or column i of a tile belongs to register reg(i) of lane group grp(i) in
+// the result layout (FP32: row 4 g + r, FP64: row 4 r + g).  mirror<RQ>(x):
+// the value of the lane whose register index differs by ^ RQ.
 template <>
 struct MmaTile<float> {
   typedef float V4 __attribute__((ext_vector_type(4)));
   static __device__ __forceinline__ V4 mma(float a, float b, V4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
   }
-  static __host__ __device__ __forceinline__ int col(int i) { return 4 * (i & 3) + (i >> 2); }
-  static __host__ __device__ __forceinline__ bool valid(int i, int RN) { return (i & 3) < RN; }
+  static __host__ __device__ __forceinline__ constexpr int reg(int i) { return i & 3; }
+  static __host__ __device__ __forceinline__ constexpr int grp(int i) { return i >> 2; }
+  static __host__ __device__ __forceinline__ constexpr int at(int r, int g) { return 4 * g + r; }
+  template <int RQ>
+  static __device__ __forceinline__ float mirror(float x) {  // i ^ RQ within each quad
+    constexpr int ctrl = RQ == 2 ? 0x4E : 0xB1;
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), ctrl, 0xF, 0xF, true));
+  }
 };
 template <>
 struct MmaTile<double> {
@@ -76,8 +91,23 @@ struct MmaTile<double> {
   static __device__ __forceinline__ V4 mma(double a, double b, V4 c) {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
   }
-  static __host__ __device__ __forceinline__ int col(int i) { return i; }
-  static __host__ __device__ __forceinline__ bool valid(int i, int RN) { return i < 4 * RN; }
+  static __host__ __device__ __forceinline__ constexpr int reg(int i) { return i >> 2; }
+  static __host__ __device__ __forceinline__ constexpr int grp(int i) { return i & 3; }
+  static __host__ __device__ __forceinline__ constexpr int at(int r, int g) { return 4 * r + g; }
+  template <int RQ>
+  static __device__ __forceinline__ double mirror(double x) {  // i ^ (4 RQ) within each 16
+    int lo = __double2loint(x), hi = __double2hiint(x);
+    if constexpr (RQ == 2) {  // row rotation by 8
+      lo = __builtin_amdgcn_update_dpp(0, lo, 0x128, 0xF, 0xF, true);
+      hi = __builtin_amdgcn_update_dpp(0, hi, 0x128, 0xF, 0xF, true);
+    } else {  // half-row mirror (7 - i), then each quad reversed
+      lo = __builtin_amdgcn_update_dpp(0, lo, 0x141, 0xF, 0xF, true);
+      hi = __builtin_amdgcn_update_dpp(0, hi, 0x141, 0xF, 0xF, true);
+      lo = __builtin_amdgcn_update_dpp(0, lo, 0x1B, 0xF, 0xF, true);
+      hi = __builtin_amdgcn_update_dpp(0, hi, 0x1B, 0xF, 0xF, true);
+    }
+    return __hiloint2double(hi, lo);
+  }
 };
 
 constexpr int kPlanarMaxGroups = 32;
@@ -89,8 +119,13 @@ struct PlanarGroup {
 
 template <typename T, int N>
 struct PlanarShape {
-  static constexpr int HN = N / 2, RN = N / 8, NN = N * N, n = NN * N;
-  static constexpr int NR = 4 * RN;  // operand values per lane of one shift's matrices
+  static constexpr int M = N / 2, Q = N / 4, NN = N * N, n = NN * N;
+  static constexpr int RQ = (Q + 3) / 4;         // K steps (registers) of one part
+  static constexpr int NT = (N == 16) ? 1 : 2;   // 16-wide tiles of an axis: j and j + M, or both in one
+  static constexpr int NR = 4 * RQ;              // operand values per lane of one shift's matrices
+  static constexpr int ND = NR * NT;             // operand values per lane of a plane
+  static constexpr int plane = 64 * ND;
+  static constexpr int LN = 16 * NT;             // values of a line, in tile order
   // x-halves per work item: the FP64 32^3 field (256 KB) does not fit in LDS
   // in one piece.  The halves repeat the first move of the pairs (x, .): 22
   // pair moves per p for 18.
@@ -104,31 +139,47 @@ struct PlanarShape {
   static constexpr int PY = N + 1;
   static constexpr int PX = N * PY + ((N == 16) ? 20 : 4);
   static constexpr int s_elems = NX * PX;
-  static constexpr int ln_elems = (XH == 2) ? 3 * NN : 4 * NN;
+  static constexpr int ln_elems = (XH == 2) ? 3 * N * LN : 4 * N * LN;
   static constexpr size_t lds_bytes = (static_cast<size_t>(s_elems) + ln_elems) * sizeof(T);
-  static constexpr size_t per_point = 3 * static_cast<size_t>(n) + 6 * NN + 3 * N;  // operand values of one point
+  // operand values of one point: the planes, the six Nyquist sums, three lines
+  static constexpr size_t per_point = static_cast<size_t>(3 * N + 6) * plane + 4 * N;
   static constexpr int nslots = N / 2;  // real-plane pairs of T
   // planes of slot s
   static __host__ __device__ __forceinline__ constexpr int x1(int s) {
-    if (XH == 1) return s;
-    return s < N / 4 ? s : N - 1 - (s - N / 4);
+    return (XH == 1 || s < N / 4) ? s : s + N / 4;
   }
   static __host__ __device__ __forceinline__ constexpr int x2(int s) {
-    if (XH == 1) return s + N / 2;
-    return s < N / 4 ? s + N / 4 : N - 1 - s;
+    return x1(s) + ((XH == 1) ? N / 2 : N / 4);
   }
-  static_assert(N % 8 == 0 && N <= 32, "tiles of N/2 <= 16 rows");
+  // index of output register r in lane group g; the mirror image (M - 1 - j,
+  // in the same half of N) is register r ^ RQ of the same group
+  static __host__ __device__ __forceinline__ constexpr int slot(int r, int g) {
+    if (RQ == 2) return r < 2 ? 4 * r + g : M - 1 - 4 * (r - 2) - g;
+    return ((r & 1) ? M - 1 - g : g) + ((r & 2) ? M : 0);
+  }
+  // whether the register holds anything (Q = 6 at N = 24 leaves gaps)
+  static __host__ __device__ __forceinline__ constexpr bool filled(int r, int g) {
+    return RQ == 1 || 4 * (r & 1) + g < Q;
+  }
+  // tile and register of part `sub` (ce, co, de, do), index 4 q + g, on the
+  // lane axis of a plane
+  static __host__ __device__ __forceinline__ constexpr int part_tile(int sub) { return NT == 2 ? sub >> 1 : 0; }
+  static __host__ __device__ __forceinline__ constexpr int part_reg(int sub, int q) {
+    return NT == 2 ? 2 * (sub & 1) + q : sub;
+  }
+  static_assert(N == 16 || N == 24 || N == 32, "tiles of N/2 <= 16 rows");
 };
 
 // ---------------------------------------------------------------------------
 // Operand form of the points: per axis pair and plane of the third axis the
-// even / odd parts of f along both axes, stored so that a wave of the gain
-// reads its 64 lanes' operand registers as one contiguous block:
-//   [pair][s][v index][lane group][r][u even/odd][v even/odd], u index 4 r + g,
-// followed by the six Nyquist sums (same form, the plane index as lanes) and
-// the three lines f^_uv(s).  A workgroup takes a point; N/4 x-planes at a time
-// (both mirror images of every fourth x) pass through LDS, read once from f.
-// Bound by its stores (3 n values per point).
+// parts (ce, co, de, do) x (ce, co, de, do) of f along both axes, stored as the
+// gain's lanes hold them:
+//   [pair][s][lane][K step q][v tile][u part], u index 4 q + lane / 16, v by lane % 16,
+// followed by the six Nyquist sums (same form, the plane index on the lanes) and
+// the three lines f^_uv(s).  A workgroup takes a point; the x-planes with one
+// residue of their part index modulo 4 (four mirror and half-shift images of
+// each) pass through LDS at a time, read once from f.  Bound by its stores (3 n
+// values per point).
 // ---------------------------------------------------------------------------
 template <typename T>
 struct PlanarPrepArgs {
@@ -140,45 +191,69 @@ struct PlanarPrepArgs {
 template <typename T, int N>
 __global__ __launch_bounds__(256) void k_planar_prep(PlanarPrepArgs<T> a) {
   using PS = PlanarShape<T, N>;
-  constexpr int HN = PS::HN, RN = PS::RN, NN = PS::NN, n = PS::n, NR = PS::NR, PP = N * (N + 1), Q = 2 * RN;
+  using MT = MmaTile<T>;
+  constexpr int M = PS::M, Q = PS::Q, RQ = PS::RQ, NT = PS::NT, NN = PS::NN, n = PS::n, ND = PS::ND, PLN = PS::plane;
+  constexpr int PP = N * (N + 1), NQ = 4 * RQ, KP = 4 * RQ;  // staged planes, part indices (with gaps)
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
-  T* pl = reinterpret_cast<T*>(smem_raw);  // [Q][N][N + 1]
-  T* fx = pl + Q * PP;                     // Nyquist sums over x: [y][z]
+  T* pl = reinterpret_cast<T*>(smem_raw);  // [NQ][N][N + 1]
+  T* fx = pl + NQ * PP;                    // Nyquist sums over x: [y][z]
   T* fy = fx + PP;                         // over y: [x][z]
   T* fz = fy + PP;                         // over z: [x][y]
   const int tid = threadIdx.x;
-  auto combine = [](T* o, T a0, T b0, T c0, T d0) {
-    const double s = static_cast<double>(a0) + b0, d = static_cast<double>(a0) - b0;
-    const double t = static_cast<double>(c0) + d0, e = static_cast<double>(c0) - d0;
-    o[0] = static_cast<T>(0.25 * (s + t));
-    o[1] = static_cast<T>(0.25 * (s - t));
-    o[2] = static_cast<T>(0.25 * (d + e));
-    o[3] = static_cast<T>(0.25 * (d - e));
+  // image m of part index k: k, M - 1 - k, k + M, N - 1 - k
+  auto image = [](int k, int m) { return ((m & 1) ? M - 1 - k : k) + ((m & 2) ? M : 0); };
+  auto parts = [](double p0, double p1, double p2, double p3, double* o) {
+    const double s = p0 + p2, t = p1 + p3, d = p0 - p2, e = p1 - p3;
+    o[0] = s + t;
+    o[1] = s - t;
+    o[2] = d + e;
+    o[3] = d - e;
+  };
+  // the 4 x 4 parts of f(image(ku, .), image(kv, .)) into a plane; get(mu, mv)
+  // gives the value, `on` whether the indices exist
+  auto put = [&](T* P, int ku, int kv, bool on, auto&& get) {
+    double h[4][4];  // [v image][u part]
+#pragma unroll
+    for (int mv = 0; mv < 4; ++mv) {
+      if (on)
+        parts(get(0, mv), get(1, mv), get(2, mv), get(3, mv), h[mv]);
+      else
+        h[mv][0] = h[mv][1] = h[mv][2] = h[mv][3] = 0.0;
+    }
+    double o[4][4];  // [u part][v part]
+#pragma unroll
+    for (int su = 0; su < 4; ++su) parts(h[0][su], h[1][su], h[2][su], h[3][su], o[su]);
+#pragma unroll
+    for (int sv = 0; sv < 4; ++sv) {
+      const int i = MT::at(PS::part_reg(sv, kv >> 2), kv & 3);
+      T* d = P + (16 * (ku & 3) + i) * ND + ((ku >> 2) * NT + PS::part_tile(sv)) * 4;
+#pragma unroll
+      for (int su = 0; su < 4; ++su) d[su] = static_cast<T>(0.0625 * o[su][sv]);
+    }
   };
   for (int pt = xcd_slot(); pt < a.npts; pt += gridDim.x) {
     const double* f = a.f + static_cast<size_t>(pt) * n;
     T* op = a.op + static_cast<size_t>(pt) * PS::per_point;
     for (int e = tid; e < PP; e += 256) fx[e] = T(0);
     for (int g = 0; g < 4; ++g) {
+      const int nq = (4 * (RQ - 1) + g < Q) ? NQ : NQ - 4;  // planes whose part index exists
       __syncthreads();
-      for (int e = tid; e < Q * NN; e += 256) {
+      for (int e = tid; e < nq * NN; e += 256) {
         const int q = e / NN, rem = e - q * NN, y = rem / N, z = rem - y * N;
-        const int k = 4 * (q >> 1) + g, x = (q & 1) ? N - 1 - k : k;
-        pl[q * PP + y * (N + 1) + z] = static_cast<T>(f[x * NN + rem]);
+        pl[q * PP + y * (N + 1) + z] = static_cast<T>(f[image(4 * (q >> 2) + g, q & 3) * NN + rem]);
       }
       __syncthreads();
       for (int e = tid; e < NN; e += 256) {
         const int y = e / N, z = e - y * N;
         double s = 0.0;
-        for (int q = 0; q < Q; ++q) {
+        for (int q = 0; q < nq; ++q) {
           const double v = pl[q * PP + y * (N + 1) + z];
-          s += ((g + q) & 1) ? -v : v;  // x = 4 r + g, or its mirror image
+          s += ((g + q) & 1) ? -v : v;  // images 1 and 3 have the other parity (M is even)
         }
         fx[y * (N + 1) + z] = static_cast<T>(static_cast<double>(fx[y * (N + 1) + z]) + s);
       }
-      for (int e = tid; e < Q * N; e += 256) {
-        const int q = e / N, i = e - q * N;
-        const int k = 4 * (q >> 1) + g, x = (q & 1) ? N - 1 - k : k;
+      for (int e = tid; e < nq * N; e += 256) {
+        const int q = e / N, i = e - q * N, x = image(4 * (q >> 2) + g, q & 3);
         double s = 0.0, t = 0.0;
         for (int j = 0; j < N; ++j) {
           const double v = pl[q * PP + j * (N + 1) + i], w = pl[q * PP + i * (N + 1) + j];
@@ -188,46 +263,33 @@ __global__ __launch_bounds__(256) void k_planar_prep(PlanarPrepArgs<T> a) {
         fy[x * (N + 1) + i] = static_cast<T>(s);
         fz[x * (N + 1) + i] = static_cast<T>(t);
       }
-      T o[NR];
-      for (int e = tid; e < HN * N; e += 256) {  // (x, y), plane z = s
-        const int j = e / N, s = e - j * N;
-#pragma unroll
-        for (int r = 0; r < RN; ++r) {
-          const T* p0 = pl + 2 * r * PP;
-          combine(o + 4 * r, p0[j * (N + 1) + s], p0[PP + j * (N + 1) + s], p0[(N - 1 - j) * (N + 1) + s],
-                  p0[PP + (N - 1 - j) * (N + 1) + s]);
-        }
-        T* d = op + static_cast<size_t>(s) * NN + (j * 4 + g) * NR;
-#pragma unroll
-        for (int k = 0; k < NR; ++k) d[k] = o[k];
+      for (int e = tid; e < RQ * KP * N; e += 256) {
+        const int s = e % N, kv = (e / N) % KP, r = e / (N * KP), ku = 4 * r + g;
+        const bool on = ku < Q && kv < Q;
+        const T* p0 = pl + 4 * r * PP;
+        // (x, y), plane z = s
+        put(op + static_cast<size_t>(s) * PLN, ku, kv, on,
+            [&](int mu, int mv) -> double { return p0[mu * PP + image(kv, mv) * (N + 1) + s]; });
       }
-      for (int e = tid; e < HN * N; e += 256) {  // (x, z), plane y = s
-        const int s = e / HN, j = e - s * HN;
-#pragma unroll
-        for (int r = 0; r < RN; ++r) {
-          const T* p0 = pl + 2 * r * PP + s * (N + 1);
-          combine(o + 4 * r, p0[j], p0[PP + j], p0[N - 1 - j], p0[PP + N - 1 - j]);
-        }
-        T* d = op + static_cast<size_t>(N + s) * NN + (j * 4 + g) * NR;
-#pragma unroll
-        for (int k = 0; k < NR; ++k) d[k] = o[k];
+      for (int e = tid; e < RQ * KP * N; e += 256) {
+        const int kv = e % KP, s = (e / KP) % N, r = e / (N * KP), ku = 4 * r + g;
+        const bool on = ku < Q && kv < Q;
+        const T* p0 = pl + 4 * r * PP + s * (N + 1);
+        // (x, z), plane y = s
+        put(op + static_cast<size_t>(N + s) * PLN, ku, kv, on,
+            [&](int mu, int mv) -> double { return p0[mu * PP + image(kv, mv)]; });
       }
-      for (int e = tid; e < Q * HN * 4; e += 256) {  // (y, z), plane x
-        const int j = e % HN, lg = (e / HN) % 4, q = e / (HN * 4);
-        const int kx = 4 * (q >> 1) + g, x = (q & 1) ? N - 1 - kx : kx;
-#pragma unroll
-        for (int r = 0; r < RN; ++r) {
-          const int y = 4 * r + lg;
-          const T *pa = pl + q * PP + y * (N + 1), *pb = pl + q * PP + (N - 1 - y) * (N + 1);
-          combine(o + 4 * r, pa[j], pb[j], pa[N - 1 - j], pb[N - 1 - j]);
-        }
-        T* d = op + static_cast<size_t>(2 * N + x) * NN + (j * 4 + lg) * NR;
-#pragma unroll
-        for (int k = 0; k < NR; ++k) d[k] = o[k];
+      for (int e = tid; e < nq * KP * KP; e += 256) {
+        const int kv = e % KP, ku = (e / KP) % KP, q = e / (KP * KP), x = image(4 * (q >> 2) + g, q & 3);
+        const bool on = ku < Q && kv < Q;
+        const T* p0 = pl + q * PP;
+        // (y, z), plane x
+        put(op + static_cast<size_t>(2 * N + x) * PLN, ku, kv, on,
+            [&](int mu, int mv) -> double { return p0[image(ku, mu) * (N + 1) + image(kv, mv)]; });
       }
     }
     __syncthreads();
-    T* ny = op + 3 * static_cast<size_t>(n);
+    T* ny = op + static_cast<size_t>(3 * N) * PLN;
     // contraction index k, plane index s of the six sums
     auto src = [&](int w, int k, int s) -> double {
       switch (w) {
@@ -239,14 +301,18 @@ __global__ __launch_bounds__(256) void k_planar_prep(PlanarPrepArgs<T> a) {
         default: return fz[s * (N + 1) + k];
       }
     };
-    for (int e = tid; e < 6 * NN; e += 256) {
-      const int w = e / NN, rem = e - w * NN;
-      const int st = rem & 1, eo = (rem >> 1) & 1, rg = rem >> 2, r = rg % RN, lg = (rg / RN) & 3, j = rg / (4 * RN);
-      const int k = 4 * r + lg, s = st ? N - 1 - j : j;
-      const double va = src(w, k, s), vb = src(w, N - 1 - k, s);
-      ny[e] = static_cast<T>(0.5 * (eo ? va - vb : va + vb));
+    for (int e = tid; e < 6 * 64 * RQ * NT; e += 256) {
+      const int t = e % NT, r = (e / NT) % RQ, lane = (e / (NT * RQ)) & 63, w = e / (64 * RQ * NT);
+      const int g = lane >> 4, i = lane & 15, k = 4 * r + g;
+      const int s = PS::slot(MT::reg(i), MT::grp(i)) + t * M;
+      double o[4] = {0.0, 0.0, 0.0, 0.0};
+      if (k < Q && PS::filled(MT::reg(i), MT::grp(i)))
+        parts(src(w, image(k, 0), s), src(w, image(k, 1), s), src(w, image(k, 2), s), src(w, image(k, 3), s), o);
+      T* d = ny + w * PLN + lane * ND + (r * NT + t) * 4;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) d[j] = static_cast<T>(0.25 * o[j]);
     }
-    T* line = ny + 6 * NN;
+    T* line = ny + 6 * PLN;
     for (int e = tid; e < 3 * N; e += 256) {
       const int w = e / N, s = e - w * N;
       double acc = 0.0;
@@ -263,38 +329,41 @@ __global__ __launch_bounds__(256) void k_planar_prep(PlanarPrepArgs<T> a) {
 template <typename T>
 struct PlanarGainArgs {
   const T* op;        // [npts][per_point]
-  const T* smat;      // [Nrho][nshift][64][NR] operand values of R(shift), per lane
+  const T* smat;      // [Nrho][nshift][64][NR] operand values of R(shift), per lane [part][K step]
   const double* beta; // [Nrho][nshift]
   cpx<T>* Tb;         // [npts][Nrho][N/2][N][N]
   int nitems, ngroups, ppg, Nrho, nshift, ngr;
   PlanarGroup gr[kPlanarMaxGroups];
 };
 
-// G = R e and H = R o of both row tiles; DATA_A: the data is the A operand
-// (its lanes become the result's rows), else the B operand.  The accumulators
-// start at c1, c2 (G) and zero (H).
-template <typename T, int RN, bool DATA_A>
-__device__ __forceinline__ void pair_move(const T (&e)[RN], const T (&o)[RN], const T (&S)[4 * RN],
-                                          typename MmaTile<T>::V4 c1, typename MmaTile<T>::V4 c2,
-                                          typename MmaTile<T>::V4& G1, typename MmaTile<T>::V4& G2,
-                                          typename MmaTile<T>::V4& H1, typename MmaTile<T>::V4& H2) {
-  using M = MmaTile<T>;
-  G1 = c1;
-  G2 = c2;
-  H1 = H2 = typename M::V4{T(0), T(0), T(0), T(0)};
+// products of the four parts with their matrices: Gc, Hc from ce, co and Gd, Hd
+// from de, do; x and S are indexed [part][K step].  DATA_A: the data is the A
+// operand (its lanes become the result's rows), else the B operand.  Gc
+// starts at `init`, the others at zero.
+template <typename T, int RQ, bool DATA_A>
+__device__ __forceinline__ void pair_move(const T (&x)[4 * RQ], const T (&S)[4 * RQ], typename MmaTile<T>::V4 init,
+                                          typename MmaTile<T>::V4 (&o)[4]) {
+  using MT = MmaTile<T>;
+  o[0] = init;
+  o[1] = o[2] = o[3] = typename MT::V4{T(0), T(0), T(0), T(0)};
 #pragma unroll
-  for (int r = 0; r < RN; ++r) {
-    if constexpr (DATA_A) {
-      G1 = M::mma(e[r], S[r], G1);
-      G2 = M::mma(e[r], S[RN + r], G2);
-      H1 = M::mma(o[r], S[2 * RN + r], H1);
-      H2 = M::mma(o[r], S[3 * RN + r], H2);
-    } else {
-      G1 = M::mma(S[r], e[r], G1);
-      G2 = M::mma(S[RN + r], e[r], G2);
-      H1 = M::mma(S[2 * RN + r], o[r], H1);
-      H2 = M::mma(S[3 * RN + r], o[r], H2);
-    }
+  for (int q = 0; q < RQ; ++q)
+#pragma unroll
+    for (int p = 0; p < 4; ++p)
+      o[p] = DATA_A ? MT::mma(x[p * RQ + q], S[p * RQ + q], o[p]) : MT::mma(S[p * RQ + q], x[p * RQ + q], o[p]);
+}
+
+// the two moves of one register from its four products: pa, pb at j and j + M
+// for the shift, ma, mb at the mirror images of j and j + M for the opposite
+// shift (NT = 1: j + M is in the products' rows, pb and mb are not formed)
+template <typename T, int NT>
+__device__ __forceinline__ void pair_sums(T gc, T hc, T gd, T hd, T& pa, T& pb, T& ma, T& mb) {
+  const T c = gc + hc, d = gd + hd, e = gc - hc, f = gd - hd;
+  pa = c + d;
+  ma = e + f;
+  if constexpr (NT == 2) {
+    pb = c - d;
+    mb = e - f;
   }
 }
 
@@ -303,125 +372,141 @@ __device__ __forceinline__ void pair_move(const T (&e)[RN], const T (&o)[RN], co
 // and the group's lines and the previous sum of S are read ahead of the
 // products that use them.
 template <typename T, int N, int PAIR>
-__device__ __forceinline__ void planar_planes(const T* op, const T (&Sa)[4 * (N / 8)], const T (&Sb)[4 * (N / 8)],
-                                              T bab, T* S, const T* ln, int half, bool first) {
+__device__ __forceinline__ void planar_planes(const T* op, const T (&Sa)[PlanarShape<T, N>::NR],
+                                              const T (&Sb)[PlanarShape<T, N>::NR], T bab, T* S, const T* ln, int half,
+                                              bool first) {
   using PS = PlanarShape<T, N>;
-  using M = MmaTile<T>;
-  using V4 = typename M::V4;
-  constexpr int RN = PS::RN, HN = PS::HN, NN = PS::NN, NR = PS::NR, XH = PS::XH, NX = PS::NX, NW = PS::NW;
-  constexpr bool HALF_U = XH == 2 && PAIR < 2;       // only the u tile of this x-half is wanted
-  constexpr int NT = HALF_U ? 1 : 2;                 // u tiles
+  using MT = MmaTile<T>;
+  using V4 = typename MT::V4;
+  constexpr int RQ = PS::RQ, M = PS::M, NT = PS::NT, ND = PS::ND, XH = PS::XH, NX = PS::NX, NW = PS::NW, LN = PS::LN;
+  constexpr bool HALF_U = XH == 2 && PAIR < 2;         // only the u tile of this x-half is wanted
+  constexpr int NU = HALF_U ? 1 : NT;                  // u tiles
   constexpr int NS = (XH == 2 && PAIR == 2) ? NX : N;  // planes of the item
-  constexpr int NU = HALF_U ? HN : N;                  // u values of the lines
+  constexpr int LU = HALF_U ? 16 : LN;                 // u values of the lines
   // strides of S along u, v and the plane index
   constexpr int TU = PAIR == 2 ? PS::PY : PS::PX, TV = PAIR == 0 ? PS::PY : 1;
   constexpr int TS = PAIR == 0 ? 1 : PAIR == 1 ? PS::PY : PS::PX;
-  const int lane = threadIdx.x & 63, lg = lane >> 4, i = lane & 15;
+  const int lane = threadIdx.x & 63, g = lane >> 4, i = lane & 15;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int ci = M::col(i);
-  const bool ok = (RN == 4) || M::valid(i, RN);
-  const int cc = ok ? ci : 0;
-  const T* eU = ln + lg * RN;
-  const T* dU = eU + NS * N;
-  const T* eV = ln + 2 * NS * N + (cc & 3) * RN + (cc >> 2);  // this lane's u
-  const T* dV = eV + NS * NU;
-  const T* line = op + 3 * PS::n + 6 * NN + PAIR * N;
-  const T sg = ((ci + lg) & 1) ? -bab : bab;
-  T* Su[2] = {S + cc * TU, S + (N - 1 - cc) * TU};
-  const T* P0 = op + static_cast<size_t>(PAIR * N) * NN + (cc * 4 + lg) * NR;
-  auto plane = [&](int sl) { return (PAIR == 2 && XH == 2 && half) ? N - 1 - sl : sl; };
-  T fr[NR], c0;
+  const int ri = MT::reg(i), gi = MT::grp(i);
+  const bool ok = PS::filled(ri, gi);
+  const int cu = ok ? PS::slot(ri, gi) : 0;  // this lane's u (in its tile)
+  const T* eU = ln + 4 * g;                  // [s][LN]: tile, lane group, register
+  const T* dU = eU + NS * LN;
+  const T* eV = ln + 2 * NS * LN + 4 * gi + ri;  // [s][LU]
+  const T* dV = eV + NS * LU;
+  const T* line = op + static_cast<size_t>(3 * N + 6) * PS::plane + PAIR * N;
+  // -w_u w_v beta_a beta_b of register 0: the sign changes with the mirror images
+  const T sg = (((gi + g) & 1) != ((ri & RQ) != 0)) ? bab : -bab;
+  T* S0 = S + cu * TU;
+  // register r of v: the rows 4 r + g (or g, M + g) from one base, their mirror
+  // images from another
+  auto vrow = [&](T* b, int r) -> T* {
+    const bool mir = (r & RQ) != 0;
+    const int off = (RQ == 2) ? (mir ? 4 * (3 - r) : 4 * r) : ((r & 2) ? M : 0);
+    return b + (mir ? (M - 1 - 4 * (RQ - 1) - g) * TV : g * TV) + off * TV;
+  };
+  const T* P0 = op + static_cast<size_t>(PAIR * N) * PS::plane + lane * ND;
+  auto plane = [&](int sl) { return (PAIR == 2 && XH == 2 && half) ? sl + M : sl; };
+  T fr[ND], l0;
   {
     const int s = plane(w);
-    const T* P = P0 + static_cast<size_t>(s) * NN;
+    const T* P = P0 + static_cast<size_t>(s) * PS::plane;
 #pragma unroll
-    for (int k = 0; k < NR; ++k) fr[k] = P[k];
-    c0 = line[s];
+    for (int k = 0; k < ND; ++k) fr[k] = P[k];
+    l0 = line[s];
   }
 #pragma unroll 1
   for (int sl = w; sl < NS; sl += NW) {
-    const T ck = sg * c0;
-    // move along u: X+-[tile][v even / odd][r], lanes u, registers v
-    T Xp[NT][2][RN], Xm[NT][2][RN];
+    const T ck = sg * l0;
+    // move along u: lanes u, registers v.  Xp[u tile] at u, Xm[u tile] at the
+    // mirror image of u; both [v part][K step] as the second move reads them
+    T Xp[NU][PS::NR], Xm[NU][PS::NR];
     const V4 z4{T(0), T(0), T(0), T(0)};
-    {
-      V4 G1[2], G2[2], H1[2], H2[2];
-#pragma unroll
-      for (int vt = 0; vt < 2; ++vt) {
-        T e[RN], o[RN];
-#pragma unroll
-        for (int r = 0; r < RN; ++r) {
-          e[r] = fr[4 * r + vt];
-          o[r] = fr[4 * r + 2 + vt];
-        }
-        pair_move<T, RN, true>(e, o, Sa, z4, z4, G1[vt], G2[vt], H1[vt], H2[vt]);
-      }
-#pragma unroll
-      for (int vt = 0; vt < 2; ++vt)
-#pragma unroll
-        for (int r = 0; r < RN; ++r) {
-          if constexpr (HALF_U) {
-            Xp[0][vt][r] = half ? G2[vt][r] + H2[vt][r] : G1[vt][r] + H1[vt][r];
-            Xm[0][vt][r] = half ? G1[vt][r] - H1[vt][r] : G2[vt][r] - H2[vt][r];
-          } else {
-            Xp[0][vt][r] = G1[vt][r] + H1[vt][r];
-            Xm[0][vt][r] = G2[vt][r] - H2[vt][r];
-            Xp[NT - 1][vt][r] = G2[vt][r] + H2[vt][r];
-            Xm[NT - 1][vt][r] = G1[vt][r] - H1[vt][r];
-          }
-        }
-    }
-    {  // the next plane (the last iteration reads its own again)
-      const int s = plane(sl + NW < NS ? sl + NW : sl);
-      const T* P = P0 + static_cast<size_t>(s) * NN;
-#pragma unroll
-      for (int k = 0; k < NR; ++k) fr[k] = P[k];
-      c0 = line[s];
-    }
-    T u1[RN], u2[RN], d1[RN], d2[RN];
-#pragma unroll
-    for (int r = 0; r < RN; ++r) {
-      u1[r] = eU[sl * N + r];
-      u2[r] = eU[sl * N + HN + r];
-      d1[r] = dU[sl * N + r];
-      d2[r] = dU[sl * N + HN + r];
-    }
+    V4 o1[NT][4];
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      // S at (u of the tile, v = 4 r + lg) and its mirror images in v, lowest address first
-      T* S1 = Su[t] + sl * TS + lg * TV;
-      T* S2 = Su[t] + sl * TS + (N - 1 - 4 * (RN - 1) - lg) * TV;
-      T p1[RN], p2[RN];
+      T x[PS::NR];
 #pragma unroll
-      for (int r = 0; r < RN; ++r) p1[r] = p2[r] = T(0);
+      for (int q = 0; q < RQ; ++q)
+#pragma unroll
+        for (int p = 0; p < 4; ++p) x[p * RQ + q] = fr[(q * NT + t) * 4 + p];
+      pair_move<T, RQ, true>(x, Sa, z4, o1[t]);
+    }
+#pragma unroll
+    for (int p = 0; p < 4; ++p)
+#pragma unroll
+      for (int q = 0; q < RQ; ++q) {
+        const int t = PS::part_tile(p), r = PS::part_reg(p, q);
+        T pa, pb = T(0), ma, mb = T(0);
+        pair_sums<T, NT>(o1[t][0][r], o1[t][1][r], o1[t][2][r], o1[t][3][r], pa, pb, ma, mb);
+        if constexpr (HALF_U) {
+          Xp[0][p * RQ + q] = half ? pb : pa;
+          Xm[0][p * RQ + q] = half ? mb : ma;
+        } else {
+          Xp[0][p * RQ + q] = pa;
+          Xm[0][p * RQ + q] = ma;
+          Xp[NU - 1][p * RQ + q] = NT == 2 ? pb : pa;
+          Xm[NU - 1][p * RQ + q] = NT == 2 ? mb : ma;
+        }
+      }
+    {  // the next plane (the last iteration reads its own again)
+      const int s = plane(sl + NW < NS ? sl + NW : sl);
+      const T* P = P0 + static_cast<size_t>(s) * PS::plane;
+#pragma unroll
+      for (int k = 0; k < ND; ++k) fr[k] = P[k];
+      l0 = line[s];
+    }
+    T ul[NT][4], dl[NT][4];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        ul[t][r] = eU[sl * LN + 16 * t + r];
+        dl[t][r] = dU[sl * LN + 16 * t + r];
+      }
+#pragma unroll
+    for (int t = 0; t < NU; ++t) {
+      T* B = S0 + sl * TS + t * M * TU;
+      T prev[NT][4];
+#pragma unroll
+      for (int v = 0; v < NT; ++v)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) prev[v][r] = T(0);
       if (!first) {
 #pragma unroll
-        for (int r = 0; r < RN; ++r) {
-          p1[r] = S1[4 * r * TV];
-          p2[r] = S2[4 * (RN - 1 - r) * TV];
-        }
-      }
-      const bool mirror = HALF_U ? half != 0 : t != 0;  // u = N - 1 - ci
-      const T ct = mirror ? -ck : ck;
-      const V4 cp{ct, ct, ct, ct}, cn{-ct, -ct, -ct, -ct};
-      V4 G1p, G2p, H1p, H2p, G1m, G2m, H1m, H2m;
-      pair_move<T, RN, false>(Xp[t][0], Xp[t][1], Sb, cn, cp, G1p, G2p, H1p, H2p);
-      pair_move<T, RN, false>(Xm[t][0], Xm[t][1], Sb, cp, cn, G1m, G2m, H1m, H2m);
-      const T ev = eV[sl * NU + (t ? HN : 0)], dv = dV[sl * NU + (t ? HN : 0)];
-      T q1[RN], q2[RN];
+        for (int v = 0; v < NT; ++v)
 #pragma unroll
-      for (int r = 0; r < RN; ++r) {
-        const T a1 = (G1p[r] + H1p[r]) * (G2m[r] - H2m[r]) + (G2p[r] - H2p[r]) * (G1m[r] + H1m[r]);
-        const T a2 = (G2p[r] + H2p[r]) * (G1m[r] - H1m[r]) + (G1p[r] - H1p[r]) * (G2m[r] + H2m[r]);
-        q1[r] = p1[r] + (a1 + (u1[r] + ev - d1[r] * dv));
-        q2[r] = p2[r] + (a2 + (u2[r] + ev - d2[r] * dv));
+          for (int r = 0; r < 4; ++r) prev[v][r] = vrow(B + v * M * TV, r)[0];
       }
+      const V4 init = (RQ == 2) ? V4{ck, ck, -ck, -ck} : V4{ck, -ck, ck, -ck};
+      V4 op2[4], om2[4];
+      pair_move<T, RQ, false>(Xp[t], Sb, init, op2);
+      pair_move<T, RQ, false>(Xm[t], Sb, init, om2);
+      // Z(+,+) = pp, Z(+,-) = pm (rows mirrored), Z(-,+) = mp (lanes mirrored),
+      // Z(-,-) = mm (both)
+      T pp[2][4], pm[2][4], mp[2][4], mm[2][4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        pair_sums<T, NT>(op2[0][r], op2[1][r], op2[2][r], op2[3][r], pp[0][r], pp[1][r], pm[0][r], pm[1][r]);
+        pair_sums<T, NT>(om2[0][r], om2[1][r], om2[2][r], om2[3][r], mp[0][r], mp[1][r], mm[0][r], mm[1][r]);
+      }
+      const T ev = eV[sl * LU + 16 * t], dv = dV[sl * LU + 16 * t];
+      T q[NT][4];
+#pragma unroll
+      for (int v = 0; v < NT; ++v)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          T x = MT::template mirror<RQ>(mm[v][r ^ RQ]) * pp[v][r];
+          x += MT::template mirror<RQ>(mp[v][r]) * pm[v][r ^ RQ];
+          q[v][r] = prev[v][r] + (x + (ul[v][r] + ev - dl[v][r] * dv));
+        }
       if (ok) {
 #pragma unroll
-        for (int r = 0; r < RN; ++r) {
-          S1[4 * r * TV] = q1[r];
-          S2[4 * (RN - 1 - r) * TV] = q2[r];
-        }
+        for (int v = 0; v < NT; ++v)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (PS::filled(r, g)) vrow(B + v * M * TV, r)[0] = q[v][r];
       }
     }
   }
@@ -431,25 +516,24 @@ template <typename T, int N>
 __global__ __launch_bounds__((PlanarShape<T, N>::NW * 64), (PlanarShape<T, N>::WPE)) void k_vhs_gain_planar(
     PlanarGainArgs<T> a) {
   using PS = PlanarShape<T, N>;
-  using M = MmaTile<T>;
-  using V4 = typename M::V4;
-  constexpr int RN = PS::RN, HN = PS::HN, NN = PS::NN, NR = PS::NR, XH = PS::XH, NX = PS::NX, NW = PS::NW;
+  using MT = MmaTile<T>;
+  using V4 = typename MT::V4;
+  constexpr int RQ = PS::RQ, M = PS::M, NT = PS::NT, NN = PS::NN, NR = PS::NR, ND = PS::ND, LN = PS::LN;
+  constexpr int XH = PS::XH, NX = PS::NX, NW = PS::NW;
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   T* S = reinterpret_cast<T*>(smem_raw);
   T* ln = S + PS::s_elems;
-  const int lane = threadIdx.x & 63, lg = lane >> 4, i = lane & 15;
+  const int lane = threadIdx.x & 63, g = lane >> 4, i = lane & 15;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int ci = M::col(i);
-  const bool ok = M::valid(i, RN);
-  const int cc = ok ? ci : 0;
+  const int ri = MT::reg(i), gi = MT::grp(i);
   for (int item = xcd_slot(); item < a.nitems; item += gridDim.x) {
     const int half = (XH == 2) ? item % 2 : 0, pg = item / XH;
     const int pt = pg / a.ngroups, grp = pg - pt * a.ngroups;
     const int p0 = grp * a.ppg, p1 = min(p0 + a.ppg, a.Nrho);
     const T* op = a.op + static_cast<size_t>(pt) * PS::per_point;
     for (int p = p0; p < p1; ++p) {
-      for (int gi = 0; gi < a.ngr; ++gi) {
-        const int pair = a.gr[gi].pair, ia = a.gr[gi].ia, ib = a.gr[gi].ib;
+      for (int gr = 0; gr < a.ngr; ++gr) {
+        const int pair = a.gr[gr].pair, ia = a.gr[gr].ia, ib = a.gr[gr].ib;
         T Sa[NR], Sb[NR];
         {
           const T* sa = a.smat + (static_cast<size_t>(p * a.nshift + ia) * 64 + lane) * NR;
@@ -461,53 +545,56 @@ __global__ __launch_bounds__((PlanarShape<T, N>::NW * 64), (PlanarShape<T, N>::W
         }
         const T ba = static_cast<T>(a.beta[p * a.nshift + ia]), bb = static_cast<T>(a.beta[p * a.nshift + ib]);
         const bool half_s = XH == 2 && pair == 2, half_u = XH == 2 && pair < 2;
-        const int NS = half_s ? NX : N, NU = half_u ? HN : N;
+        const int NS = half_s ? NX : N, LU = half_u ? 16 : LN;
         __syncthreads();  // the previous group's (or p's) readers of the lines and of S are done
         if (w < 4) {
-          // lines of the group: wave 2 * (V line) + (mirrored plane tile)
+          // lines of the group: wave 2 * (V line) + (tile of the plane index)
           const bool vline = w & 2;
           const int st = w & 1;
-          if (!half_s || st == half) {
-            const T* P = op + 3 * PS::n + (2 * pair + (vline ? 1 : 0)) * NN + (cc * 4 + lg) * NR;
-            T de[RN], dd[RN];
+          if (st < NT && (!half_s || st == half)) {
+            const T* P = op + static_cast<size_t>(3 * N + 2 * pair + (vline ? 1 : 0)) * PS::plane + lane * ND;
+            T x[NR];
 #pragma unroll
-            for (int r = 0; r < RN; ++r) {
-              de[r] = P[4 * r + st];
-              dd[r] = P[4 * r + 2 + st];
-            }
+            for (int q = 0; q < RQ; ++q)
+#pragma unroll
+              for (int p4 = 0; p4 < 4; ++p4) x[p4 * RQ + q] = P[(q * NT + st) * 4 + p4];
             const V4 z4{T(0), T(0), T(0), T(0)};
-            V4 G1, G2, H1, H2;
+            V4 o[4];
             if (vline)
-              pair_move<T, RN, true>(de, dd, Sa, z4, z4, G1, G2, H1, H2);
+              pair_move<T, RQ, true>(x, Sa, z4, o);
             else
-              pair_move<T, RN, true>(de, dd, Sb, z4, z4, G1, G2, H1, H2);
+              pair_move<T, RQ, true>(x, Sb, z4, o);
             const T e2 = vline ? T(2) * bb * bb : T(2) * ba * ba;
-            const T ds = ((ci & 1) ? T(-1) : T(1)) * (vline ? ba : bb);
-            const int NL = vline ? NU : N;
-            T* e = ln + (vline ? 2 * NS * N : 0);
-            T* d = e + NS * NL;
-            const int pos = (cc & 3) * RN + (cc >> 2);
+            // w of this lane's index (the same at j + M) times the other shift's beta
+            const T ds = (((gi & 1) != ((ri & RQ) != 0)) ? T(-1) : T(1)) * (vline ? ba : bb);
+            const int LL = vline ? LU : LN;
+            T* e = ln + (vline ? 2 * NS * LN : 0) + 4 * gi + ri;
+            T* d = e + NS * LL;
 #pragma unroll
-            for (int r = 0; r < RN; ++r) {
-              const int si = 4 * r + lg, s = (st && !half_s) ? N - 1 - si : si;
-              const T a1 = G1[r] + H1[r], b1 = G2[r] - H2[r];  // index ci: shift +, -
-              const T a2 = G2[r] + H2[r], b2 = G1[r] - H1[r];  // index N - 1 - ci
-              if (ok) {
+            for (int r = 0; r < 4; ++r) {
+              T pa, pb = T(0), ma, mb = T(0);
+              pair_sums<T, NT>(o[0][r], o[1][r], o[2][r], o[3][r], pa, pb, ma, mb);
+              ma = MT::template mirror<RQ>(ma);
+              mb = MT::template mirror<RQ>(mb);
+              const int s = PS::slot(r, g) + ((half_s || NT == 1) ? 0 : st * M);
+              if (PS::filled(r, g) && PS::filled(ri, gi)) {
                 if (vline && half_u) {
-                  e[s * NL + pos] = half ? e2 * a2 * b2 : e2 * a1 * b1;
-                  d[s * NL + pos] = half ? -ds * (a2 - b2) : ds * (a1 - b1);
+                  e[s * LL] = half ? e2 * pb * mb : e2 * pa * ma;
+                  d[s * LL] = half ? ds * (pb - mb) : ds * (pa - ma);
                 } else {
-                  e[s * NL + pos] = e2 * a1 * b1;
-                  e[s * NL + HN + pos] = e2 * a2 * b2;
-                  d[s * NL + pos] = ds * (a1 - b1);
-                  d[s * NL + HN + pos] = -ds * (a2 - b2);
+                  e[s * LL] = e2 * pa * ma;
+                  d[s * LL] = ds * (pa - ma);
+                  if constexpr (NT == 2) {
+                    e[s * LL + 16] = e2 * pb * mb;
+                    d[s * LL + 16] = ds * (pb - mb);
+                  }
                 }
               }
             }
           }
         }
         __syncthreads();
-        const bool first = gi == 0;
+        const bool first = gr == 0;
         if (pair == 0)
           planar_planes<T, N, 0>(op, Sa, Sb, ba * bb, S, ln, half, first);
         else if (pair == 1)
