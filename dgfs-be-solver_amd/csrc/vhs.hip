@@ -2350,18 +2350,48 @@ static int planar_slots() {
   return occ * cu_count();
 }
 
+// Parts that the planar gain's groups are split into, work items of their own
+// whose transforms the x pass sums: as many as keep one item per slot.  Only
+// for batches that would leave slots idle with one radial node to an item (one
+// point at 24^3 FP32 has 12 items of 6 groups each, 75 us of gain at one part).
+// An explicit group count and the allocation-free mode keep one part.
+template <typename T, int N>
+static int planar_split(const VhsHandle* h, int npts, int slots) {
+  const int ngr = static_cast<int>(h->pgroups.size());
+  if (h->groups_override > 0 || h->no_alloc) return 1;
+  const long items = static_cast<long>(npts) * h->Nrho * PlanarShape<T, N>::XH;
+  for (int g = ngr; g > 1; --g)
+    if (ngr % g == 0 && items * g <= slots) return g;
+  return 1;
+}
+
+// points' worth of transforms that any batch of up to npts points needs, so
+// that a smaller batch after a larger one (a captured one, say) finds its room
+template <typename T, int N>
+static size_t planar_tb_points(const VhsHandle* h, int npts, int slots) {
+  long most = npts;
+  const int ngr = static_cast<int>(h->pgroups.size());
+  if (h->groups_override > 0 || h->no_alloc) return static_cast<size_t>(most);
+  for (int g = 2; g <= ngr; ++g)
+    if (ngr % g == 0)
+      most = std::max(most, std::min<long>(npts, slots / (static_cast<long>(h->Nrho) * PlanarShape<T, N>::XH * g)) * g);
+  return static_cast<size_t>(most);
+}
+
 // planar-direction gain: spectra, operand form, the planes, x transform, finish
 template <typename T, int N>
 static int run_planar(VhsHandle* h, const double* fc, double* Qc, int npts, hipStream_t st) {
   if constexpr (planar_available<N>()) {
     using PS = PlanarShape<T, N>;
     const int slots = planar_slots<T, N>();
-    const int groups = pick_groups(h, npts * PS::XH, slots);
+    const int gsplit = planar_split<T, N>(h, npts, slots);
+    const int groups = gsplit > 1 ? h->Nrho : pick_groups(h, npts * PS::XH, slots);
     const int ppg = (h->Nrho + groups - 1) / groups;
     int rc = grow_ws(h, &h->plop, &h->cap_plop, static_cast<size_t>(npts) * PS::per_point * sizeof(T), "plane operands");
     if (!rc)
       rc = grow_ws(h, &h->Tb, &h->cap_tb,
-                   static_cast<size_t>(npts) * h->Nrho * PS::nslots * PS::NN * sizeof(cpx<T>), "plane transforms");
+                   planar_tb_points<T, N>(h, npts, slots) * h->Nrho * PS::nslots * PS::NN * sizeof(cpx<T>),
+                   "plane transforms");
     if (rc) return rc;
     GainArgs<T> ga;
     rc = stage_prep<T, N>(h, fc, npts, 1, slots, true, &ga, st, false);
@@ -2371,11 +2401,26 @@ static int run_planar(VhsHandle* h, const double* fc, double* Qc, int npts, hipS
     {
       PlanarPrepArgs<T> pa{fc, static_cast<T*>(h->plop), npts};
       const size_t lds = (static_cast<size_t>(4 * PS::RQ) + 3) * N * (N + 1) * sizeof(T);
-      const void* kfn = reinterpret_cast<const void*>(k_planar_prep<T, N>);
-      DGFS_HIP_TRY(hipFuncSetAttribute(kfn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
-      const int grid = rr_edge_grid(kfn, 256, lds, npts);
+      // 512 threads to a point where its workgroup is alone on a CU (one point
+      // at 24^3 FP32 30 -> 22 us) and always at 32^3, whose LDS leaves few
+      // workgroups room (4096 points FP32 1.07 -> 0.86 ms); 256 otherwise (512
+      // points at 24^3: 80 us, 103 us with 512 threads)
+      auto prep = [&](auto nth) -> int {
+        constexpr int NTH = decltype(nth)::value;
+        const void* kfn = reinterpret_cast<const void*>(k_planar_prep<T, N, NTH>);
+        DGFS_HIP_TRY(hipFuncSetAttribute(kfn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
+        const int grid = rr_edge_grid(kfn, NTH, lds, npts);
+        hipLaunchKernelGGL((k_planar_prep<T, N, NTH>), dim3(grid), dim3(NTH), lds, st, pa);
+        return DGFS_OK;
+      };
       KTimerT<VhsHandle> t0(h, 0, st);
-      hipLaunchKernelGGL((k_planar_prep<T, N>), dim3(grid), dim3(256), lds, st, pa);
+      if constexpr (N == 32)
+        rc = prep(std::integral_constant<int, 512>{});
+      else if (npts <= cu_count())
+        rc = prep(std::integral_constant<int, 512>{});
+      else
+        rc = prep(std::integral_constant<int, 256>{});
+      if (rc) return rc;
       DGFS_LAUNCH_CHECK("planar_prep");
       t0.stop();
     }
@@ -2384,7 +2429,8 @@ static int run_planar(VhsHandle* h, const double* fc, double* Qc, int npts, hipS
     pg.smat = static_cast<const T*>(h->smat);
     pg.beta = h->pbeta;
     pg.Tb = static_cast<cpx<T>*>(h->Tb);
-    pg.nitems = npts * groups * PS::XH;
+    pg.nitems = npts * groups * gsplit * PS::XH;
+    pg.gsplit = gsplit;
     pg.ngroups = groups;
     pg.ppg = ppg;
     pg.Nrho = h->Nrho;
@@ -2396,10 +2442,17 @@ static int run_planar(VhsHandle* h, const double* fc, double* Qc, int npts, hipS
     hipLaunchKernelGGL((k_vhs_gain_planar<T, N>), dim3(grid), dim3(PS::NW * 64), PS::lds_bytes, st, pg);
     DGFS_LAUNCH_CHECK("vhs_gain_planar");
     PlanarXfwdArgs<T> xa{static_cast<const cpx<T>*>(h->Tb), static_cast<const T*>(h->b1), h->wgt,
-                         static_cast<cpx<T>*>(h->Ghat), npts, h->Nrho};
-    const long cols = static_cast<long>(npts) * (N / 2 + 1) * N;
-    const long per = (sizeof(T) == 8) ? 128 : 256;
-    hipLaunchKernelGGL((k_planar_xfwd<T, N>), dim3(static_cast<unsigned>((cols + per - 1) / per)), dim3(256), 0, st, xa);
+                         static_cast<cpx<T>*>(h->Ghat), npts, h->Nrho, gsplit};
+    const int cols = npts * (N / 2 + 1) * N;
+    // the sum over p spread over waves where the pencils alone are less than
+    // one wave per SIMD
+    if (static_cast<long>(cols) * (sizeof(T) / 4) <= 64L * 4 * cu_count()) {
+      const int nb = (cols + 63) / 64 * static_cast<int>(sizeof(T) / 4);
+      hipLaunchKernelGGL((k_planar_xfwd<T, N, kXfwdWaves>), dim3(nb), dim3(xfwd_threads<kXfwdWaves>()), 0, st, xa);
+    } else {
+      const int per = xfwd_pencils<T, 1>();
+      hipLaunchKernelGGL((k_planar_xfwd<T, N, 1>), dim3((cols + per - 1) / per), dim3(xfwd_threads<1>()), 0, st, xa);
+    }
     DGFS_LAUNCH_CHECK("planar_xfwd");
     t1.stop();
     h->threads = PS::NW * 64;

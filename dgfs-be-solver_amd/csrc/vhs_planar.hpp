@@ -188,8 +188,8 @@ struct PlanarPrepArgs {
   int npts;
 };
 
-template <typename T, int N>
-__global__ __launch_bounds__(256) void k_planar_prep(PlanarPrepArgs<T> a) {
+template <typename T, int N, int NTH>
+__global__ __launch_bounds__(NTH, NTH / 128) void k_planar_prep(PlanarPrepArgs<T> a) {
   using PS = PlanarShape<T, N>;
   using MT = MmaTile<T>;
   constexpr int M = PS::M, Q = PS::Q, RQ = PS::RQ, NT = PS::NT, NN = PS::NN, n = PS::n, ND = PS::ND, PLN = PS::plane;
@@ -234,58 +234,56 @@ __global__ __launch_bounds__(256) void k_planar_prep(PlanarPrepArgs<T> a) {
   for (int pt = xcd_slot(); pt < a.npts; pt += gridDim.x) {
     const double* f = a.f + static_cast<size_t>(pt) * n;
     T* op = a.op + static_cast<size_t>(pt) * PS::per_point;
-    for (int e = tid; e < PP; e += 256) fx[e] = T(0);
+    for (int e = tid; e < PP; e += NTH) fx[e] = T(0);
     for (int g = 0; g < 4; ++g) {
       const int nq = (4 * (RQ - 1) + g < Q) ? NQ : NQ - 4;  // planes whose part index exists
       __syncthreads();
-      for (int e = tid; e < nq * NN; e += 256) {
+      for (int e = tid; e < nq * NN; e += NTH) {
         const int q = e / NN, rem = e - q * NN, y = rem / N, z = rem - y * N;
         pl[q * PP + y * (N + 1) + z] = static_cast<T>(f[image(4 * (q >> 2) + g, q & 3) * NN + rem]);
       }
       __syncthreads();
-      for (int e = tid; e < NN; e += 256) {
-        const int y = e / N, z = e - y * N;
-        double s = 0.0;
-        for (int q = 0; q < nq; ++q) {
-          const double v = pl[q * PP + y * (N + 1) + z];
-          s += ((g + q) & 1) ? -v : v;  // images 1 and 3 have the other parity (M is even)
+      // what is formed of the staged planes, as one range of tasks: the three
+      // axis pairs' parts (whole waves each), then the Nyquist sums
+      constexpr int EA = RQ * KP * N, EB = 2 * EA;
+      static_assert(EA % 64 == 0, "a wave's tasks are of one kind");
+      const int EC = EB + nq * KP * KP, ED = EC + NN, EE = ED + nq * N;
+      for (int e = tid; e < EE; e += NTH) {
+        if (e < EA) {  // (x, y), plane z = s
+          const int s = e % N, kv = (e / N) % KP, r = e / (N * KP), ku = 4 * r + g;
+          const T* p0 = pl + 4 * r * PP;
+          put(op + static_cast<size_t>(s) * PLN, ku, kv, ku < Q && kv < Q,
+              [&](int mu, int mv) -> double { return p0[mu * PP + image(kv, mv) * (N + 1) + s]; });
+        } else if (e < EB) {  // (x, z), plane y = s
+          const int t = e - EA, kv = t % KP, s = (t / KP) % N, r = t / (N * KP), ku = 4 * r + g;
+          const T* p0 = pl + 4 * r * PP + s * (N + 1);
+          put(op + static_cast<size_t>(N + s) * PLN, ku, kv, ku < Q && kv < Q,
+              [&](int mu, int mv) -> double { return p0[mu * PP + image(kv, mv)]; });
+        } else if (e < EC) {  // (y, z), plane x
+          const int t = e - EB, kv = t % KP, ku = (t / KP) % KP, q = t / (KP * KP);
+          const int x = image(4 * (q >> 2) + g, q & 3);
+          const T* p0 = pl + q * PP;
+          put(op + static_cast<size_t>(2 * N + x) * PLN, ku, kv, ku < Q && kv < Q,
+              [&](int mu, int mv) -> double { return p0[image(ku, mu) * (N + 1) + image(kv, mv)]; });
+        } else if (e < ED) {
+          const int t = e - EC, y = t / N, z = t - y * N;
+          double s = 0.0;
+          for (int q = 0; q < nq; ++q) {
+            const double v = pl[q * PP + y * (N + 1) + z];
+            s += ((g + q) & 1) ? -v : v;  // images 1 and 3 have the other parity (M is even)
+          }
+          fx[y * (N + 1) + z] = static_cast<T>(static_cast<double>(fx[y * (N + 1) + z]) + s);
+        } else {
+          const int d = e - ED, q = d / N, i = d - q * N, x = image(4 * (q >> 2) + g, q & 3);
+          double s = 0.0, t = 0.0;
+          for (int j = 0; j < N; ++j) {
+            const double v = pl[q * PP + j * (N + 1) + i], w = pl[q * PP + i * (N + 1) + j];
+            s += (j & 1) ? -v : v;
+            t += (j & 1) ? -w : w;
+          }
+          fy[x * (N + 1) + i] = static_cast<T>(s);
+          fz[x * (N + 1) + i] = static_cast<T>(t);
         }
-        fx[y * (N + 1) + z] = static_cast<T>(static_cast<double>(fx[y * (N + 1) + z]) + s);
-      }
-      for (int e = tid; e < nq * N; e += 256) {
-        const int q = e / N, i = e - q * N, x = image(4 * (q >> 2) + g, q & 3);
-        double s = 0.0, t = 0.0;
-        for (int j = 0; j < N; ++j) {
-          const double v = pl[q * PP + j * (N + 1) + i], w = pl[q * PP + i * (N + 1) + j];
-          s += (j & 1) ? -v : v;
-          t += (j & 1) ? -w : w;
-        }
-        fy[x * (N + 1) + i] = static_cast<T>(s);
-        fz[x * (N + 1) + i] = static_cast<T>(t);
-      }
-      for (int e = tid; e < RQ * KP * N; e += 256) {
-        const int s = e % N, kv = (e / N) % KP, r = e / (N * KP), ku = 4 * r + g;
-        const bool on = ku < Q && kv < Q;
-        const T* p0 = pl + 4 * r * PP;
-        // (x, y), plane z = s
-        put(op + static_cast<size_t>(s) * PLN, ku, kv, on,
-            [&](int mu, int mv) -> double { return p0[mu * PP + image(kv, mv) * (N + 1) + s]; });
-      }
-      for (int e = tid; e < RQ * KP * N; e += 256) {
-        const int kv = e % KP, s = (e / KP) % N, r = e / (N * KP), ku = 4 * r + g;
-        const bool on = ku < Q && kv < Q;
-        const T* p0 = pl + 4 * r * PP + s * (N + 1);
-        // (x, z), plane y = s
-        put(op + static_cast<size_t>(N + s) * PLN, ku, kv, on,
-            [&](int mu, int mv) -> double { return p0[mu * PP + image(kv, mv)]; });
-      }
-      for (int e = tid; e < nq * KP * KP; e += 256) {
-        const int kv = e % KP, ku = (e / KP) % KP, q = e / (KP * KP), x = image(4 * (q >> 2) + g, q & 3);
-        const bool on = ku < Q && kv < Q;
-        const T* p0 = pl + q * PP;
-        // (y, z), plane x
-        put(op + static_cast<size_t>(2 * N + x) * PLN, ku, kv, on,
-            [&](int mu, int mv) -> double { return p0[image(ku, mu) * (N + 1) + image(kv, mv)]; });
       }
     }
     __syncthreads();
@@ -301,7 +299,7 @@ __global__ __launch_bounds__(256) void k_planar_prep(PlanarPrepArgs<T> a) {
         default: return fz[s * (N + 1) + k];
       }
     };
-    for (int e = tid; e < 6 * 64 * RQ * NT; e += 256) {
+    for (int e = tid; e < 6 * 64 * RQ * NT; e += NTH) {
       const int t = e % NT, r = (e / NT) % RQ, lane = (e / (NT * RQ)) & 63, w = e / (64 * RQ * NT);
       const int g = lane >> 4, i = lane & 15, k = 4 * r + g;
       const int s = PS::slot(MT::reg(i), MT::grp(i)) + t * M;
@@ -313,7 +311,7 @@ __global__ __launch_bounds__(256) void k_planar_prep(PlanarPrepArgs<T> a) {
       for (int j = 0; j < 4; ++j) d[j] = static_cast<T>(0.25 * o[j]);
     }
     T* line = ny + 6 * PLN;
-    for (int e = tid; e < 3 * N; e += 256) {
+    for (int e = tid; e < 3 * N; e += NTH) {
       const int w = e / N, s = e - w * N;
       double acc = 0.0;
       for (int j = 0; j < N; ++j) {
@@ -331,8 +329,9 @@ struct PlanarGainArgs {
   const T* op;        // [npts][per_point]
   const T* smat;      // [Nrho][nshift][64][NR] operand values of R(shift), per lane [part][K step]
   const double* beta; // [Nrho][nshift]
-  cpx<T>* Tb;         // [npts][Nrho][N/2][N][N]
+  cpx<T>* Tb;         // [npts][Nrho][gsplit][N/2][N][N]
   int nitems, ngroups, ppg, Nrho, nshift, ngr;
+  int gsplit;  // parts of the groups, each a work item of its own
   PlanarGroup gr[kPlanarMaxGroups];
 };
 
@@ -497,9 +496,10 @@ __device__ __forceinline__ void planar_planes(const T* op, const T (&Sa)[PlanarS
       for (int v = 0; v < NT; ++v)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          T x = MT::template mirror<RQ>(mm[v][r ^ RQ]) * pp[v][r];
+          T x = ul[v][r] + ev - dl[v][r] * dv;
+          x += MT::template mirror<RQ>(mm[v][r ^ RQ]) * pp[v][r];
           x += MT::template mirror<RQ>(mp[v][r]) * pm[v][r ^ RQ];
-          q[v][r] = prev[v][r] + (x + (ul[v][r] + ev - dl[v][r] * dv));
+          q[v][r] = prev[v][r] + x;
         }
       if (ok) {
 #pragma unroll
@@ -527,12 +527,13 @@ __global__ __launch_bounds__((PlanarShape<T, N>::NW * 64), (PlanarShape<T, N>::W
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int ri = MT::reg(i), gi = MT::grp(i);
   for (int item = xcd_slot(); item < a.nitems; item += gridDim.x) {
-    const int half = (XH == 2) ? item % 2 : 0, pg = item / XH;
+    const int half = (XH == 2) ? item % 2 : 0, part = (item / XH) % a.gsplit, pg = item / (XH * a.gsplit);
     const int pt = pg / a.ngroups, grp = pg - pt * a.ngroups;
+    const int gr0 = part * a.ngr / a.gsplit, gr1 = (part + 1) * a.ngr / a.gsplit;
     const int p0 = grp * a.ppg, p1 = min(p0 + a.ppg, a.Nrho);
     const T* op = a.op + static_cast<size_t>(pt) * PS::per_point;
     for (int p = p0; p < p1; ++p) {
-      for (int gr = 0; gr < a.ngr; ++gr) {
+      for (int gr = gr0; gr < gr1; ++gr) {
         const int pair = a.gr[gr].pair, ia = a.gr[gr].ia, ib = a.gr[gr].ib;
         T Sa[NR], Sb[NR];
         {
@@ -594,7 +595,7 @@ __global__ __launch_bounds__((PlanarShape<T, N>::NW * 64), (PlanarShape<T, N>::W
           }
         }
         __syncthreads();
-        const bool first = gr == 0;
+        const bool first = gr == gr0;
         if (pair == 0)
           planar_planes<T, N, 0>(op, Sa, Sb, ba * bb, S, ln, half, first);
         else if (pair == 1)
@@ -631,7 +632,7 @@ __global__ __launch_bounds__((PlanarShape<T, N>::NW * 64), (PlanarShape<T, N>::W
         }
         FFT<T, N, -1>::run(v);
         if (act) {
-          cpx<T>* t = a.Tb + ((static_cast<size_t>(pt) * a.Nrho + p) * PS::nslots + half * NPP + pp) * NN + l;
+          cpx<T>* t = a.Tb + (((static_cast<size_t>(pt) * a.Nrho + p) * a.gsplit + part) * PS::nslots + half * NPP + pp) * NN + l;
 #pragma unroll
           for (int y = 0; y < N; ++y) t[y * N] = v[y];
         }
@@ -643,27 +644,30 @@ __global__ __launch_bounds__((PlanarShape<T, N>::NW * 64), (PlanarShape<T, N>::W
 // x-forward transform and the weighted sum over p:
 // G^[pt](k) = sum_p w_p b1_p(k) FFT_x(T_p)(k).  A thread takes the pencil
 // (ky, kz) with ky <= N/2 and, as S_p is real, writes its mirror image
-// (-ky, -kz) too.  HV of the N kx sums are kept per pass (all in FP32, half in
-// FP64, whose waves share a pencil), in registers over p.  Bound by reading T.
+// (-ky, -kz) too.  The kx sums are kept in registers over p: all in FP32, half
+// of them per wave in FP64.  Bound by reading T where the pencils fill the
+// chip; PW > 1 spreads the sum over p of 64 pencils over PW waves for batches
+// that leave it idle (one point at 24^3 FP32: 51 us with one wave per pencil
+// block, whose 12 reads of T follow one another).
 template <typename T>
 struct PlanarXfwdArgs {
   const cpx<T>* Tb;
   const T* b1;        // [Nrho][n]
   const double* wgt;  // [Nrho]
   cpx<T>* Ghat;       // [npts][n]
-  int npts, Nrho;
+  int npts, Nrho, gsplit;
 };
 
 template <typename T, int N, int K0, int KN>
-__device__ __forceinline__ void planar_xfwd_part(const PlanarXfwdArgs<T>& a, int pt, int ky, int kz) {
+__device__ __forceinline__ void planar_xfwd_sum(const PlanarXfwdArgs<T>& a, int pt, int i1, int i2, int q0, int dq,
+                                                cpx<T> (&acc)[KN]) {
   using PS = PlanarShape<T, N>;
   constexpr int NN = N * N, n = NN * N;
-  const int i1 = ky * N + kz, my = (N - ky) % N, mz = (N - kz) % N, i2 = my * N + mz;
-  cpx<T> acc[KN];
 #pragma unroll
   for (int k = 0; k < KN; ++k) acc[k] = cpx<T>{T(0), T(0)};
-  for (int p = 0; p < a.Nrho; ++p) {
-    const cpx<T>* Tp = a.Tb + (static_cast<size_t>(pt) * a.Nrho + p) * PS::nslots * NN;
+  for (int q = q0; q < a.Nrho * a.gsplit; q += dq) {
+    const int p = q / a.gsplit;
+    const cpx<T>* Tp = a.Tb + (static_cast<size_t>(pt) * a.Nrho * a.gsplit + q) * PS::nslots * NN;
     cpx<T> A[N / 2], B[N / 2];
 #pragma unroll
     for (int s = 0; s < N / 2; ++s) {
@@ -683,6 +687,38 @@ __device__ __forceinline__ void planar_xfwd_part(const PlanarXfwdArgs<T>& a, int
 #pragma unroll
     for (int k = 0; k < KN; ++k) acc[k] = acc[k] + (wp * b[static_cast<size_t>(k + K0) * NN]) * v[k + K0];
   }
+}
+
+template <typename T, int N, int K0, int KN, int PW>
+__device__ __forceinline__ void planar_xfwd_part(const PlanarXfwdArgs<T>& a, cpx<T>* red, int col, int w) {
+  constexpr int NN = N * N, n = NN * N, NV = (N / 2 + 1) * N;
+  const int lane = threadIdx.x & 63;
+  bool act = col < a.npts * NV;
+  const int pt = act ? col / NV : 0, i1 = act ? col - pt * NV : 0, ky = i1 / N, kz = i1 - ky * N;
+  const int i2 = ((N - ky) % N) * N + (N - kz) % N;
+  // on the self-conjugate rows ky = 0 and N/2 the second half of kz is the
+  // mirror image of the first
+  if ((ky == 0 || ky == N / 2) && kz > N / 2) act = false;
+  cpx<T> acc[KN];
+  if (act) planar_xfwd_sum<T, N, K0, KN>(a, pt, i1, i2, PW > 1 ? w : 0, PW, acc);
+  if constexpr (PW > 1) {
+#pragma unroll 1
+    for (int h = PW / 2; h; h >>= 1) {
+      cpx<T>* r = red + (w & (h - 1)) * KN * 64 + lane;
+      if (act && w >= h && w < 2 * h) {
+#pragma unroll
+        for (int k = 0; k < KN; ++k) r[k * 64] = acc[k];
+      }
+      __syncthreads();
+      if (act && w < h) {
+#pragma unroll
+        for (int k = 0; k < KN; ++k) acc[k] = acc[k] + r[k * 64];
+      }
+      __syncthreads();
+    }
+    if (w) return;
+  }
+  if (!act) return;
   cpx<T>* G = a.Ghat + static_cast<size_t>(pt) * n;
 #pragma unroll
   for (int k = 0; k < KN; ++k) G[static_cast<size_t>(k + K0) * NN + i1] = acc[k];
@@ -695,24 +731,35 @@ __device__ __forceinline__ void planar_xfwd_part(const PlanarXfwdArgs<T>& a, int
   }
 }
 
-template <typename T, int N>
-__global__ __launch_bounds__(256) void k_planar_xfwd(PlanarXfwdArgs<T> a) {
-  constexpr int NV = (N / 2 + 1) * N, SPLIT = sizeof(T) == 8 ? 2 : 1, PER = 256 / SPLIT;
-  const int w = threadIdx.x / 64, lane = threadIdx.x & 63;
-  const long col = static_cast<long>(blockIdx.x) * PER + (w / SPLIT) * 64 + lane;
-  if (col >= static_cast<long>(a.npts) * NV) return;
-  const int pt = static_cast<int>(col / NV), idx = static_cast<int>(col - static_cast<long>(pt) * NV);
-  const int ky = idx / N, kz = idx - (idx / N) * N;
-  // on the self-conjugate rows ky = 0 and N/2 the second half of kz is the
-  // mirror image of the first
-  if ((ky == 0 || ky == N / 2) && kz > N / 2) return;
-  if constexpr (SPLIT == 1) {
-    planar_xfwd_part<T, N, 0, N>(a, pt, ky, kz);
-  } else {
-    if (w & 1)
-      planar_xfwd_part<T, N, N / 2, N / 2>(a, pt, ky, kz);
+// waves over p of 64 pencils, and threads of a workgroup
+constexpr int kXfwdWaves = 8;
+template <int PW>
+constexpr int xfwd_threads() {
+  return PW > 1 ? 64 * PW : 256;
+}
+// pencils per workgroup (FP64: two waves, or two workgroups, per 64 pencils)
+template <typename T, int PW>
+constexpr int xfwd_pencils() {
+  return PW > 1 ? 64 : (sizeof(T) == 8 ? 128 : 256);
+}
+
+template <typename T, int N, int PW>
+__global__ __launch_bounds__((xfwd_threads<PW>()), (PW == 1 && sizeof(T) == 4 ? 3 : 1)) void k_planar_xfwd(PlanarXfwdArgs<T> a) {
+  constexpr int SPLIT = sizeof(T) == 8 ? 2 : 1, KN = N / SPLIT;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x & 63;
+  if constexpr (PW > 1) {
+    __shared__ cpx<T> red[PW / 2 * KN * 64];
+    const int col = static_cast<int>(blockIdx.x / SPLIT) * 64 + lane;
+    if (SPLIT == 2 && (blockIdx.x & 1))
+      planar_xfwd_part<T, N, N - KN, KN, PW>(a, red, col, w);
     else
-      planar_xfwd_part<T, N, 0, N / 2>(a, pt, ky, kz);
+      planar_xfwd_part<T, N, 0, KN, PW>(a, red, col, w);
+  } else {
+    const int col = static_cast<int>(blockIdx.x) * xfwd_pencils<T, 1>() + (w / SPLIT) * 64 + lane;
+    if (SPLIT == 2 && (w & 1))
+      planar_xfwd_part<T, N, N - KN, KN, 1>(a, nullptr, col, 0);
+    else
+      planar_xfwd_part<T, N, 0, KN, 1>(a, nullptr, col, 0);
   }
 }
 

@@ -122,3 +122,29 @@ def test_other_designs_keep_the_general_gain(device):
         say("general design", len(sz))
         auto, named = run(make(N, sz, 64), f, device), run(make(N, sz, 64, algorithm=6), f, device)
         assert np.array_equal(auto, named)
+
+
+@pytest.mark.parametrize("N,npts", [(16, 400), (24, 60)])
+def test_small_batch_captured_after_a_larger_one(N, npts, device):
+    """A batch small enough to split its groups over work items finds room for
+    the parts' transforms in the workspace of a larger batch: captured without
+    an allocation, every replay equal to the eager result."""
+    import torch
+    rng = np.random.default_rng(N)
+    f = rng.uniform(0.0, 1.0, size=(npts, N ** 3))
+    say("planar capture", N, npts)
+    op = make(N, designs()["m12"], 64)
+    big = run(op, f, device)
+    for n in (1, 3, 11):
+        ft = torch.as_tensor(f[:n], device=device)
+        Qt = torch.zeros_like(ft)
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            op.eval_contig(ft.data_ptr(), Qt.data_ptr(), n, torch.cuda.current_stream().cuda_stream)
+        eager = run(op, f[:n], device)
+        assert rel(eager, big[:n]) < 1e-12
+        for _ in range(3):
+            Qt.zero_()
+            g.replay()
+            torch.cuda.synchronize()
+            assert np.array_equal(Qt.cpu().numpy(), eager)
