@@ -123,6 +123,30 @@ __device__ __forceinline__ void pencil_accumulate(const GA& G, const BA& b, T w,
   }
 }
 
+// acc summed over the PW waves of a workgroup into wave 0, halving the waves
+// that hold a sum; red holds PW / 2 sums of 64 lanes.  `act`: this lane's sum
+// exists (the same in every wave).
+template <typename T, int KN, int PW>
+__device__ __forceinline__ void wave_tree_sum(cpx<T> (&acc)[KN], cpx<T>* red, int w, int lane, bool act) {
+#pragma unroll 1
+  for (int h = PW / 2; h; h >>= 1) {
+    cpx<T>* r = red + (w & (h - 1)) * KN * 64 + lane;
+    if (act && w >= h && w < 2 * h) {
+#pragma unroll
+      for (int k = 0; k < KN; ++k) r[k * 64] = acc[k];
+    }
+    __syncthreads();
+    if (act && w < h) {
+#pragma unroll
+      for (int k = 0; k < KN; ++k) acc[k] = acc[k] + r[k * 64];
+    }
+    __syncthreads();
+  }
+}
+
+// waves that share a sum over the radial nodes where a batch leaves the chip idle
+constexpr int kXfwdWaves = 8;
+
 // Consecutive workgroups of a launch go round-robin to the 8 XCDs of an
 // MI355X, each XCD with its own L2.  xcd_slot() renumbers block b so that the
 // blocks of one XCD hold consecutive slots (persistent grids then give the

@@ -1168,39 +1168,60 @@ struct XfwdArgs {
   int npts, Nrho;
 };
 
-template <typename T, int N, int K0>
-__device__ __forceinline__ void xfwd_half(const XfwdArgs<T>& a, int pt, int idx) {
+template <typename T, int N, int K0, int PW>
+__device__ __forceinline__ void xfwd_half(const XfwdArgs<T>& a, cpx<T>* red, long col, int w) {
   constexpr int NN = N * N, n = NN * N, H = N / 2;
+  const int lane = threadIdx.x & 63;
+  const bool act = col < static_cast<long>(a.npts) * NN;
+  if (PW == 1 && !act) return;
+  const int pt = act ? static_cast<int>(col / NN) : 0, idx = act ? static_cast<int>(col - static_cast<long>(pt) * NN) : 0;
   cpx<T> acc[H];
 #pragma unroll
   for (int k = 0; k < H; ++k) acc[k] = cpx<T>{T(0), T(0)};
-  for (int p = 0; p < a.Nrho; ++p) {
-    const cpx<T>* Tp = a.Tb + (static_cast<size_t>(pt) * a.Nrho + p) * n + idx;
-    cpx<T> v[N];
+  if (act) {
+    for (int p = w; p < a.Nrho; p += PW) {
+      const cpx<T>* Tp = a.Tb + (static_cast<size_t>(pt) * a.Nrho + p) * n + idx;
+      cpx<T> v[N];
 #pragma unroll
-    for (int x = 0; x < N; ++x) v[x] = Tp[static_cast<size_t>(x) * NN];
-    FFT<T, N, -1>::run(v);
-    const T wp = static_cast<T>(a.wgt[p]);
-    const T* b = a.b1 + static_cast<size_t>(p) * n + idx;
+      for (int x = 0; x < N; ++x) v[x] = Tp[static_cast<size_t>(x) * NN];
+      FFT<T, N, -1>::run(v);
+      const T wp = static_cast<T>(a.wgt[p]);
+      const T* b = a.b1 + static_cast<size_t>(p) * n + idx;
 #pragma unroll
-    for (int k = 0; k < H; ++k) acc[k] = acc[k] + (wp * b[static_cast<size_t>(k + K0) * NN]) * v[k + K0];
+      for (int k = 0; k < H; ++k) acc[k] = acc[k] + (wp * b[static_cast<size_t>(k + K0) * NN]) * v[k + K0];
+    }
   }
+  if constexpr (PW > 1) {
+    wave_tree_sum<T, H, PW>(acc, red, w, lane, act);
+    if (w) return;
+  }
+  if (!act) return;
   cpx<T>* G = a.Ghat + static_cast<size_t>(pt) * n + idx;
 #pragma unroll
   for (int k = 0; k < H; ++k) G[static_cast<size_t>(k + K0) * NN] = acc[k];
 }
 
-template <typename T, int N>
-__global__ __launch_bounds__(256) void k_vhs_xfwd(XfwdArgs<T> a) {
-  constexpr int NN = N * N;
-  const int w = threadIdx.x / 64, lane = threadIdx.x - (threadIdx.x / 64) * 64;
-  const long col = static_cast<long>(blockIdx.x) * 128 + (w >> 1) * 64 + lane;
-  if (col >= static_cast<long>(a.npts) * NN) return;
-  const int pt = static_cast<int>(col / NN), idx = static_cast<int>(col - static_cast<long>(pt) * NN);
-  if (w & 1)
-    xfwd_half<T, N, N / 2>(a, pt, idx);
-  else
-    xfwd_half<T, N, 0>(a, pt, idx);
+// PW = 1: two waves (the kx halves) per 64 pencils, all radial nodes in turn.
+// PW > 1: a workgroup per 64 pencils and kx half, the radial nodes spread over
+// PW waves, for batches whose pencils are less than a wave per SIMD (4 points
+// at 16^3 FP64, 8 nodes: 17.4 -> 5.7 us).
+template <typename T, int N, int PW>
+__global__ __launch_bounds__(PW > 1 ? 64 * PW : 256) void k_vhs_xfwd(XfwdArgs<T> a) {
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x & 63;
+  if constexpr (PW > 1) {
+    __shared__ cpx<T> red[PW / 2 * (N / 2) * 64];
+    const long col = static_cast<long>(blockIdx.x >> 1) * 64 + lane;
+    if (blockIdx.x & 1)
+      xfwd_half<T, N, N / 2, PW>(a, red, col, w);
+    else
+      xfwd_half<T, N, 0, PW>(a, red, col, w);
+  } else {
+    const long col = static_cast<long>(blockIdx.x) * 128 + (w >> 1) * 64 + lane;
+    if (w & 1)
+      xfwd_half<T, N, N / 2, 1>(a, nullptr, col, 0);
+    else
+      xfwd_half<T, N, 0, 1>(a, nullptr, col, 0);
+  }
 }
 
 template <typename T>
@@ -1508,7 +1529,7 @@ __global__ __launch_bounds__(RRShape<N>::NT) void k_vhs_finalize_rr(FinRRArgs<T>
   }
 }
 
-// One-pencil register-resident prep and finalize (FP32, N = 24), in the
+// One-pencil register-resident prep and finalize (FP32 N = 24, FP64 N = 16), in the
 // one-pencil gain kernel's layout: N*N threads per point, thread t = g N + l,
 // the field exchanged through LDS ([kx][y][z], kx stride N (N + 1)) and the
 // in-plane transposes through padded kx planes.
@@ -1953,6 +1974,15 @@ template <typename T, int N>
 constexpr bool rr1_available() {
   return std::is_same<T, float>::value && (N == 16 || N == 24);
 }
+// prep and finalize through the one-pencil kernels: FP64 at N = 16 as well,
+// whose exchange field (68 KB) leaves room for two workgroups on a CU, instead
+// of scratch cubes in global memory (4 points: prep 15.1 -> 5.4 us, finalize
+// 18.2 -> 6.8 us; 1000 points: prep 50 -> 28 us, finalize and projection 85 ->
+// 51 us).  At N = 24 the FP64 field does not fit.
+template <typename T, int N>
+constexpr bool rr1_edges() {
+  return rr1_available<T, N>() || (std::is_same<T, double>::value && N == 16);
+}
 static bool rr2_ok(const VhsHandle* h) { return h->prec == 32 && (h->N == 16 || h->N == 32); }
 static bool rr1_ok(const VhsHandle* h) { return h->prec == 32 && (h->N == 16 || h->N == 24); }
 static bool slab_ok(const VhsHandle* h) { return h->N == 16 || h->N == 24 || h->N == 32; }
@@ -2155,7 +2185,11 @@ static int run_gain_slab(VhsHandle* h, int npts, int groups, int ppg, hipStream_
     XfwdArgs<T> xa{static_cast<const cpx<T>*>(h->Tb), static_cast<const T*>(h->b1), h->wgt,
                    static_cast<cpx<T>*>(h->Ghat), npts, h->Nrho};
     const long cols = static_cast<long>(npts) * NN;
-    hipLaunchKernelGGL((k_vhs_xfwd<T, N>), dim3(static_cast<unsigned>((cols + 127) / 128)), dim3(256), 0, st, xa);
+    if (2 * cols <= 64L * 4 * cu_count())
+      hipLaunchKernelGGL((k_vhs_xfwd<T, N, kXfwdWaves>), dim3(static_cast<unsigned>((cols + 63) / 64 * 2)),
+                         dim3(64 * kXfwdWaves), 0, st, xa);
+    else
+      hipLaunchKernelGGL((k_vhs_xfwd<T, N, 1>), dim3(static_cast<unsigned>((cols + 127) / 128)), dim3(256), 0, st, xa);
     DGFS_LAUNCH_CHECK("vhs_xfwd");
     t1.stop();
     h->threads = SS::NT;
@@ -2240,7 +2274,7 @@ static int stage_prep(VhsHandle* h, const double* fc, int npts, int groups, int 
       DGFS_LAUNCH_CHECK("vhs_prep_rr");
       done = true;
     }
-  } else if constexpr (rr1_available<T, N>()) {
+  } else if constexpr (rr1_edges<T, N>()) {
     if (rr) {  // one-pencil register-resident prep
       const size_t lds = static_cast<size_t>(RR1Shape<N>::field) * sizeof(cpx<T>);
       DGFS_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(k_vhs_prep_rr1<T, N>),
@@ -2289,7 +2323,7 @@ static int stage_finish(VhsHandle* h, const double* fc, double* Qc, int npts, in
     DGFS_LAUNCH_CHECK("vhs_finalize_rr");
     t2.stop();
     return DGFS_OK;
-  } else if constexpr (rr1_available<T, N>()) {
+  } else if constexpr (rr1_edges<T, N>()) {
     FinRRArgs<T> fr;
     fr.fa = fa;
     std::memcpy(fr.Ainv, h->Ainv, sizeof(fr.Ainv));

@@ -699,23 +699,11 @@ __device__ __forceinline__ void planar_xfwd_part(const PlanarXfwdArgs<T>& a, cpx
   // on the self-conjugate rows ky = 0 and N/2 the second half of kz is the
   // mirror image of the first
   if ((ky == 0 || ky == N / 2) && kz > N / 2) act = false;
+  if (PW == 1 && !act) return;
   cpx<T> acc[KN];
   if (act) planar_xfwd_sum<T, N, K0, KN>(a, pt, i1, i2, PW > 1 ? w : 0, PW, acc);
   if constexpr (PW > 1) {
-#pragma unroll 1
-    for (int h = PW / 2; h; h >>= 1) {
-      cpx<T>* r = red + (w & (h - 1)) * KN * 64 + lane;
-      if (act && w >= h && w < 2 * h) {
-#pragma unroll
-        for (int k = 0; k < KN; ++k) r[k * 64] = acc[k];
-      }
-      __syncthreads();
-      if (act && w < h) {
-#pragma unroll
-        for (int k = 0; k < KN; ++k) acc[k] = acc[k] + r[k * 64];
-      }
-      __syncthreads();
-    }
+    wave_tree_sum<T, KN, PW>(acc, red, w, lane, act);
     if (w) return;
   }
   if (!act) return;
@@ -731,8 +719,7 @@ __device__ __forceinline__ void planar_xfwd_part(const PlanarXfwdArgs<T>& a, cpx
   }
 }
 
-// waves over p of 64 pencils, and threads of a workgroup
-constexpr int kXfwdWaves = 8;
+// threads of a workgroup
 template <int PW>
 constexpr int xfwd_threads() {
   return PW > 1 ? 64 * PW : 256;
