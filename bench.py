@@ -974,19 +974,24 @@ def main():
     gain_ms, gain_n = tim["gain"]
     launch_s = gain_ms / max(gain_n, 1) / 1e3
     pts_per_launch = P * args.steps / max(gain_n, 1)
-    flops = own_flops(nv, K, args.nrho)
+    planar = bool(op32.planar) and not args.algorithm
+    # planar-direction gain: per (p, pair of mirrored directions) 3 N lines' worth
+    # of moves on each of N planes, N^2 operations a line; the other kernels:
+    # their transforms
+    flops = args.nrho * (args.M // 2) * 3 * nv ** 4 if planar else own_flops(nv, K, args.nrho)
     achieved_tf = flops * pts_per_launch / launch_s / 1e12
     bq32 = algorithmic_bytes(nv, K, 8)
     traffic, traffic_src = None, None
     tname = {2: f"vhs_gain_rr_fp32_n{nv}_traffic.json", 3: f"vhs_gain_rr_inl_fp32_n{nv}_traffic.json",
              4: f"vhs_gain_rr1_fp32_n{nv}_traffic.json", 5: f"vhs_gain_rr_wl_fp32_n{nv}_traffic.json"}.get(algo, "")
-    tr = read_traffic(tname)
+    tr = None if planar else read_traffic(tname)
     if tr and tr.get("points_per_dispatch"):
         traffic = tr["bytes_per_dispatch"] * pts_per_launch / tr["points_per_dispatch"]
         traffic_src = (f"profiles/{tname}: rocprofv3 FETCH_SIZE and WRITE_SIZE runs of this kernel "
                        f"({tr.get('points_per_dispatch')} points per dispatch), scaled by the copy-kernel "
                        f"calibration and to this launch's points; not measured in this run")
-    kname = (f"k_vhs_gain_rr<float,{nv},{'true' if algo == 3 else 'false'}>" if algo in (2, 3)
+    kname = (f"k_vhs_gain_planar<float,{nv}>" if planar
+             else f"k_vhs_gain_rr<float,{nv},{'true' if algo == 3 else 'false'}>" if algo in (2, 3)
              else f"k_vhs_gain_rr<float,{nv},false,true>" if algo == 5
              else f"k_vhs_gain_rr1<float,{nv}>" if algo == 4 else f"k_vhs_gain<float,{nv}>")
 
@@ -1023,10 +1028,14 @@ def main():
             "traffic": traffic,
             "traffic_source": traffic_src,
             "kernel": kname,
-            "compute_unit": "FP32 vector ALU (FFT butterflies and products; packed FP32 is disabled by the "
+            "compute_unit": "FP32 matrix cores (the moves) and vector ALU (sums, products, y and z transforms)"
+                            if planar else
+                            "FP32 vector ALU (FFT butterflies and products; packed FP32 is disabled by the "
                             "build, so 78.6 TFLOP/s of the 157.3 is reachable)",
             "flops_per_eval": flops,
-            "flops_model": "this kernel's own count: K packed complex 3D transforms, Nrho forward transforms, "
+            "flops_model": "the matrix products alone: 3 N^4 per radial node and pair of directions; the "
+                           "launch time includes the x-forward pass" if planar else
+                           "this kernel's own count: K packed complex 3D transforms, Nrho forward transforms, "
                            "3 more, 3K Nyquist-plane 2D transforms (5 N log2 N each), 24 K n pointwise",
             "points_per_launch": pts_per_launch,
             "avg_launch_ms": launch_s * 1e3,
@@ -1035,13 +1044,16 @@ def main():
             "hbm_counter_frac": (traffic / launch_s / HBM_PEAK) if traffic else None,
             "frac_survey_flops": survey_flops(nv, K) * pts_per_launch / launch_s / FP32_PEAK,
             "frac_ref_dataflow": bq32 * pts_per_launch / launch_s / HBM_PEAK,
-            "frac_own_transforms": own_bytes(nv, K, args.nrho, 8) * pts_per_launch / launch_s / HBM_PEAK,
+            "frac_own_transforms": None if planar else own_bytes(nv, K, args.nrho, 8) * pts_per_launch / launch_s / HBM_PEAK,
             "algorithmic_bytes_per_eval": bq32,
-            "note": "frac = this kernel's FLOPs / FP32 peak (the kernel keeps every transform on chip and is "
-                    "bound by VALU issue, LDS transposes and barriers); frac_ref_dataflow prices the "
+            "note": ("frac = this kernel's FLOPs / FP32 peak (its matrix products and its vector work share the "
+                     "SIMDs' issue slots); " if planar else
+                     "frac = this kernel's FLOPs / FP32 peak (the kernel keeps every transform on chip and is "
+                     "bound by VALU issue, LDS transposes and barriers); ") +
+                    "frac_ref_dataflow prices the "
                     "reference dataflow's 3K+3 transforms crossing HBM once (B_Q = 2*8*n*(3K+3)) and "
                     "exceeds 1 because they never do; frac_survey_flops counts the reference dataflow's "
-                    "(3K+3) transforms, 2.25x this kernel's",
+                    "(3K+3) transforms, 2.25x the transform kernels' count",
         },
         "kernel_ms_per_step": {k: v[0] / args.steps for k, v in tim.items()},
         "event_ms_total": ev_ms,
