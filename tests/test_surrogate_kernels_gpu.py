@@ -46,7 +46,7 @@ def test_gemm_f32_edges(M, N, K, ta, tb, device):
 @pytest.mark.parametrize("P", [1, 3, 17])
 def test_layers_small_batches(P, device):
     """Forward and every gradient at small and odd batches against the FP64
-    checker: 1e-5 of each output's norm (FP32 sums of up to 512 P terms)."""
+    oracle: 1e-5 of each output's norm (FP32 sums of up to 512 P terms)."""
     import torch
     from dgfs_hip.surrogate import SpectralSurrogate
     sur = SpectralSurrogate(8, 5.0, (10.0 / 8) ** 3, 0.38, 1.0, max_batch=32, device=device, seed=3)
@@ -73,7 +73,7 @@ def test_layers_small_batches(P, device):
 def test_encode_decode_grids(N, device):
     """Encoder and projecting decoder on every built grid, one point and more
     points than fit one sweep of workgroups' columns, against the FP64
-    checker: FP32 rounding on the modes, 1e-10 on the FP64 outputs plus the
+    oracle: FP32 rounding on the modes, 1e-10 on the FP64 outputs plus the
     forward error of the per-axis factorisations, at most about eps times the
     condition number of their Gram matrices, three axes, with a margin of 4.
     (At N = 8 the eight functions fill the eight points: the Gram matrix is
