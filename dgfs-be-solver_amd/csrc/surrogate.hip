@@ -30,6 +30,9 @@
 #include <cstdint>
 #include <cstring>
 #include <memory>
+#include <mutex>
+#include <new>
+#include <optional>
 #include <vector>
 
 #include "common.hpp"
@@ -377,12 +380,71 @@ __global__ __launch_bounds__(256) void k_gemm_reduce(const float* __restrict__ p
 constexpr size_t kGemmPartFloats = size_t{1} << 24;
 struct GemmWs {
   float* part = nullptr;
+  // a workspace that calls on several streams and threads share: a product
+  // waits on the device for the reduction of the one before (event `done`),
+  // and the mutex keeps wait, launches and record of one call together
+  bool shared = false;
+  std::mutex mu;
+  hipEvent_t done = nullptr;
   int init() {
     if (!part) DGFS_HIP_TRY(hipMalloc(&part, kGemmPartFloats * sizeof(float)));
+    if (shared && !done) DGFS_HIP_TRY(hipEventCreateWithFlags(&done, hipEventDisableTiming));
     return DGFS_OK;
   }
-  ~GemmWs() { (void)hipFree(part); }
+  ~GemmWs() {
+    (void)hipFree(part);
+    if (done) (void)hipEventDestroy(done);
+  }
 };
+
+// one split product's hold on the workspace, from before its launch to after
+// its reduction's
+class GemmWsUse {
+ public:
+  GemmWsUse(GemmWs* ws, hipStream_t st) : ws_(ws), st_(st) {
+    if (ws_->shared) lock_ = std::unique_lock<std::mutex>(ws_->mu);
+  }
+  GemmWsUse(const GemmWsUse&) = delete;
+  GemmWsUse& operator=(const GemmWsUse&) = delete;
+  int begin() {
+    int rc = ws_->init();
+    if (rc || !ws_->shared) return rc;
+    DGFS_HIP_TRY(hipStreamWaitEvent(st_, ws_->done, 0));
+    held_ = true;
+    return DGFS_OK;
+  }
+  ~GemmWsUse() {
+    if (held_ && hipEventRecord(ws_->done, st_) != hipSuccess) (void)hipStreamSynchronize(st_);
+  }
+
+ private:
+  GemmWs* ws_;
+  hipStream_t st_;
+  std::unique_lock<std::mutex> lock_;
+  bool held_ = false;
+};
+
+// the current device's workspace for products without a handle, or null on a
+// stream under capture: the replays of the graph would not be ordered against
+// other calls, so a captured product runs unsplit
+static GemmWs* shared_gemm_ws(hipStream_t st) {
+  constexpr int kMaxDev = 64;
+  static std::mutex mu;
+  static GemmWs* table[kMaxDev] = {};  // process-lifetime (released by the driver at exit)
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  int dev = 0;
+  if (hipStreamIsCapturing(st, &cap) != hipSuccess || hipGetDevice(&dev) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  if (cap != hipStreamCaptureStatusNone || dev < 0 || dev >= kMaxDev) return nullptr;
+  std::lock_guard<std::mutex> lock(mu);
+  if (!table[dev]) {
+    table[dev] = new (std::nothrow) GemmWs();
+    if (table[dev]) table[dev]->shared = true;
+  }
+  return table[dev];
+}
 
 static int gemm(GemmWs* ws, int transA, int transB, int M, int N, int K, float alpha, const float* A, long lda,
                 const float* B, long ldb, float beta, float* C, long ldc, bool bf16, hipStream_t st) {
@@ -397,10 +459,11 @@ static int gemm(GemmWs* ws, int transA, int transB, int M, int N, int K, float a
       int kchunk = (K + splits - 1) / splits;
       kchunk = (kchunk + kBK - 1) / kBK * kBK;
       splits = (K + kchunk - 1) / kchunk;
-      int rc = ws->init();
-      if (rc) return rc;
       if (static_cast<size_t>(splits) * M * N > kGemmPartFloats) splits = 1;
       else {
+        GemmWsUse use(ws, st);
+        int rc = use.begin();
+        if (rc) return rc;
         g.kchunk = kchunk;
         g.part = ws->part;
         hipLaunchKernelGGL(k_gemm_bf16_big<0>, dim3(gx, gy, splits), dim3(256), 0, st, g);
@@ -425,13 +488,15 @@ static int gemm(GemmWs* ws, int transA, int transB, int M, int N, int K, float a
     const int bx = (N + kFN - 1) / kFN, by = (M + kFM - 1) / kFM;
     const long tl = static_cast<long>(bx) * by, want = 2L * cu_count();
     int splits = 1;
+    std::optional<GemmWsUse> use;
     if (ws && tl < want && K >= 512) splits = static_cast<int>(std::min<long>(want / tl, K / 256));
     if (splits > 1) {
       int kchunk = (K + splits - 1) / splits;
       kchunk = (kchunk + kFK - 1) / kFK * kFK;
       splits = (K + kchunk - 1) / kchunk;
       if (splits > 1 && static_cast<size_t>(splits) * M * N <= kGemmPartFloats) {
-        int rc = ws->init();
+        use.emplace(ws, st);
+        int rc = use->begin();
         if (rc) return rc;
         g.kchunk = kchunk;
         g.part = ws->part;
@@ -466,10 +531,11 @@ static int gemm(GemmWs* ws, int transA, int transB, int M, int N, int K, float a
     int kchunk = (K + splits - 1) / splits;
     kchunk = (kchunk + kGK - 1) / kGK * kGK;
     splits = (K + kchunk - 1) / kchunk;
-    int rc = ws->init();
-    if (rc) return rc;
     if (static_cast<size_t>(splits) * M * N > kGemmPartFloats)
       return fail(DGFS_ERR_INVALID_VALUE, "split-K workspace too small");
+    GemmWsUse use(ws, st);
+    int rc = use.begin();
+    if (rc) return rc;
     g.kchunk = kchunk;
     g.part = ws->part;
     if (bf16)
@@ -1725,10 +1791,9 @@ extern "C" int dgfs_nn_gemm(int transA, int transB, int M, int N, int K, float a
   if (lda < (transA ? M : K) || ldb < (transB ? K : N) || ldc < N)
     return fail(DGFS_ERR_INVALID_VALUE, "leading dimension too small");
   if ((M + kGT - 1) / kGT > 65535) return fail(DGFS_ERR_INVALID_VALUE, "M = %d exceeds the grid (65535 row tiles)", M);
-  // process-lifetime workspace (released by the driver at exit)
-  static GemmWs* ws = new GemmWs();
-  return gemm(ws, transA ? 1 : 0, transB ? 1 : 0, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, bf16 != 0,
-              static_cast<hipStream_t>(stream));
+  auto st = static_cast<hipStream_t>(stream);
+  return gemm(shared_gemm_ws(st), transA ? 1 : 0, transB ? 1 : 0, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc,
+              bf16 != 0, st);
 }
 
 extern "C" int dgfs_sur_create(const dgfs_sur_desc* d, void** out) {

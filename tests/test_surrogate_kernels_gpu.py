@@ -118,3 +118,90 @@ def test_encode_decode_grids(N, device):
         sc = np.abs(q0).max()
         assert np.abs(Q0.cpu().numpy()[i] - q0).max() < tol * sc
         assert np.abs(Q.cpu().numpy()[i] - S.project(q0, N, L)).max() < tol * sc
+
+
+def _stream_products(n, device, seed):
+    """n products of the split form (512 x 512, K split in two; 64 x 64 from a
+    long K through the general kernel) on each of two streams."""
+    import torch
+    g = torch.Generator(device="cpu").manual_seed(seed)
+    shapes = [(512, 512, 512), (64, 60, 9001), (512, 512, 1500)]
+    jobs = []
+    for s in range(2):
+        ops = []
+        for i in range(n):
+            M, N, K = shapes[(i + s) % 3]
+            ops.append((M, N, K, torch.randn((M, K), generator=g).to(device), torch.randn((K, N), generator=g).to(device),
+                        torch.full((M, N), float("nan"), device=device)))
+        jobs.append(ops)
+    return jobs
+
+
+def _launch(ops, stream):
+    from dgfs_hip import surrogate as D
+    for M, N, K, A, B, Cm in ops:
+        D.gemm(0, 0, M, N, K, 1.0, A, K, B, N, 0.0, Cm, N, bf16=False, stream=stream.cuda_stream)
+
+
+@pytest.mark.parametrize("threads", [False, True])
+def test_split_products_on_two_streams(threads, device):
+    """Products whose reduction is split, on two streams at once (from one
+    thread in turn, and from two threads): each equals, bitwise, the same
+    product with nothing else in flight, whose order of sums is the same."""
+    import threading
+    import torch
+    jobs = _stream_products(12, device, 11)
+    print("split products on two streams", threads, flush=True)
+    quiet = torch.cuda.Stream()
+    want = []
+    for ops in jobs:
+        _launch(ops, quiet)
+        torch.cuda.synchronize()
+        want.append([o[-1].clone() for o in ops])
+    for ops in jobs:
+        for o in ops:
+            o[-1].fill_(float("nan"))
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    if threads:
+        ts = [threading.Thread(target=_launch, args=(ops, s)) for ops, s in zip(jobs, streams)]
+        for t in ts:
+            t.start()
+        for t in ts:
+            t.join()
+    else:
+        for a, b in zip(*jobs):
+            _launch([a], streams[0])
+            _launch([b], streams[1])
+    torch.cuda.synchronize()
+    for ops, ws in zip(jobs, want):
+        for o, w in zip(ops, ws):
+            assert torch.equal(o[-1], w)
+
+
+def test_captured_product_takes_no_shared_workspace(device):
+    """Under capture the product runs unsplit: replays with eager split
+    products on another stream in between stay equal to the first one, and to
+    the eager product within the order of the sums (bound of the module)."""
+    import torch
+    (job, other) = _stream_products(3, device, 5)
+    M, N, K, A, B, Cm = job[0]
+    s = torch.cuda.Stream()
+    _launch([job[0]], s)
+    torch.cuda.synchronize()
+    eager = Cm.clone()
+    g = torch.cuda.CUDAGraph()
+    print("captured product", flush=True)
+    with torch.cuda.graph(g):
+        _launch([job[0]], torch.cuda.current_stream())
+    first = None
+    for _ in range(4):
+        Cm.fill_(float("nan"))
+        torch.cuda.synchronize()
+        _launch(other, s)
+        g.replay()
+        torch.cuda.synchronize()
+        first = Cm.clone() if first is None else first
+        assert torch.equal(Cm, first)
+    bound = 8 * np.sqrt(K) * 2.0 ** -22 * float(A.abs().max()) * float(B.abs().max())
+    assert float((first - eager).abs().max()) <= bound
