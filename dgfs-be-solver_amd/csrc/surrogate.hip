@@ -378,6 +378,7 @@ __global__ __launch_bounds__(256) void k_gemm_reduce(const float* __restrict__ p
 // need at most 16 M floats.  Allocated once at that size and never resized
 // while work may be in flight; a split that would not fit runs unsplit.
 constexpr size_t kGemmPartFloats = size_t{1} << 24;
+constexpr int kGemmSplitK = 512;  // shortest reduction that any shape splits
 struct GemmWs {
   float* part = nullptr;
   // a workspace that calls on several streams and threads share: a product
@@ -489,7 +490,7 @@ static int gemm(GemmWs* ws, int transA, int transB, int M, int N, int K, float a
     const long tl = static_cast<long>(bx) * by, want = 2L * cu_count();
     int splits = 1;
     std::optional<GemmWsUse> use;
-    if (ws && tl < want && K >= 512) splits = static_cast<int>(std::min<long>(want / tl, K / 256));
+    if (ws && tl < want && K >= kGemmSplitK) splits = static_cast<int>(std::min<long>(want / tl, K / 256));
     if (splits > 1) {
       int kchunk = (K + splits - 1) / splits;
       kchunk = (kchunk + kFK - 1) / kFK * kFK;
@@ -1792,7 +1793,8 @@ extern "C" int dgfs_nn_gemm(int transA, int transB, int M, int N, int K, float a
     return fail(DGFS_ERR_INVALID_VALUE, "leading dimension too small");
   if ((M + kGT - 1) / kGT > 65535) return fail(DGFS_ERR_INVALID_VALUE, "M = %d exceeds the grid (65535 row tiles)", M);
   auto st = static_cast<hipStream_t>(stream);
-  return gemm(shared_gemm_ws(st), transA ? 1 : 0, transB ? 1 : 0, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc,
+  // no shape splits a reduction shorter than kGemmSplitK
+  return gemm(K >= kGemmSplitK ? shared_gemm_ws(st) : nullptr, transA ? 1 : 0, transB ? 1 : 0, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc,
               bf16 != 0, st);
 }
 
