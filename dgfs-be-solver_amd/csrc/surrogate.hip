@@ -1794,8 +1794,8 @@ extern "C" int dgfs_nn_gemm(int transA, int transB, int M, int N, int K, float a
   if ((M + kGT - 1) / kGT > 65535) return fail(DGFS_ERR_INVALID_VALUE, "M = %d exceeds the grid (65535 row tiles)", M);
   auto st = static_cast<hipStream_t>(stream);
   // no shape splits a reduction shorter than kGemmSplitK
-  return gemm(K >= kGemmSplitK ? shared_gemm_ws(st) : nullptr, transA ? 1 : 0, transB ? 1 : 0, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc,
-              bf16 != 0, st);
+  return gemm(K >= kGemmSplitK ? shared_gemm_ws(st) : nullptr, transA ? 1 : 0, transB ? 1 : 0, M, N, K, alpha, A,
+              lda, B, ldb, beta, C, ldc, bf16 != 0, st);
 }
 
 extern "C" int dgfs_sur_create(const dgfs_sur_desc* d, void** out) {
@@ -1829,6 +1829,9 @@ extern "C" int dgfs_sur_create(const dgfs_sur_desc* d, void** out) {
   DGFS_HIP_TRY(hipMalloc(&h->dU, act));
   DGFS_HIP_TRY(hipMalloc(&h->part, std::max(static_cast<size_t>(kRedBlocks) * kSurWidth,
                                             static_cast<size_t>(kLayBwdBlocks) * kLayPart) * sizeof(float)));
+  // the products of any batch may split their reduction: no call allocates later
+  rc = h->ws.init();
+  if (rc) return rc;
   *out = h.release();
   return DGFS_OK;
 }

@@ -205,3 +205,32 @@ def test_captured_product_takes_no_shared_workspace(device):
         assert torch.equal(Cm, first)
     bound = 8 * np.sqrt(K) * 2.0 ** -22 * float(A.abs().max()) * float(B.abs().max())
     assert float((first - eager).abs().max()) <= bound
+
+
+@pytest.mark.parametrize("P", [5, 130])
+def test_first_forward_and_backward_captured(P, device):
+    """A handle's first forward and backward may be under capture: nothing is
+    allocated after its creation, and every replay equals the eager result."""
+    import torch
+    from dgfs_hip.surrogate import SpectralSurrogate
+    rng = np.random.default_rng(P)
+    f32 = lambda a: torch.as_tensor(a, dtype=torch.float32, device=device).contiguous()
+    x, lt, dout = f32(rng.normal(size=(P, 512))), f32(rng.normal(size=P) * 0.2), f32(rng.normal(size=(P, 512)))
+    out = torch.empty((P, 512), dtype=torch.float32, device=device)
+    sur = SpectralSurrogate(8, 5.0, (10.0 / 8) ** 3, 0.38, 1.0, max_batch=P, device=device, seed=3)
+    torch.cuda.synchronize()
+    print("captured first forward", P, flush=True)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        sur.forward(x, lt, P, out)
+        sur.backward(dout)
+    sur.forward(x, lt, P, out)
+    sur.backward(dout)
+    torch.cuda.synchronize()
+    eager, grad = out.clone(), sur.grad.clone()
+    for _ in range(3):
+        out.zero_()
+        sur.grad.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager) and torch.equal(sur.grad, grad)
