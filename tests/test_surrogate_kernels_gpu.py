@@ -234,3 +234,34 @@ def test_first_forward_and_backward_captured(P, device):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, eager) and torch.equal(sur.grad, grad)
+
+
+@pytest.mark.parametrize("P", [3, 130])
+def test_layer_sums_of_its_two_products_apart(P, device):
+    """A layer adds U W and Z R as whole sums: with U W = 2^24 everywhere and
+    Z R = 2 from 32 products of 1/16, the result is 2^24 + 2 exactly, where a
+    chain that added the small products to the large sum one after another
+    would lose every one of them.  The other layers pass it on (K = W = 0, R
+    the identity; GELU is the identity at this size)."""
+    import torch
+    from dgfs_hip.surrogate import SpectralSurrogate
+    th = np.zeros_like(S.init_params(0))
+    D, Wd = S.MODES, S.WIDTH
+    th[S.OFF_E:S.OFF_E + D * Wd] = 1.0
+    for l in range(S.LAYERS):
+        o = S.OFF_LAYERS + l * S.LAYER_SIZE
+        K, W, R = (th[a:a + n] for a, n in ((o, D * D), (o + D * D, Wd * Wd), (o + D * D + Wd * Wd, Wd * Wd)))
+        if l == 0:
+            K[:] = np.eye(D).ravel()
+            W[:] = 2.0 ** 19
+            R[:] = 2.0 ** -4
+        else:
+            R[:] = np.eye(Wd).ravel()
+    th[S.OFF_POUT] = 1.0
+    sur = SpectralSurrogate(8, 5.0, (10.0 / 8) ** 3, 0.38, 1.0, max_batch=P, device=device, seed=0)
+    f32 = lambda a: torch.as_tensor(a, dtype=torch.float32, device=device).contiguous()
+    out = torch.empty((P, D), dtype=torch.float32, device=device)
+    print("layer sums", P, flush=True)
+    sur.forward(f32(np.zeros((P, D))), f32(np.zeros(P)), P, out, params=f32(th))
+    torch.cuda.synchronize()
+    assert (out == 2.0 ** 24 + 2.0).all()
