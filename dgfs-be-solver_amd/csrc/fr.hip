@@ -391,12 +391,12 @@ __global__ __launch_bounds__(kBcPts * kBcRows) void k_bccflux(BcArgs a) {
 // bc1 += sum_{fac<0} fac f0 cw; reset when vidx == 0.  With st set (the
 // cylinder wall, dgfs-wall-diffuse-cyl-update.mako:12-44) U and T are
 // per point and f0 is the unnormalised Maxwellian.  One block per wall
-// point, kUpdUnroll velocities of every thread in flight (each is a cache line
-// of its own in the AoSoA register, so the loads are latency), a tree
-// reduction over the velocity index.  36 points at 24^3: 56 -> 27 us on MI355X
-// against 256 threads with one load at a time.
-constexpr int kUpdThreads = 1024, kUpdUnroll = 4;
-__global__ __launch_bounds__(kUpdThreads) void k_bccupdate_diffuse(int ndims, int nfpts, int nvars, int vidx,
+// point, a tree reduction over the velocity index.  Every value of ul is a
+// cache line of its own in the AoSoA register, so a point's time is the
+// latency of its threads' loads one after another; the block is wide where
+// that counts (update_threads).
+template <int NTH>
+__global__ __launch_bounds__(NTH) void k_bccupdate_diffuse(int ndims, int nfpts, int nvars, int vidx,
                                                            const double* __restrict__ L,
                                                            const long* __restrict__ loff,
                                                            const double* __restrict__ nl,
@@ -405,7 +405,7 @@ __global__ __launch_bounds__(kUpdThreads) void k_bccupdate_diffuse(int ndims, in
                                                            double Uy, double Uz, double cw,
                                                            const double* __restrict__ cv, int vsize,
                                                            const double* __restrict__ st) {
-  __shared__ double r0[kUpdThreads], r1[kUpdThreads];
+  __shared__ double r0[NTH], r1[NTH];
   const int i = blockIdx.x, tid = threadIdx.x;
   const long ol = loff[i];
   double n[3] = {0, 0, 0};
@@ -416,29 +416,20 @@ __global__ __launch_bounds__(kUpdThreads) void k_bccupdate_diffuse(int ndims, in
     Tw = st[3L * nfpts + i];
   }
   double s0 = 0.0, s1 = 0.0;
-  for (int v0 = tid; v0 < nvars; v0 += kUpdThreads * kUpdUnroll) {
-    double fac[kUpdUnroll], x[kUpdUnroll];
-#pragma unroll
-    for (int k = 0; k < kUpdUnroll; ++k) {
-      const int v = v0 + k * kUpdThreads, vv = vidx + min(v, nvars - 1);
-      fac[k] = 0.0;
-      for (int d = 0; d < ndims; ++d) fac[k] += (cv[d * static_cast<long>(vsize) + vv] - U[d]) * n[d];
-      x[k] = 0.0;
-      if (v < nvars) {
-        if (fac[k] >= 0) x[k] = L[ol + 32L * v];
-        else x[k] = st ? cyl_wall_f(cv, vsize, vv, U, Tw) : f0[vv];
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < kUpdUnroll; ++k) {
-      if (fac[k] >= 0) s0 += fac[k] * x[k] * cw;
-      else s1 += fac[k] * x[k] * cw;
-    }
+  for (int v = tid; v < nvars; v += NTH) {
+    const int vv = vidx + v;
+    double fac = 0.0;
+    for (int d = 0; d < ndims; ++d) fac += (cv[d * static_cast<long>(vsize) + vv] - U[d]) * n[d];
+    // the value first, the sums after (36 points at 24^3: 17.9 us; 20.8 with
+    // load and sum in one branch)
+    const double x = fac >= 0 ? L[ol + 32L * v] : st ? cyl_wall_f(cv, vsize, vv, U, Tw) : f0[vv];
+    if (fac >= 0) s0 += fac * x * cw;
+    else s1 += fac * x * cw;
   }
   r0[tid] = s0;
   r1[tid] = s1;
   __syncthreads();
-  for (int s = kUpdThreads / 2; s > 0; s >>= 1) {
+  for (int s = NTH / 2; s > 0; s >>= 1) {
     if (tid < s) {
       r0[tid] += r0[tid + s];
       r1[tid] += r1[tid + s];
@@ -766,6 +757,14 @@ extern "C" int dgfs_bccflux(int bctype, int ndims, int nfpts, int nvars, int vid
   return DGFS_OK;
 }
 
+// threads per wall point of the balance: 1024 while each has a velocity and the
+// points are few enough that a point's latency shows (36 points at 24^3: 48 ->
+// 18 us on MI355X against 256 threads, 1024 points 95 us either way, 4096
+// points 368 -> 357 us); with many points the narrow block's shorter reduction
+// wins (20000 points of 64 velocities 29 against 104 us, 200000 of 512 0.64
+// against 1.39 ms), and its grid takes four times as many points.
+static int update_threads(int nfpts, int nvars) { return nvars >= 1024 && nfpts <= 4096 ? 1024 : 256; }
+
 extern "C" int dgfs_bccupdate(int bctype, int ndims, int nfpts, int nvars, int vidx, const double* L,
                               const long* loff, const double* nl, const double* f0, double* bcvals,
                               double Ux, double Uy, double Uz, double cw, const double* cv, int vsize,
@@ -777,8 +776,14 @@ extern "C" int dgfs_bccupdate(int bctype, int ndims, int nfpts, int nvars, int v
   if (bctype == BC_DIFFUSE || bctype == BC_DIFFUSE_CYL) {
     if (!f0) return fail(DGFS_ERR_INVALID_VALUE, "dgfs_bccupdate: diffuse wall needs f0");
     const bool cyl = bctype == BC_DIFFUSE_CYL;
-    hipLaunchKernelGGL(k_bccupdate_diffuse, dim3(nfpts), dim3(kUpdThreads), 0, st, ndims, nfpts, nvars, vidx, L, loff,
-                       nl, cyl ? nullptr : f0, bcvals, Ux, Uy, Uz, cw, cv, vsize, cyl ? f0 : nullptr);
+#define DGFS_UPD(NTH)                                                                                              \
+  hipLaunchKernelGGL(k_bccupdate_diffuse<NTH>, dim3(nfpts), dim3(NTH), 0, st, ndims, nfpts, nvars, vidx, L, loff, nl, \
+                     cyl ? nullptr : f0, bcvals, Ux, Uy, Uz, cw, cv, vsize, cyl ? f0 : nullptr)
+    if (update_threads(nfpts, nvars) == 1024)
+      DGFS_UPD(1024);
+    else
+      DGFS_UPD(256);
+#undef DGFS_UPD
   } else if (bctype == BC_SPECULAR) {
     hipLaunchKernelGGL(k_bccupdate_specular, dim3((nfpts + 255) / 256, nvars), dim3(256), 0, st, nfpts, nvars,
                        vidx, L, loff, bcvals);

@@ -48,3 +48,36 @@ def test_diffuse_wall_edges(nf, nvars, vidx, vsize, device):
     ref = L.copy()
     ref[off[:, None] + 32 * np.arange(nvars)[None]] = fn
     assert np.abs(out - ref).max() < 1e-13 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("nf,nvars", [(4096, 1024), (4097, 1024), (4096, 1023), ((1 << 22) + 3, 2)])
+def test_diffuse_balance_of_many_points(nf, nvars, device):
+    """Both sides of the limits of the wide block (1024 velocities, 4096
+    points), and more points than a grid of 1024-thread blocks takes (2^32
+    threads): every point against the same sums in torch, FP64 sums of up to
+    1024 terms, so 1e-13 of the largest value."""
+    import torch
+    from dgfs_hip import fr
+    g = torch.Generator(device=device).manual_seed(nf)
+    r = lambda *s: torch.rand(s, dtype=torch.float64, device=device, generator=g)
+    rows = min(nf, 4097)  # the points share these rows of states
+    L = r(-(-rows // 32) * nvars * 32)
+    i = torch.arange(nf, device=device) % rows
+    off = (i // 32) * nvars * 32 + i % 32
+    ang = 6.283 * r(nf)
+    nl = torch.stack([torch.cos(ang), torch.sin(ang)]).contiguous()
+    cv = 10 * r(3, nvars) - 5
+    f0 = r(nvars)
+    bc = torch.full((2, nf), float("nan"), dtype=torch.float64, device=device)
+    U, cw = (0.3, -0.1, 0.0), 0.7
+    print("wall balance", nf, nvars, flush=True)
+    fr.bccupdate(fr.BC_DIFFUSE, 2, nf, nvars, 0, L, off, nl, f0, bc, U, cw, cv, nvars,
+                 torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    b0, b1 = torch.zeros(nf, dtype=torch.float64, device=device), torch.zeros(nf, dtype=torch.float64, device=device)
+    for v in range(nvars):
+        fac = nl[0] * (cv[0, v] - U[0]) + nl[1] * (cv[1, v] - U[1])
+        b0 += torch.where(fac >= 0, fac * L[off + 32 * v] * cw, 0.0)
+        b1 += torch.where(fac < 0, fac * f0[v] * cw, 0.0)
+    assert float((bc[0] - b0).abs().max()) < 1e-13 * float(b0.abs().max())
+    assert float((bc[1] - b1).abs().max()) < 1e-13 * float(b1.abs().max())
