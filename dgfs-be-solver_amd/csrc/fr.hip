@@ -330,7 +330,7 @@ struct BcArgs {
 // workgroup takes kBcPts boundary points (consecutive ones are neighbouring
 // elements of an AoSoA block) by kBcRows rows of vchunk velocities: a boundary
 // has few points and many velocities, and one thread per point with 64
-// velocities each left most of the chip idle (36 points at 24^3: 47 -> 15 us on
+// velocities each left most of the chip idle (36 points at 24^3: 31 -> 7.5 us on
 // MI355X).
 constexpr int kBcPts = 32, kBcRows = 8;
 
@@ -745,13 +745,18 @@ extern "C" int dgfs_bccflux(int bctype, int ndims, int nfpts, int nvars, int vid
   BcArgs a;
   a.bctype = bctype; a.ndims = ndims; a.nfpts = nfpts; a.nvars = nvars; a.vidx = vidx;
   a.vsize = vsize;
-  // 4 velocities per thread, more where the grid's second dimension (65535)
-  // or an already full chip asks for it
+  // 4 velocities per thread (36 points at 24^3: 7.6 us, 38 with 64 each), twice
+  // as many again, up to 64, while there are more than 64 workgroups per CU,
+  // whose turnover then costs more than it hides (20000 points of 4096
+  // velocities 653 -> 596 us, 4096 points at 24^3 440 -> 418 us), or while the
+  // grid's second dimension would exceed 65535
+  const long bx = (nfpts + kBcPts - 1) / kBcPts, most = 64L * cu_count();
+  auto rows = [&](int c) -> long { return (static_cast<long>(nvars) + c * kBcRows - 1) / (c * kBcRows); };
   a.vchunk = 4;
-  while ((nvars + a.vchunk * kBcRows - 1) / (a.vchunk * kBcRows) > 16384) a.vchunk *= 2;
+  while ((a.vchunk < 64 && bx * rows(a.vchunk) > most) || rows(a.vchunk) > 65535) a.vchunk *= 2;
   a.L = L; a.loff = loff; a.nl = nl; a.magnl = magnl; a.f0 = f0; a.bcvals = bcvals; a.rmap = rmap; a.cv = cv;
   a.U[0] = Ux; a.U[1] = Uy; a.U[2] = Uz;
-  dim3 grid((nfpts + kBcPts - 1) / kBcPts, (nvars + a.vchunk * kBcRows - 1) / (a.vchunk * kBcRows));
+  dim3 grid(static_cast<unsigned>(bx), static_cast<unsigned>(rows(a.vchunk)));
   hipLaunchKernelGGL(k_bccflux, grid, dim3(kBcPts * kBcRows), 0, static_cast<hipStream_t>(stream), a);
   DGFS_LAUNCH_CHECK("dgfs_bccflux");
   return DGFS_OK;

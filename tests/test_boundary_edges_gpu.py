@@ -81,3 +81,37 @@ def test_diffuse_balance_of_many_points(nf, nvars, device):
         b1 += torch.where(fac < 0, fac * f0[v] * cw, 0.0)
     assert float((bc[0] - b0).abs().max()) < 1e-13 * float(b0.abs().max())
     assert float((bc[1] - b1).abs().max()) < 1e-13 * float(b1.abs().max())
+
+
+@pytest.mark.parametrize("nf", [32 * 511, 32 * 513, 32 * 4097 - 5])
+def test_flux_of_many_points(nf, device):
+    """Point counts on both sides of where a thread takes more than 4
+    velocities (64 workgroups per CU: 512 groups of 32 points at 1024
+    velocities on 256 CUs) and where it takes 32, a ragged last row: a wall
+    that lets through, ul = 0.5 n.c (ul + ur) + 0.5 |n.c| (ul - ur)."""
+    import torch
+    from dgfs_hip import fr
+    nvars = 1021
+    g = torch.Generator(device=device).manual_seed(nf)
+    r = lambda *s: torch.rand(s, dtype=torch.float64, device=device, generator=g)
+    L = r(-(-nf // 32) * nvars * 32)
+    i = torch.arange(nf, device=device)
+    off = (i // 32) * nvars * 32 + i % 32
+    ang = 6.283 * r(nf)
+    nl, mag = torch.stack([torch.cos(ang), torch.sin(ang)]).contiguous(), 0.5 + r(nf)
+    cv, f0 = 10 * r(3, nvars) - 5, r(nvars)
+    before = L.clone()
+    print("boundary flux", nf, flush=True)
+    fr.bccflux(fr.BC_INLET, 2, nf, nvars, 0, L, off, nl, mag, f0, None, None, (0.3, -0.1, 0.0), cv, nvars,
+               torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    worst = 0.0
+    for v in range(nvars):
+        ul = before[off + 32 * v]
+        nc = nl[0] * cv[0, v] + nl[1] * cv[1, v]
+        fac = nl[0] * (cv[0, v] - 0.3) + nl[1] * (cv[1, v] + 0.1)
+        # at fac = 0 up to rounding either side is the state: leave those points out
+        ur = torch.where(fac < 0, f0[v], ul)
+        want = mag * (0.5 * nc * (ul + ur) + 0.5 * nc.abs() * (ul - ur))
+        worst = max(worst, float(((L[off + 32 * v] - want) * (fac.abs() > 1e-12)).abs().max()))
+    assert worst < 1e-13 * float(L.abs().max())
