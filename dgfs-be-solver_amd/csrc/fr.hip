@@ -499,20 +499,18 @@ __global__ __launch_bounds__(256) void k_copy_reg(int nblocks, int count, const 
 // p = rho T.  out[upt][m][e] for m over the 15 outputs (3D layout).
 //
 // A workgroup takes EW neighbouring elements of one AoSoA block at one solution
-// point: a thread two of them at every (512 / (EW/2))-th velocity (so that a
-// velocity's abscissae are read once for two values), kMomUnroll velocities in
-// flight; then a sum over the threads of a wave and over the waves, always in
-// the same order.  Two passes over f, the bulk velocity first (the second
-// mostly from the last-level cache).  EW is the widest that still gives every
-// CU a workgroup: half of the time is FP64 arithmetic, which needs the whole
-// chip.  2304 points at 24^3 on MI355X: 9019 us with one thread per point,
-// 470 us with 72 workgroups of 32 elements, 205 us with 288 of 8 (floor: 56 us
-// for reading f once).
-constexpr int kMomUnroll = 4, kMomWaves = 8;
+// point: a thread two of them at every (64 WAVES / (EW/2))-th velocity (so that
+// a velocity's abscissae are read once for two values), kMomUnroll velocities
+// in flight; then a sum over the threads of a wave and over the waves, always
+// in the same order.  Two passes over f, the bulk velocity first (the second
+// mostly from the last-level cache).  Bound by the latency of the loads of f:
+// 2304 points at 24^3 take 205 us (9019 us with one thread per point), where
+// reading f once is 56 us and the FP64 sums about 22 us.
+constexpr int kMomUnroll = 4;
 
 // totals over the workgroup of NQ values of two elements per thread; red:
-// [kMomWaves][NQ][EW]
-template <int NQ, int EW>
+// [WAVES][NQ][EW]
+template <int NQ, int EW, int WAVES>
 __device__ __forceinline__ void mom_reduce(double (&s)[NQ][2], double* red) {
   constexpr int TPR = EW / 2;
   const int sub = threadIdx.x % TPR, wave = threadIdx.x >> 6;
@@ -522,6 +520,7 @@ __device__ __forceinline__ void mom_reduce(double (&s)[NQ][2], double* red) {
     for (int h = 0; h < 2; ++h)
 #pragma unroll
       for (int d = 32; d >= TPR; d >>= 1) s[j][h] += __shfl_xor(s[j][h], d);
+  if (WAVES == 1) return;
   __syncthreads();
   if ((threadIdx.x & 63) < TPR)
 #pragma unroll
@@ -535,17 +534,17 @@ __device__ __forceinline__ void mom_reduce(double (&s)[NQ][2], double* red) {
     for (int h = 0; h < 2; ++h) {
       double t = 0.0;
 #pragma unroll 1
-      for (int w = 0; w < kMomWaves; ++w) t += red[(w * NQ + j) * EW + 2 * sub + h];
+      for (int w = 0; w < WAVES; ++w) t += red[(w * NQ + j) * EW + 2 * sub + h];
       s[j][h] = t;
     }
 }
 
-template <int EW>
-__global__ __launch_bounds__(64 * kMomWaves) void k_moments(int neles, int vsize, const double* __restrict__ f,
-                                                            long ld, const double* __restrict__ cv, double cw,
-                                                            double* __restrict__ out) {
-  constexpr int TPR = EW / 2, ROWS = 64 * kMomWaves / TPR, NB = 32 / EW;
-  __shared__ double red[kMomWaves * 10 * EW];
+template <int EW, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void k_moments(int neles, int vsize, const double* __restrict__ f, long ld,
+                                                        const double* __restrict__ cv, double cw,
+                                                        double* __restrict__ out) {
+  constexpr int TPR = EW / 2, ROWS = 64 * WAVES / TPR, NB = 32 / EW;
+  __shared__ double red[WAVES * 10 * EW];
   const int sub = threadIdx.x % TPR, row = threadIdx.x / TPR, upt = blockIdx.y;
   const int eb = blockIdx.x / NB, l0 = (blockIdx.x % NB) * EW + 2 * sub;
   const long e = static_cast<long>(eb) * 32 + l0;
@@ -572,7 +571,7 @@ __global__ __launch_bounds__(64 * kMomWaves) void k_moments(int neles, int vsize
         m[3][h] += x[k][h] * c[k][2];
       }
   }
-  mom_reduce<4, EW>(m, red);
+  mom_reduce<4, EW, WAVES>(m, red);
   double rho[2], u[2][3];
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
@@ -606,7 +605,7 @@ __global__ __launch_bounds__(64 * kMomWaves) void k_moments(int neles, int vsize
       }
   }
   __syncthreads();  // red is read for m above
-  mom_reduce<10, EW>(q, red);
+  mom_reduce<10, EW, WAVES>(q, red);
   if (row != 0) return;
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
@@ -842,15 +841,24 @@ extern "C" int dgfs_moments(int nupts, int neles, int vsize, const double* f, lo
   if (total == 0) return DGFS_OK;
   const long blocks = nparr / 32, cus = cu_count();
   auto st = static_cast<hipStream_t>(stream);
-#define DGFS_MOM(EW)                                                                                            \
-  hipLaunchKernelGGL(k_moments<EW>, dim3(static_cast<unsigned>(blocks * (32 / EW)), nupts), dim3(64 * kMomWaves), \
+#define DGFS_MOM(EW, WAVES)                                                                                     \
+  hipLaunchKernelGGL((k_moments<EW, WAVES>), dim3(static_cast<unsigned>(blocks * (32 / EW)), nupts), dim3(64 * WAVES), \
                      0, st, neles, vsize, f, ld, cv, cw, out)
-  if (blocks * nupts >= cus)
-    DGFS_MOM(32);
+  // the widest EW that still gives every CU a workgroup (24^3, us at EW 8 / 16 /
+  // 32: 45 blocks 95 / 141 / 262, 135 blocks 333 / 375 / 384, 513 blocks 1034 /
+  // 1016 / 1118); few waves on short velocity grids, whose time is the
+  // reduction over the waves (one element of 64 velocities 16 -> 5 us, 3125
+  // blocks of 64 velocities 184 -> 27 us, of 216 velocities 116 -> 37 us)
+  if (vsize <= 256 && blocks * nupts < cus)
+    DGFS_MOM(8, 1);
+  else if (vsize <= 256)
+    DGFS_MOM(32, 2);
+  else if (blocks * nupts >= cus)
+    DGFS_MOM(32, 8);
   else if (2 * blocks * nupts >= cus)
-    DGFS_MOM(16);
+    DGFS_MOM(16, 8);
   else
-    DGFS_MOM(8);
+    DGFS_MOM(8, 8);
 #undef DGFS_MOM
   DGFS_LAUNCH_CHECK("dgfs_moments");
   return DGFS_OK;

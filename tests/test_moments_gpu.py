@@ -12,6 +12,10 @@ CASES = [
     # nupts, neles, vsize: the three widths are taken at >= 256, >= 128 and
     # fewer 32-element blocks (times nupts)
     (1, 1, 27), (1, 31, 64), (3, 33, 125), (9, 64, 216), (4, 32 * 33 - 1, 64), (4, 32 * 64 + 5, 27), (1, 2, 4096),
+    # short and long velocity grids (256) at every width
+    (3, 33, 256), (3, 33, 257), (4, 32 * 33 - 1, 260), (4, 32 * 64 + 5, 256), (4, 32 * 64 + 5, 300),
+    # many solution points (the grid's second dimension)
+    (65537, 1, 8),
 ]
 
 
