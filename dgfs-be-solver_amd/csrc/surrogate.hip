@@ -1153,19 +1153,26 @@ constexpr size_t enc_lds_doubles() {
 // together.  The Maxwellian is the product of the tables' order-0 columns, not
 // an exp per velocity.  Bound by reading f (2 x 8 n bytes per point) and by the
 // 8 FP64 multiply-adds per value: 1000 points at 32^3, 704 -> 253 us on MI355X.
+// MODES = false is for calls that want the moments and the indicator alone (no
+// x): the same sums without the x-modes, the basis tables and their LDS.
 constexpr int kEncThreads = 512;
 
 template <int N>
+constexpr size_t enc_moments_lds_doubles() {
+  return 3 * N * kSurD + kEncThreads / 64 * 5;
+}
+
+template <int N, bool MODES>
 __global__ __launch_bounds__(kEncThreads) void k_sur_encode(EncArgs a) {
   constexpr int n = N * N * N, NN = N * N, NT = kEncThreads;
   extern __shared__ double sm[];
   double* t1 = sm;                          // kSurD * N * N
   double* t2 = t1 + kSurD * NN;             // kSurD * kSurD * N
-  double* V = t2 + kSurD * kSurD * N;       // 3 * N * kSurD
+  double* V = MODES ? t2 + kSurD * kSurD * N : sm;  // 3 * N * kSurD
   double* Linv = V + 3 * N * kSurD;         // 3 * 64
   double* work = Linv + 3 * kSurD * kSurD;  // 3 * 64
   double* b3 = work + 3 * kSurD * kSurD;    // 512
-  double* red = b3 + kSurModes;             // 256
+  double* red = MODES ? b3 + kSurModes : V + 3 * N * kSurD;  // 256 (without the modes 40)
   const double hh = 2.0 * a.L / N, c0 = -a.L + 0.5 * hh;
   const double pi = 3.14159265358979323846;
   for (int pt = blockIdx.x; pt < a.npts; pt += gridDim.x) {
@@ -1193,9 +1200,16 @@ __global__ __launch_bounds__(kEncThreads) void k_sur_encode(EncArgs a) {
     const double T = (2.0 / 3.0) * (m[4] * a.cw / rho - (ux * ux + uy * uy + uz * uz));
     const double Mn = rho / pow(pi * T, 1.5);
     const double s = sqrt(0.5 * T), hs = hh / s;
-    herm_table(V, c0, hh, ux, s, N);
-    herm_table(V + N * kSurD, c0, hh, uy, s, N);
-    herm_table(V + 2 * N * kSurD, c0, hh, uz, s, N);
+    if constexpr (MODES) {
+      herm_table(V, c0, hh, ux, s, N);
+      herm_table(V + N * kSurD, c0, hh, uy, s, N);
+      herm_table(V + 2 * N * kSurD, c0, hh, uz, s, N);
+    } else {  // the order-0 columns
+      for (int e = threadIdx.x; e < 3 * N; e += NT) {
+        const double x = (c0 + (e % N) * hh - (e < N ? ux : e < 2 * N ? uy : uz)) / s;
+        V[e * kSurD] = exp(-0.5 * x * x) * kInvSqrtFact[0];
+      }
+    }
     __syncthreads();
     double ds[2] = {0, 0};  // sums of (f - M)^2 and f^2
     for (int jk = threadIdx.x; jk < NN; jk += NT) {
@@ -1210,10 +1224,12 @@ __global__ __launch_bounds__(kEncThreads) void k_sur_encode(EncArgs a) {
         const double d = v - My * Vi[0];
         ds[0] += d * d;
         ds[1] += v * v;
+        if constexpr (MODES) {
 #pragma unroll
-        for (int q = 0; q < kSurD; ++q) acc[q] += v * Vi[q];
+          for (int q = 0; q < kSurD; ++q) acc[q] += v * Vi[q];
+        }
       }
-      if (a.x) {
+      if constexpr (MODES) {
 #pragma unroll
         for (int q = 0; q < kSurD; ++q) t1[q * NN + jk] = acc[q];
       }
@@ -1224,7 +1240,7 @@ __global__ __launch_bounds__(kEncThreads) void k_sur_encode(EncArgs a) {
       mo[0] = rho; mo[1] = ux; mo[2] = uy; mo[3] = uz; mo[4] = T; mo[5] = sqrt(ds[0] / ds[1]); mo[6] = 0; mo[7] = 0;
       if (a.lt) a.lt[pt] = static_cast<float>(log(T));
     }
-    if (a.x) {
+    if constexpr (MODES) {
       herm_chol_inv<N>(V, hs, Linv, work);
       // f = M is the 000 basis function: its coefficient is prod_d L_d[0][0],
       // subtracted so that equilibrium maps to zero
@@ -1693,10 +1709,17 @@ static size_t dec_lds() {
 
 template <int N>
 static int launch_encode(const EncArgs& ea, hipStream_t st) {
+  const dim3 grid(std::min(ea.npts, 4 * cu_count()));
+  if (!ea.x) {
+    hipLaunchKernelGGL((k_sur_encode<N, false>), grid, dim3(kEncThreads), enc_moments_lds_doubles<N>() * sizeof(double),
+                       st, ea);
+    DGFS_LAUNCH_CHECK("sur_encode(moments)");
+    return DGFS_OK;
+  }
   const size_t lds = enc_lds<N>();
-  DGFS_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(k_sur_encode<N>),
+  DGFS_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(k_sur_encode<N, true>),
                                    hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
-  hipLaunchKernelGGL(k_sur_encode<N>, dim3(std::min(ea.npts, 4 * cu_count())), dim3(kEncThreads), lds, st, ea);
+  hipLaunchKernelGGL((k_sur_encode<N, true>), grid, dim3(kEncThreads), lds, st, ea);
   DGFS_LAUNCH_CHECK("sur_encode");
   return DGFS_OK;
 }

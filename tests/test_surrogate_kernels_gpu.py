@@ -265,3 +265,37 @@ def test_layer_sums_of_its_two_products_apart(P, device):
     sur.forward(f32(np.zeros((P, D))), f32(np.zeros(P)), P, out, params=f32(th))
     torch.cuda.synchronize()
     assert (out == 2.0 ** 24 + 2.0).all()
+
+
+@pytest.mark.parametrize("N", [8, 12, 16, 24, 32])
+@pytest.mark.parametrize("P", [1, 1030])
+def test_encode_without_modes(N, P, device):
+    """Moments and indicator alone (no x), one point and more points than a
+    sweep of workgroups, for drifting two-stream states: bitwise those of the
+    call that encodes the modes too, and those of the FP64 oracle (1e-10)."""
+    import torch
+    from dgfs_hip.surrogate import SpectralSurrogate
+    L = 6.0 if N >= 16 else 5.0
+    rng = np.random.default_rng(N)
+    c = S.grid(N, L)
+    I, J, K = np.meshgrid(c, c, c, indexing="ij")
+    base = []
+    for _ in range(3):
+        f = 0.0
+        for w in (0.7, 0.3):
+            u, T = rng.uniform(-0.5, 0.5, 3), rng.uniform(0.9, 1.6)
+            f = f + w * np.exp(-((I - u[0]) ** 2 + (J - u[1]) ** 2 + (K - u[2]) ** 2) / T) / (np.pi * T) ** 1.5
+        base.append(f.ravel())
+    ft = torch.as_tensor(np.array(base), device=device)[torch.arange(P, device=device) % 3].contiguous()
+    sur = SpectralSurrogate(N, L, (2 * L / N) ** 3, 0.38, 1.0, max_batch=8, device=device, seed=1)
+    mom, alone = (torch.full((P, 8), float("nan"), dtype=torch.float64, device=device) for _ in range(2))
+    x = torch.empty((P, 512), dtype=torch.float32, device=device)
+    lt, lt1 = (torch.full((P,), float("nan"), dtype=torch.float32, device=device) for _ in range(2))
+    print("moments alone", N, P, flush=True)
+    sur.encode(ft, P, mom, x, lt)
+    sur.encode(ft, P, alone, None, lt1)
+    torch.cuda.synchronize()
+    assert torch.equal(mom[:, :6], alone[:, :6]) and torch.equal(lt, lt1)
+    assert not alone[:, 6:].any()
+    for i in range(min(P, 3)):
+        assert np.abs(alone[i, :6].cpu().numpy() - S.encode(base[i], N, L)[0][:6]).max() < 1e-10
