@@ -954,7 +954,7 @@ def main():
     ev_ms = e0.elapsed_time(e1)
     tim = op32.get_timing()
     cfg = op32.get_config()
-    algo = op32.get_algorithm()
+    algo, planar = op32.get_algorithm(), op32.ran_planar()
     op32.set_timing(False)
     ms_per_step = 1e3 * wall / args.steps
     value = P * args.steps / wall
@@ -974,7 +974,6 @@ def main():
     gain_ms, gain_n = tim["gain"]
     launch_s = gain_ms / max(gain_n, 1) / 1e3
     pts_per_launch = P * args.steps / max(gain_n, 1)
-    planar = bool(op32.planar) and not args.algorithm
     # planar-direction gain: per (p, pair of mirrored directions) 3 N lines' worth
     # of moves on each of N planes, N^2 operations a line; the other kernels:
     # their transforms
@@ -1076,7 +1075,7 @@ def main():
         torch.cuda.synchronize()
         w64 = time.perf_counter() - t0
         v64 = P * args.fp64_steps / w64
-        alg64, planar64 = op64.get_algorithm(), bool(op64.planar)
+        alg64, planar64 = op64.get_algorithm(), op64.ran_planar()
         Q64 = from_aosoa(reg_q64, nupts, neles, vm.vsize()).contiguous()
         # the multi-pass FP64 kernel the slab kernel replaced, one timed eval
         # (Q bitwise unused: the default's Q64 is the reference below)

@@ -1862,6 +1862,7 @@ struct VhsHandle {
                          // from k_vhs_nyq), 5 as 2 with wave-local in-plane transposes,
                          // 6 slab kernel (x-slabs in LDS, any precision, Nv 16/24/32)
   int last_algorithm = 0;
+  int last_planar = 0;   // the last evaluation ran the planar-direction gain
   void* Wny = nullptr;   // Nyquist planes [cap_pts][K][3][N][N]
   void* Ft = nullptr;    // spectrum transposed to [kx][kz][ky] [cap_pts][n]
   size_t cap_ft = 0;
@@ -2431,6 +2432,7 @@ static int run_planar(VhsHandle* h, const double* fc, double* Qc, int npts, hipS
     rc = stage_prep<T, N>(h, fc, npts, 1, slots, true, &ga, st, false);
     if (rc) return rc;
     h->last_algorithm = rr_kind(h);
+    h->last_planar = 1;
     h->last_groups = groups;
     {
       PlanarPrepArgs<T> pa{fc, static_cast<T*>(h->plop), npts};
@@ -2501,6 +2503,7 @@ static int run_planar(VhsHandle* h, const double* fc, double* Qc, int npts, hipS
 template <typename T, int N>
 static int run_chunk(VhsHandle* h, const double* fc, double* Qc, int npts, hipStream_t st) {
   if (use_planar(h)) return run_planar<T, N>(h, fc, Qc, npts, st);
+  h->last_planar = 0;
   const bool rr = use_rr(h);
   int slots = rr ? cu_count() : h->cap_slots;
   if (!rr && h->slots_override > 0) slots = std::min(slots, h->slots_override);
@@ -2939,6 +2942,7 @@ static int run_pair(VhsHandle* ha, const double* fa, double* Qa, int na, VhsHand
   if (!rc) rc = stage_prep<T, NB>(hb, fb, nb, gB, slots, false, &gb, st);
   if (rc) return rc;
   ha->last_algorithm = hb->last_algorithm = 1;
+  ha->last_planar = hb->last_planar = 0;
   {
     KTimerT<VhsHandle> t1(ha, 1, st);
     hipLaunchKernelGGL((k_vhs_gain_pair<T, NA, NB>), dim3(std::min(ga.nitems + gb.nitems, slots)),
@@ -3253,6 +3257,15 @@ extern "C" int dgfs_vhs_get_algorithm(void* p, int* algorithm) {
   if (!h) return fail(DGFS_ERR_NOT_INITIALIZED, "invalid VHS handle");
   if (!algorithm) return fail(DGFS_ERR_INVALID_VALUE, "null output");
   *algorithm = h->last_algorithm;
+  return DGFS_OK;
+}
+
+extern "C" int dgfs_vhs_get_planar(void* p, int* automatic, int* last) {
+  VhsHandle* h = as_handle(p);
+  if (!h) return fail(DGFS_ERR_NOT_INITIALIZED, "invalid VHS handle");
+  if (!automatic || !last) return fail(DGFS_ERR_INVALID_VALUE, "null output");
+  *automatic = h->planar;
+  *last = h->last_planar;
   return DGFS_OK;
 }
 

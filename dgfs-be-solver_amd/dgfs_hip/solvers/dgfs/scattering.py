@@ -64,9 +64,9 @@ class VHSOperator:
         self._h = h
         self.Nv, self.vsize, self.precision, self.project = Nv, Nv ** 3, precision, project
         self.Nrho, self.M, self.K = Nrho, M, Nrho * M
-        # whether the automatic choice may take the planar-direction gain, which
-        # no algorithm number names (the autotuner then tries it as well)
-        self.planar = Nv in (16, 24, 32) and bool(np.all((self._sz == 0.0).sum(axis=1) == 1))
+        # whether the automatic choice takes the planar-direction gain, which no
+        # algorithm number names (the autotuner then tries it as well)
+        self.planar = self._get_planar()[0]
 
     @classmethod
     def from_mesh(cls, vm, gamma, prefac, precision=64, project=False):
@@ -114,7 +114,8 @@ class VHSOperator:
         return {"ngroups": g.value, "nslots": s.value, "threads": t.value}
 
     def set_algorithm(self, algorithm):
-        """0 automatic, 1 multi-pass, 2 register-resident (FP32, Nv 16/32),
+        """0 automatic (the planar-direction gain where ``planar`` is set, which
+        has no number of its own), 1 multi-pass, 2 register-resident (FP32, Nv 16/32),
         3 register-resident with in-kernel Nyquist planes, 4 register-resident
         with one pencil per thread (FP32, Nv 16/24), 5 as 2 with wave-local
         in-plane transposes, 6 slab kernel (x-slabs of the field in LDS, FP64
@@ -122,9 +123,20 @@ class VHSOperator:
         _lib.call("dgfs_vhs_set_algorithm", self._h, int(algorithm))
 
     def get_algorithm(self):
+        """The algorithm of the last evaluation, or the one that the
+        planar-direction gain stood in for (``ran_planar``)."""
         a = C.c_int()
         _lib.call("dgfs_vhs_get_algorithm", self._h, C.byref(a))
         return a.value
+
+    def _get_planar(self):
+        auto, last = C.c_int(), C.c_int()
+        _lib.call("dgfs_vhs_get_planar", self._h, C.byref(auto), C.byref(last))
+        return bool(auto.value), bool(last.value)
+
+    def ran_planar(self):
+        """Whether the last evaluation ran the planar-direction gain."""
+        return self._get_planar()[1]
 
     def set_timing(self, on=True):
         _lib.call("dgfs_vhs_set_timing", self._h, int(bool(on)))

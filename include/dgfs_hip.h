@@ -138,10 +138,13 @@ int dgfs_vhs_set_slots(void* handle, int nslots);
  * every direction of the design has exactly one zero component and comes with
  * its mirror image (the 24-point design, M = 12); it is not selectable by
  * number.  get_algorithm reports the kernel the last eval ran, or the one the
- * planar-direction gain stood in for.
+ * planar-direction gain stood in for; get_planar tells the two apart:
+ * *automatic is 1 if algorithm 0 of this handle runs the planar-direction gain,
+ * *last is 1 if the last eval ran it.
  * No reference counterpart (the reference has one cuFFT dataflow). */
 int dgfs_vhs_set_algorithm(void* handle, int algorithm);
 int dgfs_vhs_get_algorithm(void* handle, int* algorithm);
+int dgfs_vhs_get_planar(void* handle, int* automatic, int* last);
 
 /* Kernel timing with HIP events recorded on the launch stream around every
  * launch (no added synchronisation).  set_timing(on) also clears the totals;

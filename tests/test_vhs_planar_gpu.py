@@ -124,6 +124,31 @@ def test_other_designs_keep_the_general_gain(device):
         assert np.array_equal(auto, named)
 
 
+def test_operator_tells_which_gain_ran(device):
+    """`planar` is the library's own rule (mirror images included), and
+    ran_planar tells the planar gain from the kernel that it stands in for."""
+    N = 16
+    f = np.random.default_rng(3).uniform(0.0, 1.0, size=(2, N ** 3))
+    say("which gain ran")
+    for precision, general in ((64, 6), (32, 4)):
+        op = make(N, designs()["m12"], precision)
+        assert op.planar and not op.ran_planar()
+        run(op, f, device)
+        assert op.ran_planar() and op.get_algorithm() == general
+        for algorithm in (general, 1):
+            op.set_algorithm(algorithm)
+            run(op, f, device)
+            assert op.planar and not op.ran_planar() and op.get_algorithm() == algorithm
+        op.set_algorithm(0)
+        run(op, f, device)
+        assert op.ran_planar()
+        # each direction has one zero component, but one lacks its mirror image
+        op = make(N, designs()["m12"][:11], precision)
+        run(op, f, device)
+        assert not op.planar and not op.ran_planar() and op.get_algorithm() == general
+    assert not make(12, designs()["m12"], 64).planar
+
+
 @pytest.mark.parametrize("N,npts", [(16, 400), (24, 60)])
 def test_small_batch_captured_after_a_larger_one(N, npts, device):
     """A batch small enough to split its groups over work items finds room for
