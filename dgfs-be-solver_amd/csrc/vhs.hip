@@ -2662,6 +2662,30 @@ static bool planar_groups(const double* sz, int M, std::vector<PlanarGroup>* gro
          shifts->size() <= static_cast<size_t>(kPlanarMaxShifts);
 }
 
+// Whether the planar-direction gain pays for its operand form and its transforms
+// T, whose cost does not depend on the design.  With six groups (the 12-point
+// design) it is ahead of the general kernels from one radial node and one point
+// on: 1.04 to 2.4 times as fast over Nrho 1 to 8 and 1 to 1500 points.  With
+// fewer groups it depends on the work of all nodes; the slowest batch against
+// the general kernel on MI355X, over designs of 1, 2 and 3 groups, on either
+// side of the lines below:
+//   16^3  FP64 0.91 / 1.02   FP32 0.80 / 1.03
+//   24^3  FP64 0.86 / 0.98   FP32 0.68 / 0.99
+//   32^3  FP64 0.94 / 0.98   FP32 0.90 / 1.02
+// Large batches alone would move the lines down (two groups at 24^3 FP64 0.93
+// at one point, 1.8 at 300), but the choice is the handle's and not the
+// batch's: a small batch then finds the workspace of a larger one.
+static bool planar_pays(int N, int prec, int groups, int Nrho) {
+  if (groups >= 6) return true;
+  const int work = groups * Nrho;
+  switch (N) {
+    case 16: return work >= (prec == 64 ? 3 : 6);
+    case 24: return groups >= 3 && (prec == 64 || work >= 15);
+    case 32: return prec == 64 ? groups >= 2 : work >= 3;
+    default: return false;
+  }
+}
+
 // operand values of R(shift) (vhs_planar.hpp) for every radial node and shift:
 // [Nrho][nshift][64 lanes][part][K step], and beta = -sin(theta N/2) / N
 template <typename T, int N>
@@ -3085,7 +3109,8 @@ extern "C" int dgfs_vhs_create(const dgfs_vhs_desc* d, void** out) {
     if (rc) return rc;
   }
   std::vector<double> shifts;
-  if ((N == 16 || N == 24 || N == 32) && planar_groups(d->sz, h->M, &h->pgroups, &shifts)) {
+  if ((N == 16 || N == 24 || N == 32) && planar_groups(d->sz, h->M, &h->pgroups, &shifts) &&
+      planar_pays(N, h->prec, static_cast<int>(h->pgroups.size()), h->Nrho)) {
     std::vector<double> smat, pbeta;
     if (h->prec == 64)
       planar_tables<double>(N, alpha, shifts, &smat, &pbeta);

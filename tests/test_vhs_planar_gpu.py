@@ -149,6 +149,35 @@ def test_operator_tells_which_gain_ran(device):
     assert not make(12, designs()["m12"], 64).planar
 
 
+# groups (pairs of mirrored directions), radial nodes, whether the automatic
+# choice is planar: both sides of each line
+LINES = {(16, 64): [(1, 2, False), (1, 3, True), (2, 2, True)], (16, 32): [(1, 5, False), (1, 6, True), (2, 2, False), (2, 3, True), (6, 1, True)],
+         (24, 64): [(2, 8, False), (3, 1, True)], (24, 32): [(2, 8, False), (3, 4, False), (3, 5, True), (6, 1, True)],
+         (32, 64): [(1, 8, False), (2, 1, True)], (32, 32): [(2, 1, False), (1, 3, True), (6, 1, True)]}
+
+
+@pytest.mark.parametrize("N,precision", list(LINES))
+def test_designs_of_few_groups(N, precision, device):
+    """Designs of few directions take the planar gain from where their groups
+    and radial nodes are enough work; on both sides of the line Q is the
+    multi-pass kernel's (the module's bounds)."""
+    flat = designs()["m4_one_pair"]
+    by_groups = {1: flat[:2], 2: flat, 3: designs()["m6_cuboctahedron"], 6: designs()["m12"]}
+    f = np.random.default_rng(N).uniform(0.0, 1.0, size=(2, N ** 3))
+    for groups, Nrho, planar in LINES[N, precision]:
+        sz = by_groups[groups]
+        say("few groups", N, precision, groups, Nrho)
+        op = make(N, sz, precision, Nrho=Nrho)
+        assert op.planar == planar
+        Q = run(op, f, device)
+        assert op.ran_planar() == planar
+        ref = run(make(N, sz, 64, Nrho=Nrho, algorithm=1), f, device)
+        if precision == 64:
+            assert rel(Q, ref) < 1e-12
+        else:
+            assert rel(Q, ref) < 1.5 * rel(run(make(N, sz, 32, Nrho=Nrho, algorithm=1), f, device), ref)
+
+
 @pytest.mark.parametrize("N,npts", [(16, 400), (24, 60)])
 def test_small_batch_captured_after_a_larger_one(N, npts, device):
     """A batch small enough to split its groups over work items finds room for
