@@ -2386,17 +2386,31 @@ static int planar_slots() {
 }
 
 // Parts that the planar gain's groups are split into, work items of their own
-// whose transforms the x pass sums: as many as keep one item per slot.  Only
-// for batches that would leave slots idle with one radial node to an item (one
-// point at 24^3 FP32 has 12 items of 6 groups each, 75 us of gain at one part).
+// whose transforms the x pass sums, for batches that leave CUs idle with one
+// radial node to an item (one point at 24^3 FP32, 12 nodes: 133 us at one part,
+// 101 at three).  Measured over 3 to 16 nodes and 1 to 48 points:
+// - up to one item per CU.  A second one on a CU pays in FP32 only, and only
+//   where one part already fills half of the CUs (24 points at 24^3, 6 nodes:
+//   138 -> 120 us; 16^3 FP64, 8 nodes, 24 points: 58 -> 63 us, so not there);
+//   beyond one item per CU, as many as are resident;
+// - three parts and more only while the x pass sums at most 36 transforms (48
+//   in FP64 at 24^3 and 32^3, whose items are longest): it reads them one after
+//   another (16 nodes, 4 points: 16^3 FP64 57 us at one part, 52 at two, 55 at
+//   three, 78 at six; 24^3 FP32 136 / 115 / 122 / 165).
 // An explicit group count and the allocation-free mode keep one part.
 template <typename T, int N>
 static int planar_split(const VhsHandle* h, int npts, int slots) {
   const int ngr = static_cast<int>(h->pgroups.size());
   if (h->groups_override > 0 || h->no_alloc) return 1;
-  const long items = static_cast<long>(npts) * h->Nrho * PlanarShape<T, N>::XH;
+  const long items = static_cast<long>(npts) * h->Nrho * PlanarShape<T, N>::XH, cus = cu_count();
+  long most = slots;
+  if (2 * items <= cus)
+    most = std::min(most, cus);
+  else if (items <= cus)
+    most = sizeof(T) == 4 ? std::min(most, 2 * cus) : 0;
+  const int sums = (sizeof(T) == 8 && N > 16) ? 48 : 36;
   for (int g = ngr; g > 1; --g)
-    if (ngr % g == 0 && items * g <= slots) return g;
+    if (ngr % g == 0 && items * g <= most && (g == 2 || g * h->Nrho <= sums)) return g;
   return 1;
 }
 
@@ -2404,12 +2418,10 @@ static int planar_split(const VhsHandle* h, int npts, int slots) {
 // that a smaller batch after a larger one (a captured one, say) finds its room
 template <typename T, int N>
 static size_t planar_tb_points(const VhsHandle* h, int npts, int slots) {
+  const long split = slots / (2L * h->Nrho * PlanarShape<T, N>::XH);  // larger batches are never split
   long most = npts;
-  const int ngr = static_cast<int>(h->pgroups.size());
-  if (h->groups_override > 0 || h->no_alloc) return static_cast<size_t>(most);
-  for (int g = 2; g <= ngr; ++g)
-    if (ngr % g == 0)
-      most = std::max(most, std::min<long>(npts, slots / (static_cast<long>(h->Nrho) * PlanarShape<T, N>::XH * g)) * g);
+  for (long n = std::min<long>(npts, split); n > 0; --n)
+    most = std::max(most, n * planar_split<T, N>(h, static_cast<int>(n), slots));
   return static_cast<size_t>(most);
 }
 

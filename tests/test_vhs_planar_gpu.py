@@ -178,16 +178,17 @@ def test_designs_of_few_groups(N, precision, device):
             assert rel(Q, ref) < 1.5 * rel(run(make(N, sz, 32, Nrho=Nrho, algorithm=1), f, device), ref)
 
 
-@pytest.mark.parametrize("N,npts", [(16, 400), (24, 60)])
-def test_small_batch_captured_after_a_larger_one(N, npts, device):
+# Nrho 4 and 13: up to six parts and up to two of the groups
+@pytest.mark.parametrize("N,npts,Nrho", [(16, 400, 4), (24, 60, 4), (16, 100, 13), (24, 20, 13)])
+def test_small_batch_captured_after_a_larger_one(N, npts, Nrho, device):
     """A batch small enough to split its groups over work items finds room for
     the parts' transforms in the workspace of a larger batch: captured without
     an allocation, every replay equal to the eager result."""
     import torch
     rng = np.random.default_rng(N)
     f = rng.uniform(0.0, 1.0, size=(npts, N ** 3))
-    say("planar capture", N, npts)
-    op = make(N, designs()["m12"], 64)
+    say("planar capture", N, npts, Nrho)
+    op = make(N, designs()["m12"], 64, Nrho=Nrho)
     big = run(op, f, device)
     for n in (1, 3, 11):
         ft = torch.as_tensor(f[:n], device=device)
