@@ -2389,25 +2389,26 @@ static int planar_slots() {
 // whose transforms the x pass sums, for batches that leave CUs idle with one
 // radial node to an item (one point at 24^3 FP32, 12 nodes: 133 us at one part,
 // 101 at three).  Measured over 3 to 16 nodes and 1 to 48 points:
-// - up to one item per CU.  A second one on a CU pays in FP32 only, and only
-//   where one part already fills half of the CUs (24 points at 24^3, 6 nodes:
-//   138 -> 120 us; 16^3 FP64, 8 nodes, 24 points: 58 -> 63 us, so not there);
-//   beyond one item per CU, as many as are resident;
+// - up to one item per CU.  A second one on a CU pays only where one part
+//   already fills half of the CUs, and there in FP32 (24 points at 24^3, 6
+//   nodes: 138 -> 120 us) or with few sums (16^3 FP64, 1 node, 130 points: 71
+//   -> 65 us; 8 nodes, 24 points: 58 -> 63 us); beyond one item per CU, as many
+//   as are resident;
 // - three parts and more only while the x pass sums at most 36 transforms (48
 //   in FP64 at 24^3 and 32^3, whose items are longest): it reads them one after
 //   another (16 nodes, 4 points: 16^3 FP64 57 us at one part, 52 at two, 55 at
 //   three, 78 at six; 24^3 FP32 136 / 115 / 122 / 165).
-// An explicit group count and the allocation-free mode keep one part.
+// An explicit group count keeps one part.
 template <typename T, int N>
-static int planar_split(const VhsHandle* h, int npts, int slots) {
+static int planar_split(const VhsHandle* h, int npts, int slots, long cus) {
   const int ngr = static_cast<int>(h->pgroups.size());
-  if (h->groups_override > 0 || h->no_alloc) return 1;
-  const long items = static_cast<long>(npts) * h->Nrho * PlanarShape<T, N>::XH, cus = cu_count();
+  if (h->groups_override > 0) return 1;
+  const long items = static_cast<long>(npts) * h->Nrho * PlanarShape<T, N>::XH;
   long most = slots;
   if (2 * items <= cus)
     most = std::min(most, cus);
   else if (items <= cus)
-    most = sizeof(T) == 4 ? std::min(most, 2 * cus) : 0;
+    most = (sizeof(T) == 4 || h->Nrho <= 3) ? std::min(most, 2 * cus) : 0;
   const int sums = (sizeof(T) == 8 && N > 16) ? 48 : 36;
   for (int g = ngr; g > 1; --g)
     if (ngr % g == 0 && items * g <= most && (g == 2 || g * h->Nrho <= sums)) return g;
@@ -2418,10 +2419,13 @@ static int planar_split(const VhsHandle* h, int npts, int slots) {
 // that a smaller batch after a larger one (a captured one, say) finds its room
 template <typename T, int N>
 static size_t planar_tb_points(const VhsHandle* h, int npts, int slots) {
+  // the scratch array is shared out for the batches of one call
+  if (h->no_alloc) return static_cast<size_t>(npts) * planar_split<T, N>(h, npts, slots, cu_count());
   const long split = slots / (2L * h->Nrho * PlanarShape<T, N>::XH);  // larger batches are never split
+  const long cus = cu_count();
   long most = npts;
   for (long n = std::min<long>(npts, split); n > 0; --n)
-    most = std::max(most, n * planar_split<T, N>(h, static_cast<int>(n), slots));
+    most = std::max(most, n * planar_split<T, N>(h, static_cast<int>(n), slots, cus));
   return static_cast<size_t>(most);
 }
 
@@ -2431,7 +2435,7 @@ static int run_planar(VhsHandle* h, const double* fc, double* Qc, int npts, hipS
   if constexpr (planar_available<N>()) {
     using PS = PlanarShape<T, N>;
     const int slots = planar_slots<T, N>();
-    const int gsplit = planar_split<T, N>(h, npts, slots);
+    const int gsplit = planar_split<T, N>(h, npts, slots, cu_count());
     const int groups = gsplit > 1 ? h->Nrho : pick_groups(h, npts * PS::XH, slots);
     const int ppg = (h->Nrho + groups - 1) / groups;
     int rc = grow_ws(h, &h->plop, &h->cap_plop, static_cast<size_t>(npts) * PS::per_point * sizeof(T), "plane operands");
@@ -2809,8 +2813,9 @@ struct ScratchPlan {
   size_t total() const { return z + s + w + F + Ghat + Ft + Wny + Tb + plop; }
 };
 
+// (pslots: the planar gain's resident work items)
 template <typename T, int N>
-static ScratchPlan plan_scratch(const VhsHandle* h, int pts, int slots) {
+static ScratchPlan plan_scratch(const VhsHandle* h, int pts, int slots, int pslots) {
   constexpr size_t n = static_cast<size_t>(N) * N * N;
   const bool rr = use_rr(h);
   int gain_slots = rr ? cu_count() : slots;
@@ -2819,13 +2824,17 @@ static ScratchPlan plan_scratch(const VhsHandle* h, int pts, int slots) {
   p.pts = pts;
   p.slots = slots;
   if constexpr (planar_available<N>()) {
-    if (use_planar(h)) {  // one G^ per point whatever the split; only the FP64 prep and finalize take slot cubes
+    // one G^ per point whatever the split; only the FP64 prep and finalize at
+    // 24^3 and 32^3 take slot cubes
+    if (use_planar(h)) {
       using PS = PlanarShape<T, N>;
       p.groups = 1;
       p.items = static_cast<size_t>(pts);
-      p.z = align_up(static_cast<size_t>(slots) * n * sizeof(cpx<T>));
+      if (!rr_available<T, N>() && !rr1_edges<T, N>())
+        p.z = align_up(static_cast<size_t>(slots) * n * sizeof(cpx<T>));
       p.F = p.Ghat = align_up(static_cast<size_t>(pts) * n * sizeof(cpx<T>));
-      p.Tb = align_up(static_cast<size_t>(pts) * h->Nrho * PS::nslots * PS::NN * sizeof(cpx<T>));
+      p.Tb = align_up(static_cast<size_t>(pts) * planar_split<T, N>(h, pts, pslots, cu_count()) * h->Nrho *
+                      PS::nslots * PS::NN * sizeof(cpx<T>));
       p.plop = align_up(static_cast<size_t>(pts) * PS::per_point * sizeof(T));
       return p;
     }
@@ -2914,19 +2923,25 @@ static int eval_noalloc_impl(VhsHandle* h, const double* f, double* Q, int npts,
   int slots = std::min(occupancy_slots<T, N>(), cu_count());
   const size_t per_slot = n * (sizeof(cpx<T>) + sizeof(T)) + 3 * N * N * sizeof(cpx<T>) + 3 * kScratchAlign;
   slots = static_cast<int>(std::max<size_t>(1, std::min<size_t>(slots, kScratchBytes / 2 / per_slot)));
+  int pslots = 0;
+  if constexpr (planar_available<N>()) {
+    if (use_planar(h)) pslots = planar_slots<T, N>();
+  }
   // largest balanced chunk that fits; the last chunk may be smaller and
-  // then split its points into more radial groups, so the gain partials'
-  // share is sized for whichever of the two needs more
+  // then split its points into more radial groups or parts, so the shares of
+  // the gain partials and of the transforms are sized for whichever of the
+  // two needs more
   auto plan_for = [&](int cap, int* chunk_out) {
     const int nchunks = (npts + cap - 1) / cap;
     const int chunk = (npts + nchunks - 1) / nchunks;
     const int last = npts - ((npts + chunk - 1) / chunk - 1) * chunk;
-    ScratchPlan a = plan_scratch<T, N>(h, chunk, slots);
-    const ScratchPlan b = plan_scratch<T, N>(h, last, slots);
+    ScratchPlan a = plan_scratch<T, N>(h, chunk, slots, pslots);
+    const ScratchPlan b = plan_scratch<T, N>(h, last, slots, pslots);
     if (b.Ghat > a.Ghat) {
       a.Ghat = b.Ghat;
       a.items = b.items;
     }
+    a.Tb = std::max(a.Tb, b.Tb);
     *chunk_out = chunk;
     return a;
   };
@@ -2936,7 +2951,7 @@ static int eval_noalloc_impl(VhsHandle* h, const double* f, double* Q, int npts,
     if (cap < 1)
       return fail(DGFS_ERR_UNSUPPORTED,
                   "one point at Nv=%d (precision %d) needs %zu bytes of workspace, beyond the %zu-byte scratch array",
-                  N, h->prec, plan_scratch<T, N>(h, 1, slots).total(), kScratchBytes);
+                  N, h->prec, plan_scratch<T, N>(h, 1, slots, pslots).total(), kScratchBytes);
     plan = plan_for(cap, &chunk);
     if (plan.total() <= kScratchBytes) break;
     const double over = static_cast<double>(plan.total()) / static_cast<double>(kScratchBytes);
