@@ -3052,7 +3052,10 @@ static VhsHandle* as_handle(void* p) {
 using namespace dgfs;
 
 extern "C" const char* dgfs_last_error(void) { return last_error_ref().c_str(); }
-extern "C" const char* dgfs_version(void) { return "dgfs_hip 0.1 (gfx950)"; }
+#ifndef DGFS_BUILD_ID  // hash of the sources, from the build
+#define DGFS_BUILD_ID "unidentified"
+#endif
+extern "C" const char* dgfs_version(void) { return "dgfs_hip 0.1 (gfx950) " DGFS_BUILD_ID; }
 
 extern "C" int dgfs_vhs_create(const dgfs_vhs_desc* d, void** out) {
   if (!d || !out) return fail(DGFS_ERR_INVALID_VALUE, "null descriptor or handle pointer");

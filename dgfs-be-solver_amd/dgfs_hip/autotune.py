@@ -1,9 +1,10 @@
 """Launch-shape autotuner of the collision operators (single-species VHS and
 two-species VSS).
 
-For a given operator (velocity grid, precision, K = M Nrho) and batch size it
-times every candidate of
-  * the gain algorithm: multi-pass (any grid), register-resident (FP32:
+For a given operator (velocity grid, precision, directions M and radial nodes
+Nrho, planar design or not) and batch size it times every candidate of
+  * the gain algorithm: the automatic choice where that is the
+    planar-direction gain, multi-pass (any grid), register-resident (FP32:
     two pencils per thread at Nv 16 / 32 with the Nyquist planes from a
     separate kernel or inside the kernel; one pencil per thread at Nv 16 / 24)
     or the slab kernel (FP64 at Nv 16 / 24 / 32);
@@ -38,6 +39,12 @@ def _key(op, npts, platform=""):
              f"-proj{int(bool(op.project))}-pts{bucket}")
     else:
         k = f"vhs-N{op.Nv}-p{op.precision}-K{op.K}-proj{int(bool(op.project))}-pts{bucket}"
+        # the design: the same K comes of other numbers of directions and
+        # nodes, and a planar design has a kernel that the others do not
+        if hasattr(op, "M"):
+            k += f"-M{op.M}"
+        if getattr(op, "planar", False):
+            k += "-planar"
     return f"{platform}|{k}" if platform else k
 
 

@@ -6,6 +6,7 @@ placed next to this file, so it travels with the source tree.
 """
 from __future__ import annotations
 
+import hashlib
 import os
 import shutil
 import subprocess
@@ -37,15 +38,29 @@ def _hipcc():
     raise RuntimeError("hipcc not found: the HIP library cannot be built")
 
 
+def source_id() -> str:
+    """Hash of everything the library is compiled from (sources, headers,
+    flags); dgfs_version ends with it, so what is remembered of one build, such
+    as tuned launch shapes, is not taken for another."""
+    h = hashlib.sha256(" ".join(HIPCC_FLAGS).encode())
+    for d in (CSRC, INCLUDE):
+        for name in sorted(os.listdir(d)):
+            if name.endswith((".hip", ".hpp", ".h")):
+                with open(os.path.join(d, name), "rb") as fh:
+                    h.update(name.encode() + b"\0" + fh.read())
+    return h.hexdigest()[:12]
+
+
 def build(verbose: bool = False, jobs: int = 4) -> str:
     hipcc = _hipcc()
+    build_id = f'-DDGFS_BUILD_ID="{source_id()}"'
     objdir = os.path.join(PKG_DIR, "_obj")
     os.makedirs(objdir, exist_ok=True)
     srcs = [s for s in SOURCES if os.path.exists(os.path.join(CSRC, s))]
 
     def compile_one(src):
         obj = os.path.join(objdir, src.replace(".hip", ".o"))
-        cmd = [hipcc, *HIPCC_FLAGS, "-I", CSRC, "-I", INCLUDE, "-c",
+        cmd = [hipcc, *HIPCC_FLAGS, build_id, "-I", CSRC, "-I", INCLUDE, "-c",
                os.path.join(CSRC, src), "-o", obj]
         if verbose:
             print(" ".join(cmd), flush=True)

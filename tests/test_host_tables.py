@@ -212,3 +212,26 @@ def test_autotune_cache_is_keyed_by_platform_and_drops_stale_entries(tmp_path, m
     best, _ = tuner.tune(op, 0, 0, 64, stream=0)
     assert best["algorithm"] in (1, 2, 3, 4, 5, 6)
     assert tuner._cache[key]["best"] == best
+
+
+def test_autotune_key_tells_designs_apart():
+    """A planar and a general design of equal K never share an entry, nor do
+    designs of equal K from other numbers of directions; the planar-direction
+    gain (algorithm 0) is a candidate for planar designs only."""
+    import types
+    from dgfs_hip.autotune import Autotuner, _key
+    ns = lambda **kw: types.SimpleNamespace(Nv=32, precision=32, K=96, project=True, **kw)
+    planar = ns(M=12, Nrho=8, planar=True)
+    general = ns(M=6, Nrho=16, planar=False)
+    tilted = ns(M=12, Nrho=8, planar=False)
+    assert len({_key(op, 64) for op in (planar, general, tilted)}) == 3
+    algos = lambda op: {c["algorithm"] for c in Autotuner.candidates(op, 256)}
+    assert algos(planar) == {0, 1, 2, 3, 5}
+    assert algos(general) == algos(tilted) == {1, 2, 3, 5}
+
+
+def test_library_version_names_its_sources():
+    """The version string that keys tuned launch shapes changes with the
+    sources the library was built from."""
+    from dgfs_hip import _lib, build
+    assert _lib.version().split()[-1] == build.source_id()
