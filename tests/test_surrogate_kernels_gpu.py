@@ -69,6 +69,43 @@ def test_layers_small_batches(P, device):
     assert e < 1e-5 and eg < 1e-5
 
 
+@pytest.mark.parametrize("P", [129, 300])
+def test_layers_of_several_tiles_per_wave(P, device):
+    """Batches beyond 128 points, where a wave of the backward layer takes more
+    than one tile and the last round is uneven, and the layer products are not
+    split: every parameter block's gradient on its own (a norm over the whole
+    vector is K's), against the FP64 oracle.  Output gradients of one sign, so
+    that no block is the small difference of large sums: FP32 sums of up to 512
+    P terms, 1e-5 of the block's norm."""
+    import torch
+    from dgfs_hip.surrogate import SpectralSurrogate
+    sur = SpectralSurrogate(8, 5.0, (10.0 / 8) ** 3, 0.38, 1.0, max_batch=P, device=device, seed=3)
+    rng = np.random.default_rng(P)
+    f32 = lambda a: torch.as_tensor(a, dtype=torch.float32, device=device).contiguous()
+    xt, ltt = f32(rng.normal(size=(P, 512)) * 0.3), f32(rng.normal(size=P) * 0.2)
+    dt = f32(rng.uniform(0.5, 1.5, size=(P, 512)))
+    out = torch.empty((P, 512), dtype=torch.float32, device=device)
+    print("layers", P, flush=True)
+    sur.forward(xt, ltt, P, out)
+    sur.backward(dt)
+    torch.cuda.synchronize()
+    th = sur.params_bf16.cpu().numpy().astype(np.float64)
+    ref, cache = S.forward(th, xt.cpu().numpy().astype(np.float64), ltt.cpu().numpy().astype(np.float64))
+    assert np.linalg.norm(out.cpu().numpy() - ref) < 1e-5 * np.linalg.norm(ref)
+    g, got = S.backward(th, cache, dt.cpu().numpy().astype(np.float64)), sur.grad.cpu().numpy()
+    sizes = [("P0", S.WIDTH), ("P1", S.WIDTH), ("E", S.MODES * S.WIDTH)]
+    for l in range(S.LAYERS):
+        sizes += [(f"K{l}", S.MODES ** 2), (f"W{l}", S.WIDTH ** 2), (f"R{l}", S.WIDTH ** 2), (f"b{l}", S.WIDTH)]
+    sizes += [("Pout", S.WIDTH), ("bout", S.MODES)]
+    assert sum(n for _, n in sizes) == g.size
+    at = 0
+    for name, n in sizes:
+        e = np.linalg.norm(got[at:at + n] - g[at:at + n]) / np.linalg.norm(g[at:at + n])
+        say(" ", name, e)
+        assert e < 1e-5, name
+        at += n
+
+
 @pytest.mark.parametrize("N", [12, 16, 24, 32])
 def test_encode_decode_grids(N, device):
     """Encoder and projecting decoder on every built grid, one point and more

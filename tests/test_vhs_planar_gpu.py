@@ -80,8 +80,9 @@ def test_planar_matches_multipass_on_rough_states(N, name, device):
 @pytest.mark.parametrize("precision", [64, 32])
 @pytest.mark.parametrize("N,npts", [(16, 1), (16, 300), (24, 5), (32, 1), (32, 37)])
 def test_planar_batches_and_registers(N, npts, precision, device):
-    """One point to more items than the chip holds, contiguous and as AoSoA
-    registers of a ragged element count, with the projection."""
+    """Small batches, contiguous and as AoSoA registers of a ragged element
+    count, with the projection; FP32 within the module's factor of 1.5 of the
+    multi-pass kernel's distance from FP64."""
     import torch
     sz = designs()["m12"]
     vm = O.VelocityMesh(N, 6.0, 4, 12)
@@ -95,7 +96,10 @@ def test_planar_batches_and_registers(N, npts, precision, device):
     ref = run(make(N, sz, 64, project=True, algorithm=1), f[sub], device)
     e = rel(Q[sub], ref)
     say("  vs FP64 multi-pass", e)
-    assert e < (1e-11 if precision == 64 else 1e-3)
+    if precision == 64:
+        assert e < 1e-11
+    else:
+        assert e < 1.5 * rel(run(make(N, sz, 32, project=True, algorithm=1), f[sub], device), ref)
     # elements [1, neles) of a register of one point per element
     neles, n = npts + 1, N ** 3
     nparr = -(-neles // 32) * 32
@@ -111,6 +115,41 @@ def test_planar_batches_and_registers(N, npts, precision, device):
     got = np.stack([qr[(e + 1) // 32, :, (e + 1) % 32] for e in range(npts)])
     assert np.array_equal(got, Q)
     assert not qr[0, :, 0].any()
+
+
+@pytest.mark.parametrize("precision", [64, 32])
+@pytest.mark.parametrize("N", [16, 24, 32])
+def test_planar_large_batches(N, precision, device):
+    """Batches on both sides of where the x pass takes a wave per pencil block
+    (its pencils are a wave per SIMD) and of where the operand kernel takes 256
+    threads (more points than CUs), with more items than are resident at once.
+    Against the FP64 oracle (1e-10; FP32 within 1.5 of the multi-pass kernel's
+    distance), and every point bitwise that of its state wherever it lies."""
+    import torch
+    cus = torch.cuda.get_device_properties(device).multi_processor_count
+    limit = 64 * 4 * cus // ((N // 2 + 1) * N * (precision // 32))
+    vm = O.VelocityMesh(N, 6.0, 4, 12)
+    rng = np.random.default_rng(N)
+    base = np.stack([0.5 * O.maxwellian(vm, 1, rng.uniform(-0.6, 0.6, 3), rng.uniform(0.5, 1.5)) +
+                     0.5 * O.maxwellian(vm, 1, rng.uniform(-0.6, 0.6, 3), rng.uniform(0.5, 1.5)) for _ in range(3)])
+    want = O.project_invariants(vm, O.VHSOracle(vm, 0.38, 1.0).q(base))
+    sz = designs()["m12"]
+    bound = 1e-10
+    if precision == 32:
+        bound = 1.5 * rel(run(make(N, sz, 32, project=True, algorithm=1), base, device), want)
+    op = make(N, sz, precision, project=True)
+    for npts in (limit, limit + 1, max(limit, 2 * cus) + 3):
+        say("planar large batch", N, precision, npts)
+        ft = torch.as_tensor(base, device=device)[torch.arange(npts, device=device) % 3].contiguous()
+        Qt = torch.full_like(ft, float("nan"))
+        op.eval_contig(ft.data_ptr(), Qt.data_ptr(), npts, torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        assert op.ran_planar()
+        e = rel(Qt[:3].cpu().numpy(), want)
+        say("  vs oracle", e)
+        assert e < bound
+        for i in range(3):
+            assert bool((Qt[i::3] == Qt[i]).all())
 
 
 def test_other_designs_keep_the_general_gain(device):
