@@ -15,7 +15,7 @@ Maxwellians, density 1) generated on the device, so the timed region starts
 with the inputs resident in HBM.
 
 Usage: python bench.py [--gpus 1] [--steps K] [--warmup W]
-Prints one JSON line.
+Prints one JSON line; the full record, with its threshold tables, goes to stderr.
 """
 import argparse
 import json
@@ -895,6 +895,31 @@ def read_traffic(name):
         return json.load(fh)
 
 
+def headline(record):
+    """The record without its threshold tables and explanatory texts, floats to
+    seven digits."""
+    def short(x):
+        if isinstance(x, dict):
+            return {k: short(v) for k, v in x.items() if k not in DETAILS}
+        if isinstance(x, list):
+            return [short(v) for v in x]
+        return float(f"{x:.7g}") if isinstance(x, float) else x
+
+    out = short(record)
+    for sec in (out.get("surrogate"), out.get("surrogate", {}).get("low_knudsen_field")):
+        if sec:
+            keep = ("unit", "workload", "points", "value", "fallback_rate", "rel_l2_vs_fp64", "fallback_threshold",
+                    "fallback_threshold_high_modes", "conservation_max_rel", "speedup_vs_fp64", "fastest_within_1e-3",
+                    "low_knudsen_field")
+            for k in [k for k in sec if k not in keep]:
+                del sec[k]
+    return out
+
+
+# explanatory texts of the full record
+DETAILS = ("note", "flops_model", "compute_unit", "traffic_source")
+
+
 def main():
     args = parse()
     world = int(os.environ.get("WORLD_SIZE", "1"))
@@ -1178,7 +1203,10 @@ def main():
             "one_core_value": 2 / t1,
         }
 
-    print(json.dumps(line), flush=True)
+    # every table and note on stderr; the one line on stdout stays short enough
+    # to be read whole from the tail of a log
+    print("# full record: " + json.dumps(line), file=sys.stderr, flush=True)
+    print(json.dumps(headline(line)), flush=True)
 
 
 if __name__ == "__main__":
