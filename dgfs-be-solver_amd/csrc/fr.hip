@@ -330,8 +330,8 @@ struct BcArgs {
 // workgroup takes kBcPts boundary points (consecutive ones are neighbouring
 // elements of an AoSoA block) by kBcRows rows of vchunk velocities: a boundary
 // has few points and many velocities, and one thread per point with 64
-// velocities each left most of the chip idle (36 points at 24^3: 31 -> 7.5 us on
-// MI355X).
+// velocities each left most of the chip idle (36 points at 24^3 on MI355X: 47
+// -> 15 us within the cavity's right-hand side, 31 -> 7.5 us repeated).
 constexpr int kBcPts = 32, kBcRows = 8;
 
 __global__ __launch_bounds__(kBcPts * kBcRows) void k_bccflux(BcArgs a) {
@@ -420,7 +420,7 @@ __global__ __launch_bounds__(NTH) void k_bccupdate_diffuse(int ndims, int nfpts,
     const int vv = vidx + v;
     double fac = 0.0;
     for (int d = 0; d < ndims; ++d) fac += (cv[d * static_cast<long>(vsize) + vv] - U[d]) * n[d];
-    // the value first, the sums after (36 points at 24^3: 17.9 us; 20.8 with
+    // the value first, the sums after (36 points at 24^3, repeated: 17.9 us; 20.8 with
     // load and sum in one branch)
     const double x = fac >= 0 ? L[ol + 32L * v] : st ? cyl_wall_f(cv, vsize, vv, U, Tw) : f0[vv];
     if (fac >= 0) s0 += fac * x * cw;
@@ -503,9 +503,11 @@ __global__ __launch_bounds__(256) void k_copy_reg(int nblocks, int count, const 
 // a velocity's abscissae are read once for two values), kMomUnroll velocities
 // in flight; then a sum over the threads of a wave and over the waves, always
 // in the same order.  Two passes over f, the bulk velocity first (the second
-// mostly from the last-level cache).  Bound by the latency of the loads of f:
-// 2304 points at 24^3 take 205 us (9019 us with one thread per point), where
-// reading f once is 56 us and the FP64 sums about 22 us.
+// mostly from the last-level cache).  Bound by a CU's work, not by memory: at
+// 24^3 180 workgroups of EW 8, one to a CU, take 95 us and 288 take 206 (2304
+// points; 9019 us with one thread per point, 56 us for reading f once).  Its
+// FP64 sums are, by count, about 17 us of a workgroup's 95; the rest is loads,
+// 64-byte rows of f and three abscissae for every two values.
 constexpr int kMomUnroll = 4;
 
 // totals over the workgroup of NQ values of two elements per thread; red:
@@ -744,7 +746,7 @@ extern "C" int dgfs_bccflux(int bctype, int ndims, int nfpts, int nvars, int vid
   BcArgs a;
   a.bctype = bctype; a.ndims = ndims; a.nfpts = nfpts; a.nvars = nvars; a.vidx = vidx;
   a.vsize = vsize;
-  // 4 velocities per thread (36 points at 24^3: 7.6 us, 38 with 64 each), twice
+  // 4 velocities per thread (36 points at 24^3, repeated: 7.6 us, 38 with 64 each), twice
   // as many again, up to 64, while there are more than 64 workgroups per CU,
   // whose turnover then costs more than it hides (20000 points of 4096
   // velocities 653 -> 596 us, 4096 points at 24^3 440 -> 418 us), or while the
@@ -762,9 +764,10 @@ extern "C" int dgfs_bccflux(int bctype, int ndims, int nfpts, int nvars, int vid
 }
 
 // threads per wall point of the balance: 1024 while each has a velocity and the
-// points are few enough that a point's latency shows (36 points at 24^3: 48 ->
-// 18 us on MI355X against 256 threads, 1024 points 95 us either way, 4096
-// points 368 -> 357 us); with many points the narrow block's shorter reduction
+// points are few enough that a point's latency shows (36 points at 24^3 on
+// MI355X: 56 -> 26 us against 256 threads within the cavity's right-hand side,
+// 48 -> 18 us repeated; 1024 points 95 us either way, 4096 points 368 -> 357
+// us); with many points the narrow block's shorter reduction
 // wins (20000 points of 64 velocities 29 against 104 us, 200000 of 512 0.64
 // against 1.39 ms), and its grid takes four times as many points.
 static int update_threads(int nfpts, int nvars) { return nvars >= 1024 && nfpts <= 4096 ? 1024 : 256; }

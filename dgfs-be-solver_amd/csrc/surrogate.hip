@@ -254,8 +254,8 @@ __global__ __launch_bounds__(256) void k_gemm_bf16_big(GemmArgs g) {
 // LDS each) share a CU.  For outputs of at least 128 x 64 with 16-byte
 // aligned operands; the 64 x 64 kernel above stages every value through a
 // bounds-checked scalar load and two barriers per 32 k and ran the network's
-// products (512 x 32 P x 512) at 39 TFLOP/s on MI355X, this one at 82 (P =
-// 256) to 89 (P = 1000).
+// products (512 x 32 P x 512) at 39 TFLOP/s on MI355X, this one at 83 (P =
+// 256) to 86 (P = 1000), 71 with op(A) = A^T.
 constexpr int kFM = 128, kFN = 64, kFK = 32, kFP = kFK + 4;
 
 // this thread's share of an R x 32 operand tile (R rows of op(A) or columns of

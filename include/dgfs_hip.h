@@ -31,7 +31,7 @@ enum dgfs_status {
 /* Text of the last error raised on this thread ("" if none). */
 const char* dgfs_last_error(void);
 
-/* Library version string. */
+/* Library version string; its last word is a hash of the sources and flags. */
 const char* dgfs_version(void);
 
 /* ------------------------------------------------------------------------
@@ -136,8 +136,9 @@ int dgfs_vhs_set_slots(void* handle, int nslots);
  * 24 and 32; 1 otherwise.  At Nv 16, 24 and 32 the automatic choice runs the
  * planar-direction gain (csrc/vhs_planar.hpp) in that kernel's place when
  * every direction of the design has exactly one zero component and comes with
- * its mirror image (the 24-point design, M = 12); it is not selectable by
- * number.  get_algorithm reports the kernel the last eval ran, or the one the
+ * its mirror image and the design is enough work for it (always with the
+ * 24-point design, M = 12; designs of fewer directions only with enough radial
+ * nodes); it is not selectable by number.  get_algorithm reports the kernel the last eval ran, or the one the
  * planar-direction gain stood in for; get_planar tells the two apart:
  * *automatic is 1 if algorithm 0 of this handle runs the planar-direction gain,
  * *last is 1 if the last eval ran it.
