@@ -2392,8 +2392,9 @@ static int planar_slots() {
 // - up to one item per CU.  A second one on a CU pays only where one part
 //   already fills half of the CUs, and there in FP32 (24 points at 24^3, 6
 //   nodes: 138 -> 120 us) or with few sums (16^3 FP64, 1 node, 130 points: 71
-//   -> 65 us; 8 nodes, 24 points: 58 -> 63 us); beyond one item per CU, as many
-//   as are resident;
+//   -> 65 us; 8 nodes, 24 points: 58 -> 63 us); beyond one item per CU, up to
+//   three (16^3 FP64, 8 nodes, 48 points: 79 -> 74 us; four in FP32, 64 points:
+//   68 -> 76 us);
 // - three parts and more only while the x pass sums at most 36 transforms (48
 //   in FP64 at 24^3 and 32^3, whose items are longest): it reads them one after
 //   another (16 nodes, 4 points: 16^3 FP64 57 us at one part, 52 at two, 55 at
@@ -2404,7 +2405,7 @@ static int planar_split(const VhsHandle* h, int npts, int slots, long cus) {
   const int ngr = static_cast<int>(h->pgroups.size());
   if (h->groups_override > 0) return 1;
   const long items = static_cast<long>(npts) * h->Nrho * PlanarShape<T, N>::XH;
-  long most = slots;
+  long most = std::min<long>(slots, 3 * cus);
   if (2 * items <= cus)
     most = std::min(most, cus);
   else if (items <= cus)
