@@ -1871,7 +1871,7 @@ struct VhsHandle {
   size_t cap_tb = 0;
   // planar-direction gain (vhs_planar.hpp): the design's groups, the operand
   // values of the moves, and the points' operand form
-  int planar = 0;        // the design is planar and the kernels exist for this grid
+  int planar = 0;        // planar design, built grid and enough work (planar_pays)
   int nshift = 0;
   std::vector<PlanarGroup> pgroups;
   void* smat = nullptr;  // [Nrho][nshift][64][NR] operand values of R(shift)
